@@ -19,6 +19,7 @@ namespace gki {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 enum DType : int { kF32 = 0, kF16 = 1, kBF16 = 2 };
 
@@ -42,6 +43,10 @@ struct F16 {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
                                                    __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   }
+  __device__ static inline floatx16 mfma32(const uint4& a, const uint4& b, floatx16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
+                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
   // eight 1.0 elements: an all-ones MFMA operand (row sums on the matrix pipe)
   __device__ static inline uint4 ones8() { return make_uint4(0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u); }
   // a.lo * b.lo + a.hi * b.hi + c in fp32 on packed pairs (v_dot2_f32_f16)
@@ -62,6 +67,10 @@ struct BF16 {
   }
   __device__ static inline floatx4 mfma(const uint4& a, const uint4& b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+  __device__ static inline floatx16 mfma32(const uint4& a, const uint4& b, floatx16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                     __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
   }
   __device__ static inline uint4 ones8() { return make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u); }
@@ -144,6 +153,13 @@ __device__ inline uint4 pack8(const floatx4& lo, const floatx4& hi) {
                     pack2<T>(hi[2], hi[3]));
 }
 
+// Registers 8 s .. 8 s + 7 of a 32x32 accumulator: one 32x32x16 MFMA operand.
+template <typename T>
+__device__ inline uint4 pack8(const floatx16& x, int s) {
+  return make_uint4(pack2<T>(x[8 * s], x[8 * s + 1]), pack2<T>(x[8 * s + 2], x[8 * s + 3]),
+                    pack2<T>(x[8 * s + 4], x[8 * s + 5]), pack2<T>(x[8 * s + 6], x[8 * s + 7]));
+}
+
 // LDS tile layout for 16-bit [64][D] tiles: row-major, no padding, 16-byte
 // chunks XOR-swizzled per row. gfx950 LDS has 64 banks of 4 bytes (one
 // 256-byte "bank row" per clock), so a read is conflict-free when the 16-byte
@@ -158,8 +174,20 @@ __device__ inline uint4 pack8(const floatx4& lo, const floatx4& hi) {
 // Tiles narrower than 256 bytes share a bank row between 256/(2D) rows; the
 // row bits that select the slice take the place of a. D = 16 keeps a 2-way
 // conflict (only 2 chunks per row).
-template <int D>
+// ROW32 (tiles read by v_mfma_f32_32x32x16): row reads take 32 consecutive rows
+// at one chunk, so the swizzle is a bijection of row & 15 (any 16 of them that
+// one clock serves land on distinct positions), and its low row bits sit above
+// the two chunk bits that a transposed read of 4 consecutive rows x 4
+// adjacent chunks covers.
+template <int D, bool ROW32 = false>
 __device__ inline int lds_swz(int row) {
+  if constexpr (ROW32) {
+    const int lo = (row >> 2) & 3;
+    if constexpr (D >= 128) return 4 * (row & 3) + lo;
+    else if constexpr (D == 64) return 4 * ((row >> 1) & 1) + lo;
+    else if constexpr (D == 32) return lo;
+    else return (row >> 3) & 1;
+  }
   const int b = (row >> 3) & 3;
   const int bb = 2 * (b & 1) + (b >> 1);
   if constexpr (D >= 128) return (4 * (row & 3) + bb) & (D / 8 - 1);
@@ -167,9 +195,9 @@ __device__ inline int lds_swz(int row) {
   else if constexpr (D == 32) return bb;
   else return 0;
 }
-template <int D>
+template <int D, bool ROW32 = false>
 __device__ inline int lds_off(int row, int col) {
-  return row * D + ((((col >> 3) ^ lds_swz<D>(row))) << 3) + (col & 7);
+  return row * D + ((((col >> 3) ^ lds_swz<D, ROW32>(row))) << 3) + (col & 7);
 }
 
 // Transposed MFMA operand from a swizzled 16-bit LDS tile via
@@ -191,17 +219,63 @@ __device__ inline uint4 lds_tr8(const uint16_t* tile, int k0, int n0, int lane) 
   return make_uint4(a.x, a.y, b.x, b.y);
 }
 // 16-byte row read (8 elements starting at a multiple-of-8 column).
-template <int D>
+template <int D, bool ROW32 = false>
 __device__ inline uint4 lds_row8(const uint16_t* tile, int row, int col) {
-  return *(const uint4*)(tile + lds_off<D>(row, col));
+  return *(const uint4*)(tile + lds_off<D, ROW32>(row, col));
 }
+
+// Operands of v_mfma_f32_32x32x16 (lane l: row or column l & 31, elements
+// 8 (l >> 5) .. +7 of the 16-long contraction) and its accumulator (lane l:
+// column l & 31, register r: row 8 (r >> 2) + 4 (l >> 5) + (r & 3)). Registers
+// 8 s .. 8 s + 7 of lane half hi therefore hold rows 16 s + 4 hi + (j & 3) +
+// 8 (j >> 2), j = 0 .. 7, and serve as an operand of a contraction over rows
+// 16 s .. 16 s + 15 whose other operand lists the same rows in the same order:
+// Lane32::cols gives lane l a column of exactly those rows, by two transposed
+// reads. (A tile of D = 16 columns has none past 15: lanes
+// 16 .. 31 of a half repeat columns 0 .. 15.)
+// The lane's byte offsets are computed once; rows 32 t / 16 s and the buffer are
+// constants of the instruction, chunks an XOR.
+template <int D>
+struct Lane32 {
+  int row;        // row l & 31, columns 8 (l >> 5) ..
+  int tr[2];      // rows 4 (l >> 5) + ((l & 15) >> 2) and that + 8, columns 16 ((l >> 4) & 1) + 4 (l & 3) ..
+  __device__ inline Lane32(int lane) {
+    const int hi = lane >> 5, i = lane & 15;
+    row = 2 * lds_off<D, true>(lane & 31, 8 * hi);
+    const int r = 4 * hi + (i >> 2), c = (D >= 32 ? 16 * ((lane >> 4) & 1) : 0) + 4 * (i & 3);
+    tr[0] = 2 * lds_off<D, true>(r, c);
+    tr[1] = 2 * lds_off<D, true>(r + 8, c);
+  }
+  // Row operand: rows 32 t + (l & 31), columns 16 ks + 8 (l >> 5) .. +7.
+  __device__ inline uint4 rows(const uint16_t* tile, int t, int ks) const {
+    return *(const uint4*)((const char*)tile + 64 * D * t + (row ^ (32 * ks)));
+  }
+  // Transposed operand: column 32 dt + (l & 31) of rows 16 st .. +15 in accumulator order.
+  __device__ inline uint4 cols(const uint16_t* tile, int st, int dt) const {
+    const char* p = (const char*)tile + 32 * D * st;
+    const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(p + (tr[0] ^ (64 * dt))));
+    const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(p + (tr[1] ^ (64 * dt))));
+    const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
+    return make_uint4(a.x, a.y, b.x, b.y);
+  }
+};
+__device__ inline floatx16 splat16(float x) {
+  return floatx16{x, x, x, x, x, x, x, x, x, x, x, x, x, x, x, x};
+}
+// The lane index afresh (mbcnt): not provably the one derived from threadIdx,
+// so that values derived from it late are not kept from the kernel's start.
+__device__ inline int lane_now() {
+  return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+}
+// Row (of 32) of register r in lane half hi of a 32x32 accumulator.
+__device__ inline int acc32_row(int r, int hi) { return 8 * (r >> 2) + 4 * hi + (r & 3); }
 
 // Stage a 64-row tile of a row-major [n, D] 16-bit matrix: each thread moves
 // P 16-byte chunks, consecutive threads covering consecutive bytes of a row.
 // The loads go through a buffer resource over the rows that exist, so rows at
 // or past n_rows read as zero without a per-element predicate, and the lane
 // offsets are 32-bit (chunk c of the tile sits at byte 16 c).
-template <int D, int NT = 256>
+template <int D, int NT = 256, bool ROW32 = false>
 struct RowTile {
   static constexpr int CPR = D / 8;          // 16-byte chunks per row
   static constexpr int CH = 64 * CPR;
@@ -229,7 +303,7 @@ struct RowTile {
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const int c = tid + NT * p;
-      if (c < CH) *(uint4*)(lds + lds_off<D>(c / CPR, (c % CPR) * 8)) = reg[p];
+      if (c < CH) *(uint4*)(lds + lds_off<D, ROW32>(c / CPR, (c % CPR) * 8)) = reg[p];
     }
   }
 };
@@ -303,7 +377,7 @@ __device__ inline void dma_wait() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 // blocks of 1 KB (block NW p + wave for p = 0, 1, ...); `off` is the lane's
 // element offset inside the tile for each block it moves (computed once).
 // Only for tiles whose 64 rows are all in bounds.
-template <int D, int NW = 4>
+template <int D, int NW = 4, bool ROW32 = false>
 struct DmaTile {
   static constexpr int NB = D / 8;                     // 1 KB blocks per tile
   static constexpr int NP = (NB + NW - 1) / NW;        // blocks per wave
@@ -316,11 +390,23 @@ struct DmaTile {
     for (int p = 0; p < NP; ++p) {
       const int e = (NW * p + wave) * 512 + 8 * lane;  // LDS element offset
       const int row = e / D, pch = (e % D) >> 3;
-      off[p] = row * D + ((pch ^ lds_swz<D>(row)) << 3);
+      off[p] = row * D + ((pch ^ lds_swz<D, ROW32>(row)) << 3);
     }
   }
-  // Rows r0 .. r0+63 of `base` through a buffer resource over those rows: the
-  // tile base is uniform, so a tile costs no per-lane address arithmetic.
+  // Rows r0 .. r0+63 (r0 < n_rows) of a matrix of n_rows rows through a buffer resource over
+  // those that exist: the tile base is uniform, so a tile costs no per-lane
+  // address arithmetic, and the resource's range check makes the rows past the
+  // last one zeros in LDS (no separate path for a ragged tile).
+  __device__ inline void load(const uint16_t* base, int r0, int n_rows, const uint16_t* lds) const {
+    const i32x4 rsrc = buffer_rsrc(base + (size_t)r0 * D, (n_rows - r0 < 64 ? n_rows - r0 : 64) * D * 2);
+    const uint32_t l0 = lds_addr(lds);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const int blk = NW * p + wave;
+      if (NB % NW == 0 || blk < NB) dma_buf16(rsrc, 2 * off[p], l0 + blk * 1024);
+    }
+  }
+  // The same for a tile known to be whole.
   __device__ inline void load(const uint16_t* base, int r0, const uint16_t* lds) const {
     const i32x4 rsrc = buffer_rsrc(base + (size_t)r0 * D, 64 * D * 2);
     const uint32_t l0 = lds_addr(lds);
@@ -517,6 +603,21 @@ struct LaneBits {
   }
 };
 
+// The same for a 32x32 accumulator: register r of lane half hi is bit
+// acc32_row(r, hi) of the 32-bit half of the word that belongs to its subtile.
+struct LaneBits32 {
+  uint32_t w;
+  __device__ inline LaneBits32(uint32_t half, int hi) : w(half >> (4 * hi)) {}
+  // 0 or -1: register r visible
+  __device__ inline int mask(int r) const {
+    return __builtin_amdgcn_sbfe((int)w, 8 * (r >> 2) + (r & 3), 1);
+  }
+  __device__ inline float pick(int r, float x, float other) const {
+    const int m = mask(r);
+    return __int_as_float((__float_as_int(x) & m) | (__float_as_int(other) & ~m));
+  }
+};
+
 // Is some (q, k) with q in [q_lo, q_hi], k in [k_lo, k_hi] (inclusive, absolute
 // positions, non-empty) visible under the token rule (k <= q) & (k < S | k >= q-W+1)?
 __device__ inline bool any_visible(long q_lo, long q_hi, long k_lo, long k_hi, long sink, long window) {
@@ -535,6 +636,13 @@ __device__ inline bool tile_all_visible(const Geom& g, int q_lo, int q_hi, int k
   const int qa = q_lo + g.q_off, qb = q_hi + g.q_off;
   if (k_hi > qa) return false;
   return (k_hi < g.sink) || (k_lo >= qb - g.window + 1);
+}
+
+// True when no row of [q_lo, q_hi] sees a key of the tile [k0, k0 + kTileN) under
+// the token rule (never for a tile the rule does not apply to).
+__host__ __device__ inline bool tile_unseen(const Geom& g, int q_lo, int q_hi, int k0) {
+  return g.causal != 0 && (k0 > q_hi + g.q_off ||
+                           (k0 >= g.sink && k0 + kTileN <= q_lo + g.q_off - word_window(g) + 1));
 }
 
 // XCD-aware remap: hardware dispatches workgroup b to XCD b % 8. Give each XCD
@@ -660,6 +768,20 @@ __device__ inline float wave_max16x4(float x) {
   return a;
 }
 #pragma clang diagnostic pop
+// Max / sum of lanes l and l ^ 32 (a column's two halves in a 32x32 accumulator).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ inline float half_max(float x) {
+  float a = x, b = x;
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1\n\tv_max_f32 %0, %0, %1" : "+v"(a), "+v"(b));
+  return a;
+}
+#pragma clang diagnostic pop
+__device__ inline float half_sum(float x) {
+  float a = x, b = x;
+  swap32(a, b);
+  return a + b;
+}
 __device__ inline float wave_sum16x4(float x) {
   float a = x, b = x;
   swap32(a, b);

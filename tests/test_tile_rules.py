@@ -1,0 +1,63 @@
+"""The rule by which a wave leaves a kv tile out (CPU).
+
+`tile_unseen` (graph-kernel-injection_amd/csrc/gki_common.cuh) must never hold
+for a tile of which some row sees a key under the oracle's token rule, and
+holds whenever no in-range row sees one (else work would be done for nothing).
+"""
+
+from __future__ import annotations
+
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+from oracle import streaming_oracle as so
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+REPO = os.path.dirname(HERE)
+CSRC = os.path.join(REPO, "graph-kernel-injection_amd", "csrc")
+TILE = 64
+
+
+@pytest.fixture(scope="module")
+def rules_exe(tmp_path_factory):
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not available")
+    exe = str(tmp_path_factory.mktemp("tile_rules") / "tile_rules_host")
+    subprocess.run([hipcc, "--offload-arch=gfx950", "-O1", "-std=c++17", f"-I{CSRC}",
+                    f"-I{os.path.join(REPO, 'include')}", os.path.join(HERE, "tile_rules_host.hip"),
+                    "-o", exe], check=True, capture_output=True, timeout=600)
+    return exe
+
+
+def test_unseen_tiles_are_exactly_those_without_a_visible_key(rules_exe):
+    rng = np.random.default_rng(5)
+    lines, want = [], []
+    for _ in range(150):
+        n_kv = int(rng.integers(1, 500))
+        n_q = int(rng.integers(1, 600))
+        causal = bool(rng.random() < 0.85)
+        sink = int(rng.choice([0, 1, 4, 64, 100]))
+        window = int(rng.choice([0, 1, 31, 64, 100, 700, 2**31 - 1]))
+        vis = so.token_mask(n_q, n_kv, sink, min(window, n_q + n_kv + 1)) if causal else np.ones((n_q, n_kv), bool)
+        for q_lo in range(0, n_q, 32):
+            for k0 in range(0, n_kv, TILE):
+                lines.append(f"{n_q} {n_kv} {int(causal)} {sink} {window} {q_lo} {q_lo + 31} {k0}")
+                want.append((not causal, bool(vis[q_lo:q_lo + 32, k0:k0 + TILE].any()), q_lo + 32 <= n_q))
+    out = subprocess.run([rules_exe], input="\n".join(lines) + "\n", capture_output=True, text=True, check=True,
+                         timeout=120).stdout.split()
+    assert len(out) == len(want)
+    skipped = 0
+    for line, got, (never, seen, whole) in zip(lines, out, want):
+        unseen = got == "1"
+        assert not (unseen and (seen or never)), line
+        # and no visited tile is for nothing, where every row exists (past the sinks; a window of 0 sees only those)
+        sink, window, k0 = (int(line.split()[i]) for i in (3, 4, 7))
+        if whole and not never and not seen and k0 >= sink and window > 0:
+            assert unseen, line
+        skipped += unseen
+    assert skipped > 1000
