@@ -3,10 +3,9 @@
 // Replaces the reference's three Triton launches in
 // `_BlockSparseFlashAttention.backward` (sparse_triton_kernel.py:719-777):
 //   * `_bwd_preprocess_kernel` (sparse_triton_kernel.py:354-392),
-//       Delta[q] = sum_d fp32(O) * fp32(dO) over the stored O: for 16-bit
-//       inputs inside dq_kernel_16, which runs first and stores -Delta for
-//       dK/dV; for fp32 inputs delta_kernel, before the other two. For 16-bit
-//       inputs the dQ kernel also turns the stored natural LSE into base 2
+//       Delta[q] = sum_d fp32(O) * fp32(dO) over the stored O, inside the dQ
+//       kernel, which runs first and stores it (negated for 16-bit inputs) for
+//       dK/dV. For 16-bit inputs the dQ kernel also turns the stored natural LSE into base 2
 //       once per row (second half of the row-term workspace), so the 16-bit
 //       kernels form P = exp(S scale - LSE) as one exp2 of an fma; the fp32
 //       kernels form it as exp2(fma(S, scale, -LSE) log2 e) from the stored
@@ -32,42 +31,8 @@
 namespace gki {
 namespace {
 
-// ---------------------------------------------------------------------------
-// Delta = rowsum(O * dO)
-// ---------------------------------------------------------------------------
-template <typename T, int D>
-__global__ __launch_bounds__(256) void delta_kernel(const typename T::storage* __restrict__ O,
-                                                    const typename T::storage* __restrict__ dO,
-                                                    float* __restrict__ delta, int64_t rows) {
-  constexpr int VEC = T::is_f32 ? 4 : 8;
-  constexpr int LPR = D / VEC;          // lanes per row (2..32)
-  constexpr int RPB = 256 / LPR;        // rows per block
-  const int tid = threadIdx.x;
-  const int64_t row = (int64_t)blockIdx.x * RPB + tid / LPR;
-  const int ch = tid % LPR;
-  float acc = 0.f;
-  if (row < rows) {
-    const uint4 a = *(const uint4*)(O + row * D + ch * VEC);
-    const uint4 b = *(const uint4*)(dO + row * D + ch * VEC);
-    if constexpr (T::is_f32) {
-      const float* fa = (const float*)&a;
-      const float* fb = (const float*)&b;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc += fa[i] * fb[i];
-    } else {
-      const uint16_t* ha = (const uint16_t*)&a;
-      const uint16_t* hb = (const uint16_t*)&b;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc += T::to_float(ha[i]) * T::to_float(hb[i]);
-    }
-  }
-#pragma unroll
-  for (int off = LPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
-  if (row < rows && ch == 0) delta[row] = acc;
-}
-
-// fp32 gradients accumulate one iteration (64 rows) at a time in a fresh
-// accumulator, which is then added to the running sum with its rounding error
+// fp32 gradients accumulate one staged step (16 or 32 rows per wave) at a time
+// in a fresh accumulator, which is then added to the running sum with its rounding error
 // kept exactly (TwoSum) in a compensation term: a long walk (the sink keys of a
 // long sequence, |dV| ~ 10 over thousands of rows) then rounds like a short
 // one. The result is sum + compensation.
@@ -82,34 +47,6 @@ __device__ inline void two_sum_fold(floatx4& sum, floatx4& comp, const floatx4& 
   }
 }
 
-template <int D>
-struct Stage32 {
-  static constexpr int LD = D + 4;
-  static constexpr int CPR = D / 4;
-  static constexpr int CH = 64 * CPR;
-  static constexpr int P = (CH + 255) / 256;
-  float4 reg[P];
-  __device__ inline void load(const float* base, int r0, int n_rows, int tid) {
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      const int c = tid + 256 * p;
-      const int r = c / CPR, ch = c - r * CPR;
-      reg[p] = (c < CH && r0 + r < n_rows) ? *(const float4*)(base + (size_t)(r0 + r) * D + ch * 4)
-                                           : make_float4(0, 0, 0, 0);
-    }
-  }
-  __device__ inline void store(float* rowmajor, int tid) const {
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      const int c = tid + 256 * p;
-      if (c < CH) {
-        const int r = c / CPR, ch = c - r * CPR;
-        *(float4*)(&rowmajor[r * LD + ch * 4]) = reg[p];
-      }
-    }
-  }
-};
-
 // Work item of workgroup b in the dK / dV grid: the items of one (b, kv head)
 // are consecutive, XCD-remapped so that neighbouring kv tiles of a head (which
 // share most q tiles) run on one XCD and meet in its L2.
@@ -119,6 +56,16 @@ struct KvItem {
 __device__ inline KvItem kv_item_of(int b, int BH, const KvWork& w, int& bh) {
   const int wg = xcd_remap(b, w.n_items * BH);
   bh = wg / w.n_items;
+  const int4 t = ((const int4*)w.items)[wg - bh * w.n_items];
+  return {t.x, t.y, t.z, t.w};
+}
+
+// The same for items cut into `parts` workgroups each (work_parts_grid); bh < 0
+// for a workgroup past the last.
+__device__ inline KvItem kv_item_part_of(int b, int BH, int parts, const KvWork& w, int& bh, int& part) {
+  const int wg = work_part_of(b, w.n_items * BH, parts, nullptr, part);
+  bh = wg < 0 ? -1 : wg / w.n_items;
+  if (wg < 0) return {0, 0, 0, -1};
   const int4 t = ((const int4*)w.items)[wg - bh * w.n_items];
   return {t.x, t.y, t.z, t.w};
 }
@@ -602,155 +549,226 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
 // ---------------------------------------------------------------------------
 // dK / dV, fp32
 // ---------------------------------------------------------------------------
-template <int D>
-struct DkdvSmem32 {
-  float q[64 * (D + 4)];
-  float dout[64 * (D + 4)];
-  float lse[64];
-  float dlt[64];
-};
-
-// One wave per SIMD from head_dim 64 up: the compensated accumulators, the
-// register-staged next tile and the four MFMA chains then fit in VGPRs + AGPRs
-// (at two waves per SIMD, head_dim 64 spilled 400 bytes per lane: the c1
-// backward took 0.284 against 0.213 ms, a B1 H16 N8192 fp32 backward 2.65
-// against 2.0 ms).
-template <int D>
-__global__ __launch_bounds__(256, D >= 64 ? 1 : 2) void dkdv_kernel_32(
+// Bound by the fp32 matrix cores and, beside them, the VALU (exponents, the
+// compensated folds): B1 H16 N8192 D64 W1024 1281 -> 763 us (dQ 671 -> 557, the
+// forward 432 -> 335; 459, 344 and 229 us at the nominal MFMA rate) against
+// 4-byte LDS reads, tiles staged through registers behind two barriers, folds
+// per 16 rows and a separate Delta launch; D128 N4096 backward 2.08 -> 1.41 ms.
+// Three waves per SIMD ran 12% slower than two (head_dim 64).
+// As the forward, a workgroup's four waves are KB blocks of 16 kv rows x 4 / KB
+// shares of the q rows of each staged step (16 rows each; two subtiles when
+// KB = 4), and an item of the work list is 4 / KB workgroups. The shares' sums
+// meet through LDS at the end, in order.
+template <int D, int KB>
+__global__ __launch_bounds__(256, D >= 128 || (D == 64 && KB == 1) ? 1 : 2) void dkdv_kernel_32(
     Geom g, const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
     const float* __restrict__ dO, float* __restrict__ dK, float* __restrict__ dV,
     const float* __restrict__ LSE, const float* __restrict__ Delta,
     const int32_t* __restrict__ col_ptr, const int32_t* __restrict__ col_idx, KvWork w) {
-  // LSE: the forward's natural LSE; Delta: rowsum(O dO) from delta_kernel
-  constexpr int KS = D / 4;
-  constexpr int DT = D / 16;
-  constexpr int LD = D + 4;
-  // the four key subtiles unrolled below head_dim 128; at 128 a rolled loop
-  // keeps the kernel in VGPRs + AGPRs (unrolled it spilled 868 bytes per lane)
-  constexpr int kSubtileUnroll = D >= 128 ? 1 : 4;
-  __shared__ __align__(16) DkdvSmem32<D> sm;
-  Stage32<D> sq, sdo;
+  // LSE: the forward's natural LSE; Delta: rowsum(O dO) from the dQ kernel, which runs first
+  constexpr int DJ = D / 16;
+  constexpr int QS = 4 / KB;                 // q-row shares
+  constexpr int TR = QS == 4 ? 64 : 32;      // q rows per staged step
+  constexpr int SUBS = TR / (16 * QS);
+  constexpr int HALVES = kTileM / TR;
+  constexpr int DV = D >= 64 ? D / 64 : 1;
+  constexpr int DE = D / (16 * DV);
+  __shared__ __align__(16) float sq[2][TR * D];
+  __shared__ __align__(16) float sdo[2][TR * D];
+  __shared__ __align__(16) float slse[2][64];
+  __shared__ __align__(16) float sdlt[2][64];
 
-  // one workgroup per (b, kv head, work item), as in the 16-bit kernel
   const int BH = g.B * g.H_kv;
-  int bh;
-  const KvItem item = kv_item_of(blockIdx.x, BH, w, bh);
+  int bh, part;
+  const KvItem item = kv_item_part_of(blockIdx.x, BH, QS, w, bh, part);
+  if (bh < 0) return;
   // an empty column (no kept q tile) only writes zeros: its K / V rows are not read
   const bool has_work = item.it1 > item.it0;
   const int kt = item.kt;
   const size_t kb = (size_t)bh * g.n_kv * D;
   const int bhq0 = (bh / g.H_kv) * g.H + (bh % g.H_kv) * g.group;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = lane >> 4, col = lane & 15;
-  const int k_w = kt * kTileN + wave * 16;
+  const int share = wave / KB;
+  const int kr0 = 16 * (part * KB + wave % KB);          // the wave's rows of the kv tile
+  const int k_w = kt * kTileN + kr0;
   const int my_kv = k_w + col;
 
-  float kf[KS], vf[KS];
+  floatx4 kf[DJ], vf[DJ];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
+  for (int j = 0; j < DJ; ++j) {
     const bool ok = has_work && my_kv < g.n_kv;
-    kf[ks] = ok ? K[kb + (size_t)my_kv * D + 4 * ks + grp] : 0.f;
-    vf[ks] = ok ? V[kb + (size_t)my_kv * D + 4 * ks + grp] : 0.f;
+    const size_t at = kb + (size_t)my_kv * D + 16 * j + 4 * grp;
+    kf[j] = ok ? *(const floatx4*)(K + at) : floatx4{0.f, 0.f, 0.f, 0.f};
+    vf[j] = ok ? *(const floatx4*)(V + at) : floatx4{0.f, 0.f, 0.f, 0.f};
   }
-  floatx4 dk[DT], dv[DT], ck[DT], cv[DT];   // running sums and their compensation
+  // running sums and their compensation; tile (v, e) column x is element 64 v + DE x + e
+  floatx4 dk[DV][DE], dv[DV][DE], ck[DV][DE], cv[DV][DE];
 #pragma unroll
-  for (int i = 0; i < DT; ++i) dk[i] = dv[i] = ck[i] = cv[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int v = 0; v < DV; ++v)
+#pragma unroll
+    for (int e = 0; e < DE; ++e) dk[v][e] = dv[v][e] = ck[v][e] = cv[v][e] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   const int e_beg = col_ptr[kt], e_end = col_ptr[kt + 1];
-  float lreg = 0.f, dreg = 0.f;
-  auto load_tile = [&](int q0, int bhq) {
-    const size_t qb = (size_t)bhq * g.n_q * D;
-    sq.load(Q + qb, q0, g.n_q, tid);
-    sdo.load(dO + qb, q0, g.n_q, tid);
-    if (tid < 64) {
-      const int r = q0 + tid;
-      lreg = r < g.n_q ? LSE[(size_t)bhq * g.n_q + r] : 0.f;
-      dreg = r < g.n_q ? Delta[(size_t)bhq * g.n_q + r] : 0.f;
-    }
-  };
+  DmaTileF32<D, TR> dma;
+  dma.init(tid);
   const int L = e_end - e_beg;
-  const int n_it = item.it1 - item.it0;
+  const int n_step = (item.it1 - item.it0) * HALVES;
   const int h0 = L > 0 ? item.it0 / L : 0;
   int e_nx = e_beg + (item.it0 - h0 * L), q_nx = bhq0 + h0;
-  if (n_it > 0) load_tile((col_idx[e_nx] & kIdxMask) * kTileM, q_nx);
+  auto stage = [&](int s, int buf) {
+    const int q0 = (col_idx[e_nx] & kIdxMask) * kTileM + (s % HALVES) * TR;
+    const size_t qb = (size_t)q_nx * g.n_q * D;
+    dma.load(Q + qb, q0, g.n_q, sq[buf]);
+    dma.load(dO + qb, q0, g.n_q, sdo[buf]);
+    if (wave < 2) {      // rows past n_q re-read the last one, which only masked elements see
+      const float* src = (wave == 0 ? LSE : Delta) + (size_t)q_nx * g.n_q + min(q0 + lane, g.n_q - 1);
+      dma_load4(src, lds_addr(wave == 0 ? slse[buf] : sdlt[buf]));
+    }
+  };
+  dma_wait();          // the K / V loads, before any LDS-DMA is in flight
+  if (n_step > 0) stage(0, 0);
+  dma_wait();
+  __syncthreads();
 
-  const int kv_hi_wave = min(k_w + 15, g.n_kv - 1);
-  for (int it = 0; it < n_it; ++it) {
+  const int kv_hi = min(k_w + 15, g.n_kv - 1);
+  for (int s = 0; s < n_step; ++s) {
+    const int buf = s & 1;
     const int ent = col_idx[e_nx];
-    if (++e_nx == e_end) {
+    if (s % HALVES == HALVES - 1 && ++e_nx == e_end) {
       e_nx = e_beg;
       ++q_nx;
     }
-    const int q0 = (ent & kIdxMask) * kTileM;
+    if (s + 1 < n_step) stage(s + 1, buf ^ 1);
+    const float *cq = sq[buf], *cdo = sdo[buf];
+    const int r0 = 16 * SUBS * share;                    // the wave's first q row of the step
+    const int q0 = (ent & kIdxMask) * kTileM + (s % HALVES) * TR + r0;
     const bool partial = (ent >> kPartialBit) & 1;
-    __syncthreads();
-    sq.store(sm.q, tid);
-    sdo.store(sm.dout, tid);
-    if (tid < 64) {
-      sm.lse[tid] = lreg;
-      sm.dlt[tid] = dreg;
-    }
-    __syncthreads();
-    if (it + 1 < n_it) load_tile((col_idx[e_nx] & kIdxMask) * kTileM, q_nx);
-
-    const bool need_mask = partial || (q0 + kTileM > g.n_q) || (k_w + 15 >= g.n_kv) ||
-                           !tile_all_visible(g, q0, min(q0 + kTileM - 1, g.n_q - 1), k_w, kv_hi_wave);
-#pragma unroll kSubtileUnroll
-    for (int t = 0; t < 4; ++t) {
-      floatx4 fk[DT], fv[DT];          // this subtile's 16 rows, folded in compensated
+    const bool need_mask = partial || (q0 + 16 * SUBS > g.n_q) || (k_w + 15 >= g.n_kv) ||
+                           !tile_all_visible(g, q0, q0 + 16 * SUBS - 1, k_w, kv_hi);
+    uint64_t bits = ~0ull;
+    if (need_mask) bits = col_valid_bits(g, my_kv, q0, partial);
+    const LaneBits16 vis(bits, grp);
+    floatx4 fk[DV][DE], fv[DV][DE];    // this step's rows, folded in compensated
 #pragma unroll
-      for (int i = 0; i < DT; ++i) fk[i] = fv[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-      const int r = rho(t, col);
-      const floatx4 s = mfma_f32_dot<KS>([&](int ks) { return sm.q[r * LD + 4 * ks + grp]; },
-                                         [&](int ks) { return kf[ks]; });
-      const floatx4 dp = mfma_f32_dot<KS>([&](int ks) { return sm.dout[r * LD + 4 * ks + grp]; },
-                                          [&](int ks) { return vf[ks]; });
+    for (int v = 0; v < DV; ++v)
+#pragma unroll
+      for (int e = 0; e < DE; ++e) fk[v][e] = fv[v][e] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < SUBS; ++t) {
+      const int r = r0 + 16 * t;
+      const floatx4 sc = mfma_f32_dot<4 * DJ>(
+          [&](int j) { return *(const floatx4*)(cq + off_f32<D>(r + col, 4 * j + grp)); }, kf);
+      const floatx4 dp = mfma_f32_dot<4 * DJ>(
+          [&](int j) { return *(const floatx4*)(cdo + off_f32<D>(r + col, 4 * j + grp)); }, vf);
+      const floatx4 lse4 = *(const floatx4*)(&slse[buf][r + 4 * grp]);
+      const floatx4 dlt4 = *(const floatx4*)(&sdlt[buf][r + 4 * grp]);
+      floatx4 pv, ds;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int qr = rho(t, 4 * grp + i);
-        float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], g.scale, -sm.lse[qr]) * kLog2e);
-        if (need_mask && !elem_valid(g, q0 + qr, my_kv, partial)) pv = 0.f;
-        const float dsv = pv * (dp[i] - sm.dlt[qr]) * g.scale;
+        pv[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], g.scale, -lse4[i]) * kLog2e);
+        if (need_mask) pv[i] = vis.keep(t, i, pv[i]);
+        ds[i] = pv[i] * (dp[i] - dlt4[i]) * g.scale;
+      }
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          fv[dt] = mfma_f32(pv, sm.dout[qr * LD + 16 * dt + col], fv[dt]);
-          fk[dt] = mfma_f32(dsv, sm.q[qr * LD + 16 * dt + col], fk[dt]);
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int v = 0; v < DV; ++v) {
+          const floatx4 xo = cols_f32<D, DE>(cdo, r + 4 * grp + i, v, col);
+          const floatx4 xq = cols_f32<D, DE>(cq, r + 4 * grp + i, v, col);
+#pragma unroll
+          for (int e = 0; e < DE; ++e) {
+            fv[v][e] = mfma_f32(pv[i], xo[e], fv[v][e]);
+            fk[v][e] = mfma_f32(ds[i], xq[e], fk[v][e]);
+          }
         }
-      }
+    }
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        two_sum_fold(dk[dt], ck[dt], fk[dt]);
-        two_sum_fold(dv[dt], cv[dt], fv[dt]);
+    for (int v = 0; v < DV; ++v)
+#pragma unroll
+      for (int e = 0; e < DE; ++e) {
+        two_sum_fold(dk[v][e], ck[v][e], fk[v][e]);
+        two_sum_fold(dv[v][e], cv[v][e], fv[v][e]);
       }
+    dma_wait();        // the next step's LDS-DMA has landed before the barrier
+    __syncthreads();
+  }
+  if constexpr (QS > 1) {
+    // shares 1 .. QS - 1 hand their sums over through LDS (free: every wave
+    // passed the last barrier); share 0 folds them in, in order
+    constexpr int SZ = 2 * 2 * 16 * D;                   // dk, ck, dv, cv of a wave
+    static_assert((QS - 1) * KB * SZ <= 2 * 2 * TR * D, "the sums fit the staging buffers");
+    float* red = sq[0];                                  // sq and sdo are contiguous (one array each, in order)
+    float* red2 = sdo[0];
+    const int blk = wave % KB;
+    // dk / ck through sq, dv / cv through sdo
+    const size_t at = ((size_t)(share - 1) * KB + blk) * (SZ / 2) + lane;
+    if (share > 0) {
+#pragma unroll
+      for (int v = 0; v < DV; ++v)
+#pragma unroll
+        for (int e = 0; e < DE; ++e)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const size_t o = at + 128 * ((v * DE + e) * 4 + i);
+            red[o] = dk[v][e][i];
+            red[o + 64] = ck[v][e][i];
+            red2[o] = dv[v][e][i];
+            red2[o + 64] = cv[v][e][i];
+          }
+    }
+    __syncthreads();
+    if (share > 0) return;
+#pragma unroll
+    for (int x = 1; x < QS; ++x) {
+      const size_t from = ((size_t)(x - 1) * KB + blk) * (SZ / 2) + lane;
+#pragma unroll
+      for (int v = 0; v < DV; ++v)
+#pragma unroll
+        for (int e = 0; e < DE; ++e) {
+          floatx4 a, b;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const size_t o = from + 128 * ((v * DE + e) * 4 + i);
+            a[i] = red[o];
+            b[i] = red2[o];
+            ck[v][e][i] += red[o + 64];
+            cv[v][e][i] += red2[o + 64];
+          }
+          two_sum_fold(dk[v][e], ck[v][e], a);
+          two_sum_fold(dv[v][e], cv[v][e], b);
+        }
     }
   }
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) {
-    dk[dt] += ck[dt];
-    dv[dt] += cv[dt];
-  }
-  if (item.pslot >= 0) {             // a split column: partials for the reduce
-    float* pk = w.partials + ((size_t)bh * w.n_pslots + item.pslot) * 2 * (kTileN * D);
-    float* pv = pk + kTileN * D;
+  for (int v = 0; v < DV; ++v)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = wave * 16 + 4 * grp + i;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        pk[r * D + 16 * dt + col] = dk[dt][i];
-        pv[r * D + 16 * dt + col] = dv[dt][i];
-      }
+    for (int e = 0; e < DE; ++e) {
+      dk[v][e] += ck[v][e];
+      dv[v][e] += cv[v][e];
     }
-    return;
-  }
+  // lane: kv rows 4 grp + i of the wave's 16, elements 64 v + DE col + e
+  const bool split = item.pslot >= 0;                    // a split column: partials for the reduce
+  float* pk = split ? w.partials + ((size_t)bh * w.n_pslots + item.pslot) * 2 * (kTileN * D) + kr0 * D
+                    : dK + kb + (size_t)k_w * D;
+  float* pv = split ? w.partials + ((size_t)bh * w.n_pslots + item.pslot) * 2 * (kTileN * D) + (kTileN + kr0) * D
+                    : dV + kb + (size_t)k_w * D;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int row = k_w + 4 * grp + i;
-    if (row < g.n_kv) {
+    const int row = 4 * grp + i;
+    if (!split && k_w + row >= g.n_kv) continue;
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        dK[kb + (size_t)row * D + 16 * dt + col] = dk[dt][i];
-        dV[kb + (size_t)row * D + 16 * dt + col] = dv[dt][i];
+    for (int v = 0; v < DV; ++v) {
+      const int c = row * D + 64 * v + DE * col;
+      if constexpr (DE == 4) {
+        *(floatx4*)(pk + c) = floatx4{dk[v][0][i], dk[v][1][i], dk[v][2][i], dk[v][3][i]};
+        *(floatx4*)(pv + c) = floatx4{dv[v][0][i], dv[v][1][i], dv[v][2][i], dv[v][3][i]};
+      } else {
+#pragma unroll
+        for (int e = 0; e < DE; ++e) {
+          pk[c + e] = dk[v][e][i];
+          pv[c + e] = dv[v][e][i];
+        }
       }
     }
   }
@@ -1110,117 +1128,175 @@ __global__ __launch_bounds__(256, 4) void dq_kernel_q64(
 // ---------------------------------------------------------------------------
 // dQ, fp32
 // ---------------------------------------------------------------------------
-template <int D>
-struct DqSmem32 {
-  float k[64 * (D + 4)];
-  float v[64 * (D + 4)];
-};
-
-// One wave per SIMD at head_dim 128 (two spilled 764 bytes per lane). At 64
-// two waves win on full grids (B1 H16 N8192 fp32 backward 2.33 -> 1.99 ms
-// against one wave; equal on c1).
-template <int D>
-__global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void dq_kernel_32(
+// Blocks and shares as in the forward (QB blocks of 16 q rows x 4 / QB shares
+// of the keys). Also Delta = rowsum(O dO) of its rows, for itself and for the
+// dK/dV kernel, which runs next.
+template <int D, int QB>
+__global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : 2) void dq_kernel_32(
     Geom g, const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
-    const float* __restrict__ dO, float* __restrict__ dQ, const float* __restrict__ LSE,
-    const float* __restrict__ Delta, const int32_t* __restrict__ row_ptr,
+    const float* __restrict__ O, const float* __restrict__ dO, float* __restrict__ dQ,
+    const float* __restrict__ LSE, float* __restrict__ Delta, const int32_t* __restrict__ row_ptr,
     const int32_t* __restrict__ row_idx, int n_qt, const int32_t* __restrict__ dq_order) {
-  constexpr int KS = D / 4;
-  constexpr int DT = D / 16;
-  constexpr int LD = D + 4;
-  // the four key subtiles in a rolled loop at head_dim 64: two waves per SIMD
-  // then fit without scratch (209 VGPRs; unrolled, 36 bytes spilled per lane)
-  constexpr int kSubtileUnroll = D == 64 ? 1 : 4;
-  __shared__ __align__(16) DqSmem32<D> sm;
-  Stage32<D> sk, sv;
+  constexpr int DJ = D / 16;
+  constexpr int KB = 4 / QB;
+  constexpr int TR = KB == 4 ? 64 : 32;
+  constexpr int SUBS = TR / (16 * KB);
+  constexpr int HALVES = kTileN / TR;
+  constexpr int DV = D >= 64 ? D / 64 : 1;
+  constexpr int DE = D / (16 * DV);
+  __shared__ __align__(16) float sk[2][TR * D];
+  __shared__ __align__(16) float sv[2][TR * D];
 
-  const int n_wg = n_qt * g.B * g.H;
-  const int wg = work_of(blockIdx.x, n_wg, dq_order);
+  int part;
+  const int wg = work_part_of(blockIdx.x, n_qt * g.B * g.H, KB, dq_order, part);
   if (wg < 0) return;
   const int bh = wg / n_qt, qt = wg - bh * n_qt;
   const size_t qb = (size_t)bh * g.n_q * D;
   const size_t kb = (size_t)kv_bh(g, bh) * g.n_kv * D;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = lane >> 4, col = lane & 15;
-  const int q0 = qt * kTileM + wave * 16;
+  const int share = wave / QB;
+  const int q0 = qt * kTileM + 16 * (part * QB + wave % QB);
   const int my_q = q0 + col;
 
-  float qf[KS], df[KS];
+  floatx4 qf[DJ], df[DJ];
+  float dlt = 0.f;
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
+  for (int j = 0; j < DJ; ++j) {
     const bool ok = my_q < g.n_q;
-    qf[ks] = ok ? Q[qb + (size_t)my_q * D + 4 * ks + grp] : 0.f;
-    df[ks] = ok ? dO[qb + (size_t)my_q * D + 4 * ks + grp] : 0.f;
+    const size_t at = qb + (size_t)my_q * D + 16 * j + 4 * grp;
+    qf[j] = ok ? *(const floatx4*)(Q + at) : floatx4{0.f, 0.f, 0.f, 0.f};
+    df[j] = ok ? *(const floatx4*)(dO + at) : floatx4{0.f, 0.f, 0.f, 0.f};
+    const floatx4 ov = ok ? *(const floatx4*)(O + at) : floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dlt = __builtin_fmaf(ov[i], df[j][i], dlt);
   }
+  dlt = wave_sum16x4(dlt);
   const float lse = my_q < g.n_q ? LSE[(size_t)bh * g.n_q + my_q] : 0.f;   // natural
-  const float dlt = my_q < g.n_q ? Delta[(size_t)bh * g.n_q + my_q] : 0.f;
-  floatx4 dq[DT], cq[DT];              // running sum and its compensation (two_sum_fold)
+  if (my_q < g.n_q && grp == 0 && share == 0) Delta[(size_t)bh * g.n_q + my_q] = dlt;
+  floatx4 dq[DV][DE], cq[DV][DE];      // running sum and its compensation (two_sum_fold)
 #pragma unroll
-  for (int i = 0; i < DT; ++i) dq[i] = cq[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int v = 0; v < DV; ++v)
+#pragma unroll
+    for (int e = 0; e < DE; ++e) dq[v][e] = cq[v][e] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  const int e_beg = row_ptr[qt], e_end = row_ptr[qt + 1];
-  if (e_beg < e_end) {
-    const int k0 = (row_idx[e_beg] & kIdxMask) * kTileN;
-    sk.load(K + kb, k0, g.n_kv, tid);
-    sv.load(V + kb, k0, g.n_kv, tid);
-  }
-  const int q_hi_wave = min(q0 + 15, g.n_q - 1);
-  for (int e = e_beg; e < e_end; ++e) {
-    const int ent = row_idx[e];
-    const int k0 = (ent & kIdxMask) * kTileN;
-    const bool partial = (ent >> kPartialBit) & 1;
-    __syncthreads();
-    sk.store(sm.k, tid);
-    sv.store(sm.v, tid);
-    __syncthreads();
-    if (e + 1 < e_end) {
-      const int k1 = (row_idx[e + 1] & kIdxMask) * kTileN;
-      sk.load(K + kb, k1, g.n_kv, tid);
-      sv.load(V + kb, k1, g.n_kv, tid);
-    }
-    const bool need_mask = partial || (q0 + 15 >= g.n_q) || (k0 + kTileN > g.n_kv) ||
-                           !tile_all_visible(g, q0, q_hi_wave, k0, k0 + kTileN - 1);
-#pragma unroll kSubtileUnroll
-    for (int t = 0; t < 4; ++t) {
-      floatx4 fq[DT];                  // this subtile's 16 keys, folded in compensated
+  const int e_beg = row_ptr[qt], n_step = (row_ptr[qt + 1] - e_beg) * HALVES;
+  DmaTileF32<D, TR> dma;
+  dma.init(tid);
+  auto step_k0 = [&](int s) {
+    return (row_idx[e_beg + s / HALVES] & kIdxMask) * kTileN + (s % HALVES) * TR;
+  };
+  auto stage = [&](int s, int buf) {
+    const int k0 = step_k0(s);
+    dma.load(K + kb, k0, g.n_kv, sk[buf]);
+    dma.load(V + kb, k0, g.n_kv, sv[buf]);
+  };
+  dma_wait();          // the row loads, before any LDS-DMA is in flight
+  if (n_step > 0) stage(0, 0);
+  dma_wait();
+  __syncthreads();
+  const int q_hi = min(q0 + 15, g.n_q - 1);
+  for (int s = 0; s < n_step; ++s) {
+    const int buf = s & 1;
+    const bool partial = (row_idx[e_beg + s / HALVES] >> kPartialBit) & 1;
+    if (s + 1 < n_step) stage(s + 1, buf ^ 1);
+    const float *ck = sk[buf], *cv = sv[buf];
+    const int r0 = 16 * SUBS * share;
+    const int k0 = step_k0(s) + r0;                      // the wave's first key
+    const bool need_mask = partial || (q0 + 15 >= g.n_q) || (k0 + 16 * SUBS > g.n_kv) ||
+                           !tile_all_visible(g, q0, q_hi, k0, k0 + 16 * SUBS - 1);
+    uint64_t bits = ~0ull;
+    if (need_mask) bits = row_valid_bits(g, my_q, k0, partial);
+    const LaneBits16 vis(bits, grp);
+    floatx4 fq[DV][DE];                // this step's keys, folded in compensated
 #pragma unroll
-      for (int i = 0; i < DT; ++i) fq[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-      const int r = rho(t, col);
-      const floatx4 s = mfma_f32_dot<KS>([&](int ks) { return sm.k[r * LD + 4 * ks + grp]; },
-                                         [&](int ks) { return qf[ks]; });
-      const floatx4 dp = mfma_f32_dot<KS>([&](int ks) { return sm.v[r * LD + 4 * ks + grp]; },
-                                          [&](int ks) { return df[ks]; });
+    for (int v = 0; v < DV; ++v)
+#pragma unroll
+      for (int e = 0; e < DE; ++e) fq[v][e] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < SUBS; ++t) {
+      const int r = r0 + 16 * t;
+      const floatx4 sc = mfma_f32_dot<4 * DJ>(
+          [&](int j) { return *(const floatx4*)(ck + off_f32<D>(r + col, 4 * j + grp)); }, qf);
+      const floatx4 dp = mfma_f32_dot<4 * DJ>(
+          [&](int j) { return *(const floatx4*)(cv + off_f32<D>(r + col, 4 * j + grp)); }, df);
+      floatx4 ds;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int kr = rho(t, 4 * grp + i);
-        float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], g.scale, -lse) * kLog2e);
-        if (need_mask && !elem_valid(g, my_q, k0 + kr, partial)) pv = 0.f;
-        const float dsv = pv * (dp[i] - dlt) * g.scale;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) fq[dt] = mfma_f32(sm.k[kr * LD + 16 * dt + col], dsv, fq[dt]);
+        float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], g.scale, -lse) * kLog2e);
+        if (need_mask) pv = vis.keep(t, i, pv);
+        ds[i] = pv * (dp[i] - dlt) * g.scale;
       }
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) two_sum_fold(dq[dt], cq[dt], fq[dt]);
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int v = 0; v < DV; ++v) {
+          const floatx4 x = cols_f32<D, DE>(ck, r + 4 * grp + i, v, col);
+#pragma unroll
+          for (int e = 0; e < DE; ++e) fq[v][e] = mfma_f32(x[e], ds[i], fq[v][e]);
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < DV; ++v)
+#pragma unroll
+      for (int e = 0; e < DE; ++e) two_sum_fold(dq[v][e], cq[v][e], fq[v][e]);
+    dma_wait();        // the next step's LDS-DMA has landed before the barrier
+    __syncthreads();
+  }
+  if constexpr (KB > 1) {              // the shares' sums, through LDS, in order
+    constexpr int SZ = 2 * 16 * D;                       // dq, cq of a wave
+    static_assert((KB - 1) * QB * SZ <= 2 * TR * D, "the sums fit one staging array");
+    float* red = sk[0];
+    const int blk = wave % QB;
+    if (share > 0) {
+      float* dst = red + ((size_t)(share - 1) * QB + blk) * SZ + lane;
+#pragma unroll
+      for (int v = 0; v < DV; ++v)
+#pragma unroll
+        for (int e = 0; e < DE; ++e)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            dst[128 * ((v * DE + e) * 4 + i)] = dq[v][e][i];
+            dst[128 * ((v * DE + e) * 4 + i) + 64] = cq[v][e][i];
+          }
+    }
+    __syncthreads();
+    if (share > 0) return;
+#pragma unroll
+    for (int x = 1; x < KB; ++x) {
+      const float* src = red + ((size_t)(x - 1) * QB + blk) * SZ + lane;
+#pragma unroll
+      for (int v = 0; v < DV; ++v)
+#pragma unroll
+        for (int e = 0; e < DE; ++e) {
+          floatx4 a;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            a[i] = src[128 * ((v * DE + e) * 4 + i)];
+            cq[v][e][i] += src[128 * ((v * DE + e) * 4 + i) + 64];
+          }
+          two_sum_fold(dq[v][e], cq[v][e], a);
+        }
     }
   }
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) dq[dt] += cq[dt];
+  for (int v = 0; v < DV; ++v)
+#pragma unroll
+    for (int e = 0; e < DE; ++e) dq[v][e] += cq[v][e];
   if (my_q < g.n_q) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      float4 w = make_float4(dq[dt][0], dq[dt][1], dq[dt][2], dq[dt][3]);
-      *(float4*)(dQ + qb + (size_t)my_q * D + 16 * dt + 4 * grp) = w;
-    }
+    for (int v = 0; v < DV; ++v)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float* dst = dQ + qb + (size_t)my_q * D + 64 * v + DE * (4 * grp + i);
+        if constexpr (DE == 4) {
+          *(floatx4*)dst = floatx4{dq[v][0][i], dq[v][1][i], dq[v][2][i], dq[v][3][i]};
+        } else {
+#pragma unroll
+          for (int e = 0; e < DE; ++e) dst[e] = dq[v][e][i];
+        }
+      }
   }
-}
-
-template <typename T, int D>
-void launch_delta(const void* o, const void* dout, float* delta, int64_t rows, hipStream_t stream) {
-  constexpr int VEC = T::is_f32 ? 4 : 8;
-  constexpr int RPB = 256 / (D / VEC);
-  const int64_t grid = (rows + RPB - 1) / RPB;
-  hipLaunchKernelGGL((delta_kernel<T, D>), dim3((unsigned)grid), dim3(256), 0, stream,
-                     (const typename T::storage*)o, (const typename T::storage*)dout, delta, rows);
 }
 
 // dQ first: it also produces -Delta and the base-2 LSE rows, which dK/dV reads
@@ -1269,19 +1345,29 @@ int launch_bwd(int dtype, const Geom& g, const void* q, const void* k, const voi
                const int32_t* row_ptr, const int32_t* row_idx, int n_qt, const int32_t* dq_order,
                const int32_t* col_ptr, const int32_t* col_idx, const KvWork& w, hipStream_t stream) {
   const int BH = g.B * g.H, BHkv = g.B * g.H_kv;
-  const int64_t rows = (int64_t)BH * g.n_q;
-  const dim3 kv_grid(w.n_items * BHkv), red_grid(w.n_split * BHkv * kReduceWgPerTile<D>);
+  const dim3 red_grid(w.n_split * BHkv * kReduceWgPerTile<D>);
   if (dtype == kF32) {
-    launch_delta<F32, D>(o, dout, delta, rows, stream);
-    hipLaunchKernelGGL(dkdv_kernel_32<D>, kv_grid, dim3(256), 0, stream, g, (const float*)q,
-                       (const float*)k, (const float*)v, (const float*)dout, (float*)dk, (float*)dv,
-                       lse, delta, col_ptr, col_idx, w);
+    // dQ first: it also writes Delta, which dK/dV reads
+    const int qgrid = n_qt * BH, kgrid = w.n_items * BHkv;
+#define GKI_DQ32(QB)                                                                                \
+  hipLaunchKernelGGL((dq_kernel_32<D, QB>), dim3(work_parts_grid(qgrid, 4 / QB)), dim3(256), 0,     \
+                     stream, g, (const float*)q, (const float*)k, (const float*)v, (const float*)o, \
+                     (const float*)dout, (float*)dq, lse, delta, row_ptr, row_idx, n_qt, dq_order)
+#define GKI_DKDV32(KB)                                                                              \
+  hipLaunchKernelGGL((dkdv_kernel_32<D, KB>), dim3(work_parts_grid(kgrid, 4 / KB)), dim3(256), 0,   \
+                     stream, g, (const float*)q, (const float*)k, (const float*)v,                  \
+                     (const float*)dout, (float*)dk, (float*)dv, lse, delta, col_ptr, col_idx, w)
+    if (qgrid <= kF32SplitGrid4) GKI_DQ32(1);
+    else if (qgrid <= kF32SplitGrid2) GKI_DQ32(2);
+    else GKI_DQ32(4);
+    if (D <= 64 && kgrid <= kF32SplitGrid4) GKI_DKDV32((D <= 64 ? 1 : 2));   // 128: would spill
+    else if (kgrid <= kF32SplitGrid2) GKI_DKDV32(2);
+    else GKI_DKDV32(4);
+#undef GKI_DQ32
+#undef GKI_DKDV32
     if (w.n_split > 0)
       hipLaunchKernelGGL((dkdv_reduce_kernel<F32, D>), red_grid, dim3(256), 0, stream, g, w,
                          (float*)dk, (float*)dv);
-    hipLaunchKernelGGL(dq_kernel_32<D>, dim3(n_qt * BH), dim3(256), 0, stream, g, (const float*)q,
-                       (const float*)k, (const float*)v, (const float*)dout, (float*)dq, lse, delta,
-                       row_ptr, row_idx, n_qt, dq_order);
   } else if (dtype == kF16) {
     launch_bwd16<F16, D>(g, q, k, v, o, dout, lse, dq, dk, dv, delta, row_ptr, row_idx, n_qt,
                          dq_order, col_ptr, col_idx, w, stream);

@@ -91,19 +91,22 @@ __device__ inline floatx4 mfma_f32(float a, float b, floatx4 c) {
 // accumulator; D = 128: 32 steps, 4 per accumulator) rounds like a short one.
 // With 4 accumulators at D = 64 the scores' and dP's rounding was the largest
 // error of the fp32 gradients at large logits (2x the eager path's on some
-// inputs); 8 halve it. a(ks) / b(ks) give step ks's operands.
-template <int KS, typename FA, typename FB>
-__device__ inline floatx4 mfma_f32_dot(FA a, FB b) {
-  constexpr int NC = KS >= 16 ? 8 : (KS >= 8 ? 4 : (KS >= 4 ? 2 : 1));
+// inputs); 8 halve it. a(j) / b[j] hold the operands of steps 4 j .. 4 j + 3.
+template <int KS, typename FA>
+__device__ inline floatx4 mfma_f32_dot(FA a, const floatx4 (&b)[KS / 4]) {
+  constexpr int NC = KS >= 16 ? 8 : (KS >= 8 ? 4 : 2);
   floatx4 c[NC];
 #pragma unroll
   for (int j = 0; j < NC; ++j) c[j] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) c[ks % NC] = mfma_f32(a(ks), b(ks), c[ks % NC]);
+  for (int j = 0; j < KS / 4; ++j) {
+    const floatx4 x = a(j);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c[(4 * j + i) % NC] = mfma_f32(x[i], b[j][i], c[(4 * j + i) % NC]);
+  }
   if constexpr (NC == 8) return ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
   else if constexpr (NC == 4) return (c[0] + c[1]) + (c[2] + c[3]);
-  else if constexpr (NC == 2) return c[0] + c[1];
-  else return c[0];
+  else return c[0] + c[1];
 }
 
 // 16-byte streaming (non-temporal) global load.
@@ -419,6 +422,73 @@ struct DmaTile {
 };
 
 // ---------------------------------------------------------------------------
+// fp32 tiles: row-major in LDS, 16-byte chunks XOR-swizzled per row, staged by
+// LDS-DMA. Two kinds of 16-byte reads feed v_mfma_f32_16x16x4f32, each four
+// MFMAs (a 4-byte read per MFMA kept the LDS as busy as the matrix cores):
+//  * a lane's four consecutive elements d = 16 j + 4 grp + i of a row: step i of
+//    a contraction over d takes {16 j + 4 grp + i, grp = 0 .. 3} (the register
+//    operand lists its elements in the same order);
+//  * four consecutive columns 4 col + e of row 4 grp + i: step i of a contraction
+//    over rows, result column (or row) col of output tile e standing for
+//    element 4 col + e.
+// The swizzle of 256-byte rows is free of conflicts for both, whether 16
+// consecutive lanes or {0-3, 12-15, 20-23, 24-27} are served per clock.
+// ---------------------------------------------------------------------------
+template <int D>
+__device__ inline int swz_f32(int row) {
+  if constexpr (D >= 64) return 4 * (row & 3) + ((-(row >> 2)) & 3);
+  else if constexpr (D == 32) return (row >> 1) & 7;
+  else return (row >> 2) & 3;
+}
+template <int D>
+__device__ inline int off_f32(int row, int chunk) { return row * D + ((chunk ^ swz_f32<D>(row)) << 2); }
+
+// Columns 64 v + DE col + e, e = 0 .. DE - 1, of a row.
+template <int D, int DE>
+__device__ inline floatx4 cols_f32(const float* tile, int row, int v, int col) {
+  if constexpr (DE == 4) {
+    return *(const floatx4*)(tile + off_f32<D>(row, 16 * v + col));
+  } else {
+    floatx4 x = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < DE; ++e) {
+      const int c = DE * col + e;
+      x[e] = tile[off_f32<D>(row, c >> 2) + (c & 3)];
+    }
+    return x;
+  }
+}
+
+// Stage TR rows of a row-major [n, D] fp32 matrix; rows past the last are zeros.
+template <int D, int TR, int NW = 4>
+struct DmaTileF32 {
+  static constexpr int NB = TR * D / 256;              // 1 KB blocks per tile
+  static constexpr int NP = (NB + NW - 1) / NW;        // blocks per wave
+  int off[NP];
+  int wave;
+  __device__ inline void init(int tid) {
+    wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const int e = (NW * p + wave) * 256 + 4 * lane;  // LDS float offset
+      const int row = e / D, ch = (e % D) >> 2;
+      off[p] = 4 * (row * D + ((ch ^ swz_f32<D>(row)) << 2));
+    }
+  }
+  __device__ inline void load(const float* base, int r0, int n_rows, const float* lds) const {
+    const int left = n_rows - r0;
+    const i32x4 rsrc = buffer_rsrc(base + (size_t)r0 * D, (left < 0 ? 0 : left < TR ? left : TR) * D * 4);
+    const uint32_t l0 = lds_addr(lds);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const int blk = NW * p + wave;
+      if (NB % NW == 0 || blk < NB) dma_buf16(rsrc, off[p], l0 + blk * 1024);
+    }
+  }
+};
+
+// ---------------------------------------------------------------------------
 // Kernel tiling. The forward uses 128x64 (q x kv) tiles, four waves per
 // workgroup, each wave owning 32 query rows; the backward kernels use 64x64
 // tiles, each wave owning 16 rows of the tile's outer axis. The decode kernel
@@ -429,6 +499,11 @@ constexpr int kTileN = 64;       // kv rows of every tile
 constexpr int kTileMF = 128;     // q rows of the forward tile (4 waves x 32 rows)
 constexpr int kDecodeTileM = 16;
 constexpr int kDecodeMaxQ = 4;
+// fp32 grids of at most this many 64-row tiles (one or two per CU) run them as
+// four / two workgroups of 16 / 32 rows whose waves share out the keys: B1 H4
+// N1024 D64 (64 tiles) forward 29 -> 11.6 us, dQ 43 -> 16.5 us. On full grids
+// (2048 tiles) two shares are level with none.
+constexpr int kF32SplitGrid4 = 256, kF32SplitGrid2 = 512;
 // dK/dV work items: at least kDkdvMinChunk iterations each, and about
 // kDkdvTargetItems items over the whole grid when the column walks are long.
 constexpr int kDkdvMinChunk = 32;
@@ -618,6 +693,15 @@ struct LaneBits32 {
   }
 };
 
+// The same for 16x16 subtiles in natural order (fp32): element i of subtile t in
+// lane group grp is bit 16 t + 4 grp + i. 0 or -1: element visible.
+struct LaneBits16 {
+  uint32_t w;
+  __device__ inline LaneBits16(uint64_t bits, int grp) : w((uint32_t)(bits >> (4 * grp))) {}
+  __device__ inline int mask(int t, int i) const { return __builtin_amdgcn_sbfe((int)w, 16 * t + i, 1); }
+  __device__ inline float keep(int t, int i, float x) const { return __int_as_float(__float_as_int(x) & mask(t, i)); }
+};
+
 // Is some (q, k) with q in [q_lo, q_hi], k in [k_lo, k_hi] (inclusive, absolute
 // positions, non-empty) visible under the token rule (k <= q) & (k < S | k >= q-W+1)?
 __device__ inline bool any_visible(long q_lo, long q_hi, long k_lo, long k_hi, long sink, long window) {
@@ -682,6 +766,15 @@ __device__ inline int work_of(int b, int n, const int32_t* order) {
   if (order == nullptr) return l;
   const int w = __builtin_amdgcn_readfirstlane(order[l]);
   return (unsigned)w < (unsigned)n ? w : -1;
+}
+
+// The same for units cut into `parts` workgroups each (grid work_parts_grid):
+// the parts of a unit run on one XCD, one after the other.
+inline int work_parts_grid(int n, int parts) { return parts == 1 ? n : kXcd * parts * ((n + kXcd - 1) / kXcd); }
+__device__ inline int work_part_of(int b, int n, int parts, const int32_t* order, int& part) {
+  const int x = b % kXcd, k = b / kXcd, slot = x + kXcd * (k / parts);
+  part = k % parts;
+  return slot < n ? work_of(slot, n, order) : -1;
 }
 
 // Reductions across the 4 lane groups (lanes l, l^16, l^32, l^48) with the

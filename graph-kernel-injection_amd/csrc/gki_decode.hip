@@ -20,8 +20,8 @@
 //     LSE itself; otherwise it writes (acc[D], m, l) to a workspace and
 //   * combine_kernel (one wave per row) merges the splits:
 //     O = sum acc_s 2^(m_s-M) / sum l_s 2^(m_s-M), LSE = (M + log2 L) ln 2
-//     (the partials' max is in base 2; the LSE is natural, as the forward
-//     stores it), with the (O = 0, LSE = 0) sentinel for empty rows.
+//     (the partials' max is in base 2, natural for fp32; the LSE is natural, as
+//     the forward stores it), with the (O = 0, LSE = 0) sentinel for empty rows.
 // Cross-workgroup merging goes through a second launch on purpose: publishing
 // partials across XCDs inside one kernel needs agent-scope fences, which on
 // gfx950 write back and invalidate L2.
@@ -139,6 +139,21 @@ struct RingTokens {
   }
 };
 
+// Units of the running max and of the exponents: base 2 for 16-bit inputs
+// (scores times scale log2 e); natural for fp32, as the prefill kernels keep
+// them: the exponent is the exact fma(S, scale, -m), so that the LSE is exact to
+// its own rounding (in base 2 the max of large scores alone was rounded by more
+// than that, and the backward forms P = exp(S scale - LSE) from it).
+template <typename T>
+__device__ inline float decode_exp(float x) {
+  return __builtin_amdgcn_exp2f(T::is_f32 ? x * kLog2e : x);
+}
+template <typename T>
+__device__ inline float decode_lse(float m, float l) {
+  if constexpr (T::is_f32) return (float)((double)m + log((double)l));
+  else return lse_natural(m, l);
+}
+
 // One round of a wave: NU passes of TPW token rows, LPT lanes per row, one
 // 16-byte K and V chunk per lane and pass.
 template <typename T, int D, int NU>
@@ -216,6 +231,7 @@ __device__ inline void decode_consume(const Geom& g, const DecodeRound<T, D, NU>
   using R = DecodeRound<T, D, NU>;
   constexpr int VEC = R::VEC, LPT = R::LPT;
   float sc[NQ][NU];
+  bool seen[NQ][NU];
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
     bool ok_u = rd.pj[u] >= 0;                // sign bit: padding row of the round
@@ -231,14 +247,21 @@ __device__ inline void decode_consume(const Geom& g, const DecodeRound<T, D, NU>
       if constexpr (!EXACT) {
         if (ok) ok = elem_valid(g, qrow[r], rd.pj[u] & kIdxMask, (rd.pj[u] >> kPartialBit) & 1);
       }
-      sc[r][u] = ok ? part * g.scale_log2 : kNegInf;
+      // fp32: the unscaled score (NaN-free mark of a masked one in `seen`)
+      if constexpr (T::is_f32) {
+        sc[r][u] = part;
+        seen[r][u] = ok;
+      } else {
+        sc[r][u] = ok ? part * g.scale_log2 : kNegInf;
+      }
     }
   }
 #pragma unroll
   for (int r = 0; r < NQ; ++r) {
     float mx = kNegInf;
 #pragma unroll
-    for (int u = 0; u < NU; ++u) mx = fmaxf(mx, sc[r][u]);
+    for (int u = 0; u < NU; ++u)
+      mx = fmaxf(mx, !T::is_f32 ? sc[r][u] : seen[r][u] ? sc[r][u] * g.scale : kNegInf);
     // Lazy reference max (wave-uniform): it moves, to the exact running max,
     // only when some score of the round exceeds it by the slack, so p stays
     // below 2^slack and the rescale (a cross-lane max, one exp2, VEC + 1
@@ -247,7 +270,7 @@ __device__ inline void decode_consume(const Geom& g, const DecodeRound<T, D, NU>
     if (__any(mx > m[r] + kDecodeSlack)) {
       mx = cross_group_max<LPT>(mx);           // scores are uniform within a token row
       const float m_new = fmaxf(m[r], mx);
-      const float alpha = __builtin_amdgcn_exp2f(m[r] - m_new);   // m = -inf: 0
+      const float alpha = decode_exp<T>(m[r] - m_new);   // m = -inf: 0
       m[r] = m_new;
       l[r] *= alpha;
 #pragma unroll
@@ -257,7 +280,9 @@ __device__ inline void decode_consume(const Geom& g, const DecodeRound<T, D, NU>
     float rs = 0.f;
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
-      const float p = __builtin_amdgcn_exp2f(sc[r][u] - mu);
+      const float p = !T::is_f32       ? __builtin_amdgcn_exp2f(sc[r][u] - mu)
+                      : seen[r][u] ? decode_exp<T>(__builtin_fmaf(sc[r][u], g.scale, -mu))
+                                   : 0.f;
       rs += p;
       const float pv = T::is_f32 ? p : T::to_float(T::from_float(p));   // P -> V dtype
       // a padding row re-reads a real V row: zero it so 0 * inf cannot appear
@@ -389,14 +414,14 @@ __global__ __launch_bounds__(64 * decode_waves<NQ>()) void decode_kernel(
     float L = 0.f, a = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      const float sw = __builtin_amdgcn_exp2f(wm[w][r] - Mu);
+      const float sw = decode_exp<T>(wm[w][r] - Mu);
       L += wl[w][r] * sw;
       a += wacc[w][r][d] * sw;
     }
     if (n_splits == 1) {
       const bool valid = L > 0.f;
       O[qb + (size_t)r * D + d] = T::from_float(valid ? a / L : 0.f);
-      if (d == 0) LSE[(size_t)bhq0 * g.n_q + r] = valid ? lse_natural(M, L) : 0.f;
+      if (d == 0) LSE[(size_t)bhq0 * g.n_q + r] = valid ? decode_lse<T>(M, L) : 0.f;
     } else {
       part[r * row_stride + d] = a;
       if (d == 0) {
@@ -431,7 +456,7 @@ __global__ __launch_bounds__(64) void combine_kernel(const float* __restrict__ w
 #pragma unroll 4
   for (int s = 0; s < n_splits; ++s) {
     const float* ps = base + s * sstride;
-    const float w = __builtin_amdgcn_exp2f(ps[D] - Mu);
+    const float w = decode_exp<T>(ps[D] - Mu);
     L += ps[D + 1] * w;
 #pragma unroll
     for (int j = 0; j < D / 64; ++j) a[j] += ps[lane + 64 * j] * w;
@@ -440,7 +465,7 @@ __global__ __launch_bounds__(64) void combine_kernel(const float* __restrict__ w
 #pragma unroll
   for (int j = 0; j < D / 64; ++j)
     O[(size_t)row * D + lane + 64 * j] = T::from_float(valid ? a[j] / L : 0.f);
-  if (lane == 0) LSE[row] = valid ? lse_natural(M, L) : 0.f;
+  if (lane == 0) LSE[row] = valid ? decode_lse<T>(M, L) : 0.f;
 }
 
 template <typename T, int D, int NQ, typename Src>

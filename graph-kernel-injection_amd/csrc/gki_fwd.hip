@@ -347,7 +347,11 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 4 : 2) void fwd_kernel_16(
 }
 
 // ---------------------------------------------------------------------------
-// fp32 path (v_mfma_f32_16x16x4f32, 64-row tiles): K and V stay row-major in LDS.
+// fp32 path (v_mfma_f32_16x16x4f32, 64-row tiles): K and V row-major in LDS
+// (swz_f32), staged by LDS-DMA, double-buffered, one barrier per 32 or 64 keys.
+// Bound by the fp32 matrix cores (154 TFLOP/s reached by a large product): B1
+// H16 N8192 D64 W1024 428 -> 334 us, N4096 D128 550 -> 319 us against 4-byte LDS
+// reads and tiles staged through registers behind two barriers.
 // The softmax runs in natural units: the running max m is that of the scaled
 // scores S * scale and each exponent is exp2(fma(S, scale, -m) * log2 e), so
 // the scale is applied exactly and only the (small) difference is rounded;
@@ -355,148 +359,209 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 4 : 2) void fwd_kernel_16(
 // LSE = m + ln(l), which therefore matches these scores to within its own
 // rounding.
 // ---------------------------------------------------------------------------
-template <int D>
-struct FwdSmem32 {
-  static constexpr int LD = D + 4;
-  float k[kTileN * LD];
-  float v[kTileN * LD];
-};
-
-// One wave per SIMD at head_dim 128: VGPRs + AGPRs hold it without scratch
-// (two waves spilled 284 bytes per lane: B1 H16 N8192 fp32 forward 1.39
-// against 1.12 ms, B1 H4 N1024 0.072 against 0.055 ms).
-template <int D>
-__global__ __launch_bounds__(256, D >= 128 ? 1 : 2) void fwd_kernel_32(
+//
+// A workgroup's four waves are QB blocks of 16 query rows x 4 / QB shares of
+// the keys of each staged step (16 keys each; two such subtiles when QB = 4), so
+// a 64-row q tile of the schedule is 4 / QB workgroups. With several shares the
+// waves keep a softmax state each and merge through LDS at the end: a grid too
+// short for the card (B1 H4 N1024: 64 tiles, 29 us) then runs on four times the
+// workgroups, each a quarter of the serial chain (11.6 us).
+template <int D, int QB>
+__global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : D * (QB == 1 ? 4 : 2) >= 256 ? 2 : 3) void fwd_kernel_32(
     Geom g, const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
     float* __restrict__ O, float* __restrict__ LSE, const int32_t* __restrict__ row_ptr,
     const int32_t* __restrict__ row_idx, int n_qt, const int32_t* __restrict__ wg_order) {
-  constexpr int KS = D / 4;
-  constexpr int DT = D / 16;
-  constexpr int CPR = D / 4;           // 16-byte chunks per row
-  constexpr int CH = kTileN * CPR;
-  constexpr int P = (CH + 255) / 256;
-  using Smem = FwdSmem32<D>;
-  __shared__ __align__(16) Smem sm;
+  constexpr int DJ = D / 16;                 // 16-byte chunks of a row per lane; output tiles
+  constexpr int KB = 4 / QB;                 // key shares
+  constexpr int TR = KB == 4 ? 64 : 32;      // keys per staged step
+  constexpr int SUBS = TR / (16 * KB);       // 16-key subtiles per wave and step
+  constexpr int HALVES = kTileN / TR;
+  constexpr int DV = D >= 64 ? D / 64 : 1;   // 16-byte reads of a V row per lane (64 columns each)
+  constexpr int DE = D / (16 * DV);          // output tiles per such read
+  __shared__ __align__(16) float sk[2][TR * D];
+  __shared__ __align__(16) float sv[2][TR * D];
 
-  const int n_wg = n_qt * g.B * g.H;
-  const int wg = work_of(blockIdx.x, n_wg, wg_order);
+  int part;
+  const int wg = work_part_of(blockIdx.x, n_qt * g.B * g.H, KB, wg_order, part);
   if (wg < 0) return;
   const int bh = wg / n_qt, qt = wg - bh * n_qt;
   const size_t qb = (size_t)bh * g.n_q * D;
   const size_t kb = (size_t)kv_bh(g, bh) * g.n_kv * D;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = lane >> 4, col = lane & 15;
-  const int q0 = qt * kTileM + wave * 16;
+  const int share = wave / QB;
+  const int q0 = qt * kTileM + 16 * (part * QB + wave % QB);
   const int my_q = q0 + col;
 
-  float qf[KS];
+  floatx4 qf[DJ];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks)
-    qf[ks] = (my_q < g.n_q) ? Q[qb + (size_t)my_q * D + 4 * ks + grp] : 0.f;
+  for (int j = 0; j < DJ; ++j)
+    qf[j] = my_q < g.n_q ? *(const floatx4*)(Q + qb + (size_t)my_q * D + 16 * j + 4 * grp)
+                         : floatx4{0.f, 0.f, 0.f, 0.f};
 
-  floatx4 o[DT];
+  // o[v][e]: row x of the tile is element 64 v + DE x + e
+  floatx4 o[DV][DE];
 #pragma unroll
-  for (int i = 0; i < DT; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int v = 0; v < DV; ++v)
+#pragma unroll
+    for (int e = 0; e < DE; ++e) o[v][e] = floatx4{0.f, 0.f, 0.f, 0.f};
   float m = kNegInf, l = 0.f;
 
-  const int e_beg = row_ptr[qt], e_end = row_ptr[qt + 1];
-  float4 kreg[P], vreg[P];
-  auto load_tile = [&](int k0) {
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      const int c = tid + 256 * p;
-      const int r = c / CPR, ch = c - r * CPR;
-      const bool ok = c < CH && k0 + r < g.n_kv;
-      kreg[p] = ok ? *(const float4*)(K + kb + (size_t)(k0 + r) * D + ch * 4) : make_float4(0, 0, 0, 0);
-      vreg[p] = ok ? *(const float4*)(V + kb + (size_t)(k0 + r) * D + ch * 4) : make_float4(0, 0, 0, 0);
-    }
+  const int e_beg = row_ptr[qt], n_step = (row_ptr[qt + 1] - e_beg) * HALVES;
+  DmaTileF32<D, TR> dma;
+  dma.init(tid);
+  auto step_k0 = [&](int s) {
+    return (row_idx[e_beg + s / HALVES] & kIdxMask) * kTileN + (s % HALVES) * TR;
   };
-  auto store_tile = [&]() {
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      const int c = tid + 256 * p;
-      if (c < CH) {
-        const int r = c / CPR, ch = c - r * CPR;
-        *(float4*)(&sm.k[r * Smem::LD + ch * 4]) = kreg[p];
-        *(float4*)(&sm.v[r * Smem::LD + ch * 4]) = vreg[p];
-      }
-    }
+  auto stage = [&](int s, int buf) {
+    const int k0 = step_k0(s);
+    dma.load(K + kb, k0, g.n_kv, sk[buf]);
+    dma.load(V + kb, k0, g.n_kv, sv[buf]);
   };
-
-  if (e_beg < e_end) load_tile((row_idx[e_beg] & kIdxMask) * kTileN);
-  const int q_hi_wave = min(q0 + 15, g.n_q - 1);
-  for (int e = e_beg; e < e_end; ++e) {
-    const int ent = row_idx[e];
-    const int k0 = (ent & kIdxMask) * kTileN;
-    const bool partial = (ent >> kPartialBit) & 1;
-    __syncthreads();
-    store_tile();
-    __syncthreads();
-    if (e + 1 < e_end) load_tile((row_idx[e + 1] & kIdxMask) * kTileN);
-
-    floatx4 s[4];
+  dma_wait();          // the Q loads, before any LDS-DMA is in flight
+  if (n_step > 0) stage(0, 0);
+  dma_wait();
+  __syncthreads();
+  const int q_hi = min(q0 + 15, g.n_q - 1);
+  for (int s = 0; s < n_step; ++s) {
+    const int buf = s & 1;
+    const bool partial = (row_idx[e_beg + s / HALVES] >> kPartialBit) & 1;
+    if (s + 1 < n_step) stage(s + 1, buf ^ 1);
+    const float *ck = sk[buf], *cv = sv[buf];
+    const int k0 = step_k0(s) + 16 * SUBS * share;       // the wave's first key
+    const bool need_mask = partial || (q0 + 15 >= g.n_q) || (k0 + 16 * SUBS > g.n_kv) ||
+                           !tile_all_visible(g, q0, q_hi, k0, k0 + 16 * SUBS - 1);
+    floatx4 p[SUBS];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int r = rho(t, col);
-      s[t] = mfma_f32_dot<KS>([&](int ks) { return sm.k[r * Smem::LD + 4 * ks + grp]; },
-                              [&](int ks) { return qf[ks]; });
+    for (int t = 0; t < SUBS; ++t) {
+      const int r = 16 * (SUBS * share + t) + col;
+      p[t] = mfma_f32_dot<4 * DJ>([&](int j) { return *(const floatx4*)(ck + off_f32<D>(r, 4 * j + grp)); }, qf);
     }
-    const bool need_mask = partial || (q0 + 15 >= g.n_q) || (k0 + kTileN > g.n_kv) ||
-                           !tile_all_visible(g, q0, q_hi_wave, k0, k0 + kTileN - 1);
-    float mx = kNegInf;
-    uint32_t vis = 0xFFFFu;            // bit 4 t + i: element visible
+    // the largest scaled score: rounding is monotone, so the largest (smallest,
+    // for a negative scale) score, scaled
+    float mx;
+    uint64_t bits = ~0ull;
+    if (need_mask) {
+      bits = row_valid_bits(g, my_q, k0, partial);
+      const LaneBits16 vis(bits, grp);
+      mx = kNegInf;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+      for (int t = 0; t < SUBS; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const bool ok = !need_mask || elem_valid(g, my_q, k0 + rho(t, 4 * grp + i), partial);
-        if (!ok) vis &= ~(1u << (4 * t + i));
-        mx = fmaxf(mx, ok ? s[t][i] * g.scale : kNegInf);
-      }
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, vis.mask(t, i) ? p[t][i] * g.scale : kNegInf);
+    } else if (g.scale >= 0.f) {
+      mx = p[0][0];
+#pragma unroll
+      for (int t = 0; t < SUBS; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, p[t][i]);
+      mx *= g.scale;
+    } else {
+      mx = p[0][0];
+#pragma unroll
+      for (int t = 0; t < SUBS; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fminf(mx, p[t][i]);
+      mx *= g.scale;
     }
-    mx = wave_max16x4(mx);
-    const float m_new = fmaxf(m, mx);
-    const float m_use = (m_new == kNegInf) ? 0.f : m_new;
-    const float alpha = __builtin_amdgcn_exp2f((m - m_use) * kLog2e);
+    if (__any(mx > m)) {               // some row's max moves
+      const float m_new = fmaxf(m, wave_max16x4(mx));
+      const float alpha = m_new == kNegInf ? 1.f : __builtin_amdgcn_exp2f((m - m_new) * kLog2e);
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int v = 0; v < DV; ++v)
+#pragma unroll
+        for (int e = 0; e < DE; ++e) o[v][e] *= alpha;
+    }
+    const float m_use = m == kNegInf ? 0.f : m;
+#pragma unroll
+    for (int t = 0; t < SUBS; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        p[t][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[t][i], g.scale, -m_use) * kLog2e);
+    if (need_mask) {
+      const LaneBits16 vis(bits, grp);
+#pragma unroll
+      for (int t = 0; t < SUBS; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[t][i] = vis.keep(t, i, p[t][i]);
+    }
     float rs = 0.f;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < SUBS; ++t) rs += (p[t][0] + p[t][1]) + (p[t][2] + p[t][3]);
+    l += rs;
+#pragma unroll
+    for (int t = 0; t < SUBS; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][i], g.scale, -m_use) * kLog2e);
-        const float p = (vis >> (4 * t + i)) & 1u ? e : 0.f;
-        s[t][i] = p;
-        rs += p;
+        const int r = 16 * (SUBS * share + t) + 4 * grp + i;
+#pragma unroll
+        for (int v = 0; v < DV; ++v) {
+          const auto x = cols_f32<D, DE>(cv, r, v, col);
+#pragma unroll
+          for (int e = 0; e < DE; ++e) o[v][e] = mfma_f32(x[e], p[t][i], o[v][e]);
+        }
       }
-    }
-    l = l * alpha + rs;
-    m = m_new;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = rho(t, 4 * grp + i);
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) o[dt] = mfma_f32(sm.v[r * Smem::LD + 16 * dt + col], s[t][i], o[dt]);
-      }
-    }
+    dma_wait();        // the next step's LDS-DMA has landed before the barrier
+    __syncthreads();
   }
 
-  const float l_tot = wave_sum16x4(l);
-  const bool valid = l_tot > 0.f;
-  if (my_q < g.n_q) {
+  l = wave_sum16x4(l);
+  if constexpr (KB > 1) {
+    // shares 1 .. KB - 1 hand (o, m, l) over through LDS (free: every wave
+    // passed the last barrier); share 0 merges them in order
+    float* red = sk[0];
+    const int blk = wave % QB;
+    if (share > 0) {
+      float* dst = red + ((size_t)(share - 1) * QB + blk) * (D + 2) * 16 + lane;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      float4 w;
-      w.x = valid ? o[dt][0] / l_tot : o[dt][0];
-      w.y = valid ? o[dt][1] / l_tot : o[dt][1];
-      w.z = valid ? o[dt][2] / l_tot : o[dt][2];
-      w.w = valid ? o[dt][3] / l_tot : o[dt][3];
-      *(float4*)(O + qb + (size_t)my_q * D + 16 * dt + 4 * grp) = w;
+      for (int v = 0; v < DV; ++v)
+#pragma unroll
+        for (int e = 0; e < DE; ++e)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) dst[64 * ((v * DE + e) * 4 + i)] = o[v][e][i];
+      if (grp == 0) {
+        dst[16 * D] = m;
+        dst[16 * D + 16] = l;
+      }
     }
-    if (grp == 0) LSE[(size_t)bh * g.n_q + my_q] = valid ? (float)((double)m + log((double)l_tot)) : 0.f;
+    __syncthreads();
+    if (share > 0) return;
+#pragma unroll
+    for (int w = 1; w < KB; ++w) {
+      const float* src = red + ((size_t)(w - 1) * QB + blk) * (D + 2) * 16;
+      const float mw = src[16 * D + col], lw = src[16 * D + 16 + col];
+      const float m_new = fmaxf(m, mw), m_use = m_new == kNegInf ? 0.f : m_new;
+      const float fa = __builtin_amdgcn_exp2f((m - m_use) * kLog2e);
+      const float fb = __builtin_amdgcn_exp2f((mw - m_use) * kLog2e);
+      l = l * fa + lw * fb;
+      m = m_new;
+#pragma unroll
+      for (int v = 0; v < DV; ++v)
+#pragma unroll
+        for (int e = 0; e < DE; ++e)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            o[v][e][i] = o[v][e][i] * fa + src[64 * ((v * DE + e) * 4 + i) + lane] * fb;
+    }
+  }
+  const bool valid = l > 0.f;
+  if (my_q < g.n_q) {
+    const float den = valid ? l : 1.f;
+#pragma unroll
+    for (int v = 0; v < DV; ++v)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float* dst = O + qb + (size_t)my_q * D + 64 * v + DE * (4 * grp + i);
+        if constexpr (DE == 4) {
+          *(floatx4*)dst = floatx4{o[v][0][i] / den, o[v][1][i] / den, o[v][2][i] / den, o[v][3][i] / den};
+        } else {
+#pragma unroll
+          for (int e = 0; e < DE; ++e) dst[e] = o[v][e][i] / den;
+        }
+      }
+    if (grp == 0) LSE[(size_t)bh * g.n_q + my_q] = valid ? (float)((double)m + log((double)l)) : 0.f;
   }
 }
 
@@ -512,9 +577,14 @@ int launch_fwd(int dtype, const Geom& g, const void* q, const void* k, const voi
                const int32_t* wg_order, hipStream_t stream) {
   const int grid = n_qt * g.B * g.H;
   if (dtype == kF32) {
-    hipLaunchKernelGGL(fwd_kernel_32<D>, dim3(grid), dim3(256), 0, stream, g, (const float*)q,
-                       (const float*)k, (const float*)v, (float*)o, lse, row_ptr, row_idx, n_qt,
-                       wg_order);
+#define GKI_FWD32(QB)                                                                               \
+  hipLaunchKernelGGL((fwd_kernel_32<D, QB>), dim3(work_parts_grid(grid, 4 / QB)), dim3(256), 0,     \
+                     stream, g, (const float*)q, (const float*)k, (const float*)v, (float*)o, lse,  \
+                     row_ptr, row_idx, n_qt, wg_order)
+    if (grid <= kF32SplitGrid4) GKI_FWD32(1);
+    else if (grid <= kF32SplitGrid2) GKI_FWD32(2);
+    else GKI_FWD32(4);
+#undef GKI_FWD32
   } else if (dtype == kF16) {
     hipLaunchKernelGGL((fwd_kernel_16<F16, D, kFwdPipe<D>>), dim3(grid), dim3(kFwdThreads), 0, stream, g,
                        (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o, lse,
