@@ -124,27 +124,39 @@ __global__ __launch_bounds__(256) void dkdv_reduce_kernel(Geom g, KvWork w,
 }
 
 // ---------------------------------------------------------------------------
-// dK / dV, 16-bit. Q and dO tiles row-major in LDS (double-buffered, staged by
-// LDS-DMA); the dV += P^T dO and dK += dS^T Q operands dO / Q come from lds_tr8.
+// dK / dV, 16-bit, in quadrants: wave w owns kv rows 32 (w & 1) .. +31 of the
+// 64-row kv tile (K / V in registers as B operands) against q rows
+// 32 (w >> 1) .. +31 of each q tile: one 32x32 block of S and of dP per wave and
+// tile, whose accumulators (v_mfma_f32_32x32x16) are the operands of
+// dV^T += dO^T P and dK^T += Q^T dS. Q and dO tiles row-major in LDS
+// (double-buffered, staged by LDS-DMA), transposed operands by Lane32::cols.
+// The two q halves' fp32 sums meet once, through LDS, at the end of the item
+// (the qh = 0 wave adds the qh = 1 wave's, a fixed order).
 // ---------------------------------------------------------------------------
-// PRE (Geom::prescale): the scale is already inside the dP accumulator
-// (V / dO operands and Delta pre-multiplied by a power-of-two scale, exact),
-// so dS = P * acc; otherwise dS = P * (acc * scale). Either way the scaled dS
-// is cast, as the reference. A template parameter, so neither form carries a
-// branch.
+// Head dims other than 64. At 128 the LDS was the bound (96 reads per 64 small
+// MFMAs with 16 kv rows per wave; 48 per 32 large ones now), then the latency of
+// operands read one at a time: B2 H32 on 8 kv heads N4096 D128 W1024 bf16, cycles
+// per workgroup and tile 5147 -> 4370 with this layout; backward 0.607 -> 0.569 ms
+// with it and 0.549 with the reads pinned ahead (B4 H8 N2000 D32 0.071 -> 0.055).
+// At head_dim 64 the card's power is the bound (1.9-2.1 GHz under the backward)
+// and this form, 7% fewer cycles at a 10% lower clock, ran 2-3% slower than the
+// 16x16x32 quadrants below.
+// PRE: Geom::prescale. A template parameter, so neither form carries a branch.
 template <typename T, int D, bool PRE>
-__global__ __launch_bounds__(256, 2) void dkdv_kernel_16(
+__global__ __launch_bounds__(256, D <= 32 ? 4 : D == 64 ? 3 : PRE ? 2 : 1) void dkdv_kernel_16(
     Geom g, const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ dO, uint16_t* __restrict__ dK,
     uint16_t* __restrict__ dV, const float* __restrict__ LSE2, const float* __restrict__ Delta,
     const int32_t* __restrict__ col_ptr, const int32_t* __restrict__ col_idx, KvWork w) {
-  // LSE2: base-2 LSE rows; Delta: -Delta rows (times the scale when PRE),
-  // both written by the dQ kernel, which runs first
-  constexpr int KS = (D + 31) / 32;
-  constexpr int DT = D / 16;
-  using Tile = RowTile<D>;
-  __shared__ __align__(16) uint16_t sq[2][64 * D];
-  __shared__ __align__(16) uint16_t sdo[2][64 * D];
+  // LSE2: -LSE / scale rows when PRE, else base-2 LSE rows; Delta: -Delta rows
+  // (times pre when PRE); both written by the dQ kernel, which runs first
+  constexpr int kAhead = 3;                    // operands read ahead (255 VGPRs at head_dim 128)
+  constexpr int KS = D / 16;                   // k-steps of the contractions over d
+  constexpr int DT = D >= 32 ? D / 32 : 1;     // 32-row tiles of dK^T / dV^T
+  constexpr int TILE = 64 * D;
+  // Q, Q, dO, dO; the waves' sums at the end
+  constexpr int LDS16 = 4 * TILE > 2 * 2 * DT * 16 * 64 * 2 ? 4 * TILE : 2 * 2 * DT * 16 * 64 * 2;
+  __shared__ __align__(16) uint16_t stile[LDS16];
   __shared__ __align__(16) float slse[2][64];
   __shared__ __align__(16) float sdlt[2][64];
 
@@ -158,48 +170,41 @@ __global__ __launch_bounds__(256, 2) void dkdv_kernel_16(
   const int kt = item.kt;
   const size_t kb = (size_t)bh * g.n_kv * D;
   const int bhq0 = (bh / g.H_kv) * g.H + (bh % g.H_kv) * g.group;   // first q head
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int grp = lane >> 4, col = lane & 15;
-  const int k_w = kt * kTileN + wave * 16;
-  const int my_kv = k_w + col;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, hi = lane >> 5, col = lane & 31;
+  const Lane32<D> at0(lane);
+  const int kh = wave & 1, qh = wave >> 1;
+  const int k_w = kt * kTileN + 32 * kh;       // the wave's first kv row
 
   uint4 kf[KS], vf[KS];
+  {
+    const int my_kv = k_w + col;
+    const bool ok = has_work && my_kv < g.n_kv;
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const int d0 = 32 * ks + 8 * grp;
-    const bool ok = has_work && my_kv < g.n_kv && d0 < D;
-    kf[ks] = ok ? *(const uint4*)(K + kb + (size_t)my_kv * D + d0) : make_uint4(0, 0, 0, 0);
-    vf[ks] = ok ? *(const uint4*)(V + kb + (size_t)my_kv * D + d0) : make_uint4(0, 0, 0, 0);
-    if constexpr (PRE) vf[ks] = scale8<T>(vf[ks], g.scale);
+    for (int ks = 0; ks < KS; ++ks) {
+      const size_t o = kb + (size_t)my_kv * D + 16 * ks + 8 * hi;
+      kf[ks] = ok ? *(const uint4*)(K + o) : make_uint4(0, 0, 0, 0);
+      vf[ks] = ok ? *(const uint4*)(V + o) : make_uint4(0, 0, 0, 0);
+      if constexpr (PRE) vf[ks] = scale8<T>(vf[ks], g.pre);
+    }
   }
-  floatx4 dk[DT], dv[DT];
+  floatx16 dk[DT], dv[DT];
 #pragma unroll
-  for (int i = 0; i < DT; ++i) dk[i] = dv[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < DT; ++i) dk[i] = dv[i] = splat16(0.f);
 
   const int e_beg = col_ptr[kt], e_end = col_ptr[kt + 1];
-  DmaTile<D> dma;
+  DmaTile<D, 4, true> dma;
   dma.init(tid);
-  // Q / dO tiles: full tiles by LDS-DMA, the ragged last one through registers
-  // (rows past n_q zero). LSE / Delta rows by a 4-byte LDS-DMA (waves 0 / 1,
-  // one lane per row; rows past n_q re-read row n_q - 1, which only masked
-  // elements see).
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  // Rows past n_q are zeros in Q and dO (the DMA's range check); LSE / Delta
+  // rows by a 4-byte LDS-DMA (waves 0 / 1, one lane per row; rows past n_q
+  // re-read row n_q - 1, which only masked elements see).
   auto load_tile = [&](int q0, int bhq, int buf) {
     const size_t qb = (size_t)bhq * g.n_q * D;
-    if (q0 + kTileM <= g.n_q) {
-      dma.load(Q + qb, q0, sq[buf]);
-      dma.load(dO + qb, q0, sdo[buf]);
-    } else {
-      Tile t;
-      t.load(Q + qb, q0, g.n_q, tid);
-      t.store(sq[buf], tid);
-      t.load(dO + qb, q0, g.n_q, tid);
-      t.store(sdo[buf], tid);
-      dma_wait();   // nothing of this branch pending where it rejoins the DMA path
-    }
-    if (wave_u < 2) {
-      const float* src = (wave_u == 0 ? LSE2 : Delta) + (size_t)bhq * g.n_q + min(q0 + lane, g.n_q - 1);
-      dma_load4(src, lds_addr(wave_u == 0 ? slse[buf] : sdlt[buf]));
+    dma.load(Q + qb, q0, g.n_q, stile + buf * TILE);
+    dma.load(dO + qb, q0, g.n_q, stile + (2 + buf) * TILE);
+    if (wave < 2) {
+      const float* src = (wave == 0 ? LSE2 : Delta) + (size_t)bhq * g.n_q + min(q0 + lane, g.n_q - 1);
+      dma_load4(src, lds_addr(wave == 0 ? slse[buf] : sdlt[buf]));
     }
   };
   // iterations [it0, it1): iteration i visits list entry e_beg + i % L of q
@@ -212,7 +217,7 @@ __global__ __launch_bounds__(256, 2) void dkdv_kernel_16(
   dma_wait();
   __syncthreads();
 
-  const int kv_hi_wave = min(k_w + 15, g.n_kv - 1);
+  const int kv_hi_wave = min(k_w + 31, g.n_kv - 1);
   for (int it = 0; it < n_it; ++it) {
     const int buf = it & 1;
     const int ent = col_idx[e_nx];
@@ -223,97 +228,135 @@ __global__ __launch_bounds__(256, 2) void dkdv_kernel_16(
     const int q0 = (ent & kIdxMask) * kTileM;
     const bool partial = (ent >> kPartialBit) & 1;
     if (it + 1 < n_it) load_tile((col_idx[e_nx] & kIdxMask) * kTileM, q_nx, buf ^ 1);
-    const uint16_t* cq = sq[buf];
-    const uint16_t* cdo = sdo[buf];
-
-    const bool need_mask = partial || (q0 + kTileM > g.n_q) || (k_w + 15 >= g.n_kv) ||
-                           !tile_all_visible(g, q0, min(q0 + kTileM - 1, g.n_q - 1), k_w, kv_hi_wave);
-    // S and dP for the four 16-row q subtiles (rows rho(t, .)); accumulator
-    // element i of lane (grp, col) is q row rho(t, 4 grp + i), kv row my_kv
-    floatx4 p[4], ds[4];
+    const uint16_t* cq = stile + buf * TILE;
+    const uint16_t* cdo = stile + (2 + buf) * TILE;
+    const int qw0 = q0 + 32 * qh;              // the wave's first q row
+    Lane32<D> at = at0;
+    if constexpr (D >= 128) at.pin();          // its offsets' XORs per tile, not held in 14 registers
+    // left out where none of the wave's rows sees one of its keys
+    if (!tile_unseen(g, qw0, qw0 + 31, k_w, 32)) {
+      const bool need_mask = partial || (qw0 + 32 > g.n_q) || (k_w + 31 >= g.n_kv) ||
+                             !tile_all_visible(g, qw0, qw0 + 31, k_w, kv_hi_wave);
+      // register r of lane (hi, col): q row qw0 + acc32_row(r, hi), kv row k_w + col.
+      // The accumulators start at the row terms of their q rows: dP at -Delta, so
+      // that it ends as dP - Delta (times pre when PRE), and with PRE S at
+      // -LSE / scale, so that P = exp2(S scale log2 e).
+      floatx16 s, dp;
+      const float* rd = &sdlt[buf][32 * qh + 4 * hi];
+      const float* rl = &slse[buf][32 * qh + 4 * hi];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      // the dP accumulator starts at -Delta of its four q rows (stored negated
-      // by the dQ kernel), so it ends as dP - Delta (times the scale when PRE)
-      const int qr0 = rho(t, 4 * grp);
-      const float4 lse4 = *(const float4*)(&slse[buf][qr0]);
-      const float4 ndl4 = *(const float4*)(&sdlt[buf][qr0]);
-      floatx4 s = floatx4{0.f, 0.f, 0.f, 0.f};
-      floatx4 dp = floatx4{ndl4.x, ndl4.y, ndl4.z, ndl4.w};
-      const int r = rho(t, col);
-      mfma_priority_hi<(D <= 64)>();
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int d0 = 32 * ks + 8 * grp;
-        const uint4 aq = (d0 < D) ? lds_row8<D>(cq, r, d0) : make_uint4(0, 0, 0, 0);
-        const uint4 ad = (d0 < D) ? lds_row8<D>(cdo, r, d0) : make_uint4(0, 0, 0, 0);
-        s = T::mfma(aq, kf[ks], s);
-        dp = T::mfma(ad, vf[ks], dp);
+      for (int q = 0; q < 4; ++q) {
+        const float4 l = *(const float4*)(rl + 8 * q), v = *(const float4*)(rd + 8 * q);
+        s[4 * q] = PRE ? l.x : 0.f, s[4 * q + 1] = PRE ? l.y : 0.f;
+        s[4 * q + 2] = PRE ? l.z : 0.f, s[4 * q + 3] = PRE ? l.w : 0.f;
+        dp[4 * q] = v.x, dp[4 * q + 1] = v.y, dp[4 * q + 2] = v.z, dp[4 * q + 3] = v.w;
       }
-      mfma_priority_lo<(D <= 64)>();
-      const float lv[4] = {lse4.x, lse4.y, lse4.z, lse4.w};          // base-2 LSE
+      // S and dP in turn, each operand read kAhead products ahead (the order is
+      // pinned: left alone the compiler has each product wait for its own read)
+      auto row_op = [&](int i) { return at.rows(i & 1 ? cdo : cq, qh, i >> 1); };
+      uint4 op[kAhead];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], g.scale_log2, -lv[i]));
-        p[t][i] = pv;
-        ds[t][i] = PRE ? pv * dp[i] : pv * (dp[i] * g.scale);
+      for (int i = 0; i < kAhead && i < 2 * KS; ++i) op[i] = row_op(i);
+#pragma unroll
+      for (int i = 0; i < 2 * KS; ++i) {
+        if (i & 1) dp = T::mfma32(op[i % kAhead], vf[i >> 1], dp);
+        else s = T::mfma32(op[i % kAhead], kf[i >> 1], s);
+        if (i + kAhead < 2 * KS) op[i % kAhead] = row_op(i + kAhead);
+        __builtin_amdgcn_sched_barrier(0);
       }
-    }
-    // Masked elements: P = dS = 0 (a bit select, so an exp that overflowed on
-    // an invisible element cannot leak). One uniform branch per tile keeps the
-    // selects off the tiles that need no mask.
-    if (need_mask) {
-      const LaneBits vis(col_valid_bits(g, my_kv, q0, partial), grp);
+      if constexpr (PRE) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          p[t][i] = vis.pick(t, i, p[t][i], 0.f);
-          ds[t][i] = vis.pick(t, i, ds[t][i], 0.f);
+        for (int r = 0; r < 16; ++r) {
+          s[r] = __builtin_amdgcn_exp2f(s[r] * g.scale_log2);
+          dp[r] *= s[r];
         }
-    }
-    mfma_priority_hi<(D <= 64)>();
+      } else {
 #pragma unroll
-    for (int st = 0; st < 2; ++st) {
-      const uint4 ap = pack8<T>(p[2 * st], p[2 * st + 1]);
-      const uint4 ad = pack8<T>(ds[2 * st], ds[2 * st + 1]);
+        for (int q = 0; q < 4; ++q) {
+          const float4 l = *(const float4*)(rl + 8 * q);             // base-2 LSE
+          const float lv[4] = {l.x, l.y, l.z, l.w};
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        dv[dt] = T::mfma(ap, lds_tr8<D>(cdo, 32 * st, 16 * dt, lane), dv[dt]);
-        dk[dt] = T::mfma(ad, lds_tr8<D>(cq, 32 * st, 16 * dt, lane), dk[dt]);
+          for (int i = 0; i < 4; ++i) {
+            const int r = 4 * q + i;
+            s[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], g.scale_log2, -lv[i]));
+            dp[r] = s[r] * (dp[r] * g.scale);
+          }
+        }
+      }
+      // Masked elements: P = dS = 0 (a bit select, so an exp that overflowed on
+      // an invisible element cannot leak). One uniform branch per tile keeps the
+      // selects off the tiles that need no mask.
+      if (need_mask) {
+        const uint64_t bits = col_valid_bits(opaque_blocks(g), k_w + (lane_now() & 31), q0, partial);
+        const LaneBits32 vis(qh ? (uint32_t)(bits >> 32) : (uint32_t)bits, lane_now() >> 5);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int m = vis.mask(r);
+          s[r] = __int_as_float(__float_as_int(s[r]) & m);
+          dp[r] = __int_as_float(__float_as_int(dp[r]) & m);
+        }
+      }
+      uint4 pk[2][2];                          // P and dS, 16 q rows each
+#pragma unroll
+      for (int st = 0; st < 2; ++st) pk[st][0] = pack8<T>(s, st), pk[st][1] = pack8<T>(dp, st);
+      auto col_op = [&](int i) { return at.cols(i & 1 ? cq : cdo, 2 * qh + i / (2 * DT), (i >> 1) % DT); };
+      uint4 ot[kAhead];
+#pragma unroll
+      for (int i = 0; i < kAhead && i < 4 * DT; ++i) ot[i] = col_op(i);
+#pragma unroll
+      for (int i = 0; i < 4 * DT; ++i) {
+        const int st = i / (2 * DT), dt = (i >> 1) % DT;
+        if (i & 1) dk[dt] = T::mfma32(ot[i % kAhead], pk[st][1], dk[dt]);
+        else dv[dt] = T::mfma32(ot[i % kAhead], pk[st][0], dv[dt]);
+        if (i + kAhead < 4 * DT) ot[i % kAhead] = col_op(i + kAhead);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    mfma_priority_lo<(D <= 64)>();
     dma_wait();        // the next tile's LDS-DMA has landed before the barrier
     __syncthreads();
   }
 
-  // dK/dV accumulators: lane holds rows k_w + 4grp + i, column 16dt + col.
-  if (item.pslot >= 0) {             // a split column: fp32 partials for the reduce
-    float* pk = w.partials + ((size_t)bh * w.n_pslots + item.pslot) * 2 * (kTileN * D);
-    float* pv = pk + kTileN * D;
+  // the q halves' sums meet in LDS (the Q / dO buffers are free: every wave
+  // passed the loop's last barrier): qh = 1 waves store, qh = 0 waves add theirs
+  floatx4* red = (floatx4*)stile + kh * (2 * DT * 4 * 64);
+  const int lane_e = lane_now(), hi_e = lane_e >> 5;
+  if (qh == 1) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = wave * 16 + 4 * grp + i;
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        pk[r * D + 16 * dt + col] = dk[dt][i];
-        pv[r * D + 16 * dt + col] = dv[dt][i];
+      for (int q = 0; q < 4; ++q) {
+        red[((2 * dt) * 4 + q) * 64 + lane_e] = floatx4{dk[dt][4 * q], dk[dt][4 * q + 1], dk[dt][4 * q + 2], dk[dt][4 * q + 3]};
+        red[((2 * dt + 1) * 4 + q) * 64 + lane_e] = floatx4{dv[dt][4 * q], dv[dt][4 * q + 1], dv[dt][4 * q + 2], dv[dt][4 * q + 3]};
+      }
+  }
+  __syncthreads();
+  if (qh == 1) return;
+  const float post = PRE ? g.post : 1.f;
+  const bool split = item.pslot >= 0;          // a split column: fp32 partials for the reduce
+  const int row = 32 * kh + (lane_e & 31);     // of the kv tile
+  if (!split && kt * kTileN + row >= g.n_kv) return;
+  float* part = w.partials + ((size_t)bh * w.n_pslots + (split ? item.pslot : 0)) * 2 * TILE + (size_t)row * D;
+  const size_t out = kb + (size_t)(kt * kTileN + row) * D;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int q = 0; q < (D >= 32 ? 4 : 2); ++q) {      // D = 16: elements past 15 do not exist
+      const floatx4 rk = red[((2 * dt) * 4 + q) * 64 + lane_e], rv = red[((2 * dt + 1) * 4 + q) * 64 + lane_e];
+      floatx4 a, b;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        a[i] = (dk[dt][4 * q + i] + rk[i]) * post;
+        b[i] = dv[dt][4 * q + i] + rv[i];
+      }
+      const int d0 = 32 * dt + 8 * q + 4 * hi_e;
+      if (split) {
+        *(floatx4*)(part + d0) = a;
+        *(floatx4*)(part + TILE + d0) = b;
+      } else {
+        *(uint2*)(dK + out + d0) = make_uint2(pack2<T>(a[0], a[1]), pack2<T>(a[2], a[3]));
+        *(uint2*)(dV + out + d0) = make_uint2(pack2<T>(b[0], b[1]), pack2<T>(b[2], b[3]));
       }
     }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = k_w + 4 * grp + i;
-    if (row < g.n_kv) {
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        dK[kb + (size_t)row * D + 16 * dt + col] = T::from_float(dk[dt][i]);
-        dV[kb + (size_t)row * D + 16 * dt + col] = T::from_float(dv[dt][i]);
-      }
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -324,7 +367,9 @@ __global__ __launch_bounds__(256, 2) void dkdv_kernel_16(
 // and transposed Q / dO read from LDS then feeds the MFMAs of both kv blocks:
 // 28 LDS reads per 32 MFMAs per wave and tile instead of 56. The two q
 // halves' fp32 dK / dV sums meet once, through LDS, at the end of the item
-// (the qh = 0 wave adds the qh = 1 wave's, a fixed order).
+// (the qh = 0 wave adds the qh = 1 wave's, a fixed order). Waves leave out the
+// 32 x 32 blocks they cannot see: B4 H16 N8192 W1024 fp16 backward 0.586 ->
+// 0.577 ms, B1 H16 N131072 W4096 7.02 -> 7.00.
 // ---------------------------------------------------------------------------
 template <typename T, bool PRE>
 __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
@@ -335,7 +380,6 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
   // LSE2: base-2 LSE rows; Delta: -Delta rows (times the scale when PRE),
   // both written by the dQ kernel, which runs first
   constexpr int D = 64, KS = 2, DT = 4;
-  using Tile = RowTile<D>;
   __shared__ __align__(16) uint16_t sq[2][64 * D];
   __shared__ __align__(16) uint16_t sdo[2][64 * D];
   __shared__ __align__(16) float slse[2][64];
@@ -364,7 +408,7 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
       const bool ok = has_work && my_kv < g.n_kv;
       kf[b][ks] = ok ? *(const uint4*)(K + kb + (size_t)my_kv * D + d0) : make_uint4(0, 0, 0, 0);
       vf[b][ks] = ok ? *(const uint4*)(V + kb + (size_t)my_kv * D + d0) : make_uint4(0, 0, 0, 0);
-      if constexpr (PRE) vf[b][ks] = scale8<T>(vf[b][ks], g.scale);
+      if constexpr (PRE) vf[b][ks] = scale8<T>(vf[b][ks], g.pre);
     }
   }
   floatx4 dk[2][DT], dv[2][DT];
@@ -379,17 +423,8 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   auto load_tile = [&](int q0, int bhq, int buf) {
     const size_t qb = (size_t)bhq * g.n_q * D;
-    if (q0 + kTileM <= g.n_q) {
-      dma.load(Q + qb, q0, sq[buf]);
-      dma.load(dO + qb, q0, sdo[buf]);
-    } else {
-      Tile t;
-      t.load(Q + qb, q0, g.n_q, tid);
-      t.store(sq[buf], tid);
-      t.load(dO + qb, q0, g.n_q, tid);
-      t.store(sdo[buf], tid);
-      dma_wait();   // nothing of this branch pending where it rejoins the DMA path
-    }
+    dma.load(Q + qb, q0, g.n_q, sq[buf]);      // rows past n_q: zeros
+    dma.load(dO + qb, q0, g.n_q, sdo[buf]);
     if (wave_u < 2) {
       const float* src = (wave_u == 0 ? LSE2 : Delta) + (size_t)bhq * g.n_q + min(q0 + lane, g.n_q - 1);
       dma_load4(src, lds_addr(wave_u == 0 ? slse[buf] : sdlt[buf]));
@@ -417,6 +452,8 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
     const uint16_t* cq = sq[buf];
     const uint16_t* cdo = sdo[buf];
     const int qw0 = q0 + 32 * qh;              // the wave's first q row
+    // left out where none of the wave's rows sees one of its keys
+    if (!tile_unseen(g, qw0, qw0 + 31, k_w, 32)) {
     const bool need_mask = partial || (qw0 + 32 > g.n_q) || (k_w + 31 >= g.n_kv) ||
                            !tile_all_visible(g, qw0, min(qw0 + 31, g.n_q - 1), k_w, kv_hi_wave);
     floatx4 p[2][2], ds[2][2];                 // [subtile 2 qh + u][kv block]
@@ -489,6 +526,7 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
       }
     }
     mfma_priority_lo<true>();
+    }
     dma_wait();        // the next tile's LDS-DMA has landed before the barrier
     __syncthreads();
   }
@@ -512,6 +550,7 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       dk[b][dt] += red[((2 * b + 0) * DT + dt) * 64 + lane];
+      if constexpr (PRE) dk[b][dt] *= g.post;
       dv[b][dt] += red[((2 * b + 1) * DT + dt) * 64 + lane];
     }
   // accumulators: lane holds kv rows k_w + 16 b + 4 grp + i, column 16 dt + col
@@ -775,22 +814,26 @@ __global__ __launch_bounds__(256, D >= 128 || (D == 64 && KB == 1) ? 1 : 2) void
 }
 
 // ---------------------------------------------------------------------------
-// dQ, 16-bit. K and V tiles row-major in LDS (double-buffered, staged by
-// LDS-DMA); the
-// dQ^T += K^T dS^T operand K^T comes from lds_tr8.
+// dQ, 16-bit, in quadrants: wave w owns q rows 32 (w >> 1) .. +31 of the 64-row
+// q tile (Q / dO in registers as B operands) against kv rows 32 (w & 1) .. +31 of
+// each kv tile; the 32x32 block of dS^T is the operand of dQ^T += K^T dS^T. K
+// and V tiles row-major in LDS (double-buffered, staged by LDS-DMA). The two kv
+// halves' fp32 sums meet once, through LDS, at the end (the kh = 0 wave adds
+// the kh = 1 wave's, a fixed order).
 // ---------------------------------------------------------------------------
 template <typename T, int D, bool PRE>
-__global__ __launch_bounds__(256, 2) void dq_kernel_16(
+__global__ __launch_bounds__(256, D > 64 ? 2 : D == 64 ? 3 : 4) void dq_kernel_16(
     Geom g, const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO,
     uint16_t* __restrict__ dQ, const float* __restrict__ LSE, float* __restrict__ Delta,
     const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ row_idx, int n_qt,
     const int32_t* __restrict__ dq_order) {
-  constexpr int KS = (D + 31) / 32;
-  constexpr int DT = D / 16;
-  using Tile = RowTile<D>;
-  __shared__ __align__(16) uint16_t sk[2][64 * D];
-  __shared__ __align__(16) uint16_t sv[2][64 * D];
+  constexpr int kAhead = 4;                    // operands read ahead
+  constexpr int KS = D / 16;
+  constexpr int DT = D >= 32 ? D / 32 : 1;
+  constexpr int TILE = 64 * D;
+  constexpr int LDS16 = 4 * TILE > 2 * DT * 16 * 64 * 2 ? 4 * TILE : 2 * DT * 16 * 64 * 2;
+  __shared__ __align__(16) uint16_t stile[LDS16];      // K, K, V, V; the waves' sums at the end
 
   const int n_wg = n_qt * g.B * g.H;
   const int wg = work_of(blockIdx.x, n_wg, dq_order);
@@ -798,137 +841,145 @@ __global__ __launch_bounds__(256, 2) void dq_kernel_16(
   const int bh = wg / n_qt, qt = wg - bh * n_qt;
   const size_t qb = (size_t)bh * g.n_q * D;
   const size_t kb = (size_t)kv_bh(g, bh) * g.n_kv * D;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int grp = lane >> 4, col = lane & 15;
-  const int q0 = qt * kTileM + wave * 16;
-  const int my_q = q0 + col;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, hi = lane >> 5, col = lane & 31;
+  const Lane32<D> at(lane);
+  const int qh = wave >> 1, kh = wave & 1;
+  const int q0w = qt * kTileM + 32 * qh;       // the wave's first q row
 
   uint4 qf[KS], df[KS];
+  float lse2, ndlt;
+  {
+    const int my_q = q0w + col;
+    const bool ok = my_q < g.n_q;
+    float part = 0.f;
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const int d0 = 32 * ks + 8 * grp;
-    const bool ok = my_q < g.n_q && d0 < D;
-    qf[ks] = ok ? *(const uint4*)(Q + qb + (size_t)my_q * D + d0) : make_uint4(0, 0, 0, 0);
-    df[ks] = ok ? *(const uint4*)(dO + qb + (size_t)my_q * D + d0) : make_uint4(0, 0, 0, 0);
-  }
-  // the stored natural LSE in base 2 (one rounding, once per row)
-  const float lse2 = my_q < g.n_q ? lse_base2(LSE[(size_t)bh * g.n_q + my_q]) : 0.f;
-  // Delta = rowsum(O * dO) in fp32 over the stored O (the preprocessing pass,
-  // sparse_triton_kernel.py:354-392, fused here): the lane already holds its
-  // row's dO chunks, the four lane groups of a row are summed across. Every q
-  // row has exactly one dQ workgroup, which writes it (and the base-2 LSE)
-  // for the dK/dV kernel that runs next.
-  float part = 0.f;
+    for (int ks = 0; ks < KS; ++ks) {
+      const size_t o = qb + (size_t)my_q * D + 16 * ks + 8 * hi;
+      qf[ks] = ok ? *(const uint4*)(Q + o) : make_uint4(0, 0, 0, 0);
+      df[ks] = ok ? *(const uint4*)(dO + o) : make_uint4(0, 0, 0, 0);
+      // Delta = rowsum(O * dO) in fp32 over the stored O (the preprocessing pass,
+      // sparse_triton_kernel.py:354-392, fused here): the lane already holds its
+      // half of the row's dO, the two halves are summed across. Every q row has
+      // exactly one dQ workgroup, which writes it (and the base-2 LSE) for the
+      // dK/dV kernel that runs next.
+      if (ok) {
+        const uint4 o4 = *(const uint4*)(O + o);
+        const uint16_t* ho = (const uint16_t*)&o4;
+        const uint16_t* hd = (const uint16_t*)&df[ks];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const int d0 = 32 * ks + 8 * grp;
-    if (my_q < g.n_q && d0 < D) {
-      const uint4 o4 = *(const uint4*)(O + qb + (size_t)my_q * D + d0);
-      const uint16_t* ho = (const uint16_t*)&o4;
-      const uint16_t* hd = (const uint16_t*)&df[ks];
+        for (int i = 0; i < 8; ++i) part += T::to_float(ho[i]) * T::to_float(hd[i]);
+      }
+    }
+    // the row's start of S: -LSE / scale with PRE, else (added after) the LSE in
+    // base 2; one rounding, once per row
+    const float lse = ok ? LSE[(size_t)bh * g.n_q + my_q] : 0.f;
+    lse2 = PRE ? (float)(-(double)lse / (double)g.scale) : lse_base2(lse);
+    // Stored negated: both kernels start their dP accumulators at -Delta, so
+    // they end as dP - Delta. With PRE the dO operand and -Delta carry pre.
+    ndlt = PRE ? -half_sum(part) * g.pre : -half_sum(part);
+    if constexpr (PRE) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) part += T::to_float(ho[i]) * T::to_float(hd[i]);
+      for (int ks = 0; ks < KS; ++ks) df[ks] = scale8<T>(df[ks], g.pre);
+    }
+    if (ok && hi == 0 && kh == 0) {            // the two kv-half waves hold the same rows
+      Delta[(size_t)bh * g.n_q + my_q] = ndlt;
+      Delta[(size_t)g.B * g.H * g.n_q + (size_t)bh * g.n_q + my_q] = lse2;
     }
   }
-  // Stored negated: both kernels start their dP accumulators at -Delta, so
-  // they end as dP - Delta. With PRE the dO operand and -Delta carry the
-  // (power-of-two) scale, so the accumulators end as (dP - Delta) * scale.
-  const float ndlt = PRE ? -wave_sum16x4(part) * g.scale : -wave_sum16x4(part);
-  if constexpr (PRE) {
+  floatx16 dq[DT];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) df[ks] = scale8<T>(df[ks], g.scale);
-  }
-  if (my_q < g.n_q && grp == 0) {
-    Delta[(size_t)bh * g.n_q + my_q] = ndlt;
-    Delta[(size_t)g.B * g.H * g.n_q + (size_t)bh * g.n_q + my_q] = lse2;
-  }
-
-  floatx4 dq[DT];
-#pragma unroll
-  for (int i = 0; i < DT; ++i) dq[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < DT; ++i) dq[i] = splat16(0.f);
 
   const int e_beg = row_ptr[qt], e_end = row_ptr[qt + 1];
-  DmaTile<D> dma;
+  DmaTile<D, 4, true> dma;
   dma.init(tid);
-  // K / V tiles: full tiles by LDS-DMA, the ragged last one through registers
-  // (rows past n_kv zero).
   auto stage = [&](int k0, int buf) {
-    if (k0 + kTileN <= g.n_kv) {
-      dma.load(K + kb, k0, sk[buf]);
-      dma.load(V + kb, k0, sv[buf]);
-    } else {
-      Tile t;
-      t.load(K + kb, k0, g.n_kv, tid);
-      t.store(sk[buf], tid);
-      t.load(V + kb, k0, g.n_kv, tid);
-      t.store(sv[buf], tid);
-      dma_wait();   // nothing of this branch pending where it rejoins the DMA path
-    }
+    dma.load(K + kb, k0, g.n_kv, stile + buf * TILE);
+    dma.load(V + kb, k0, g.n_kv, stile + (2 + buf) * TILE);
   };
   if (e_beg < e_end) stage((row_idx[e_beg] & kIdxMask) * kTileN, 0);
   dma_wait();
   __syncthreads();
-  const int q_hi_wave = min(q0 + 15, g.n_q - 1);
   for (int e = e_beg; e < e_end; ++e) {
     const int buf = (e - e_beg) & 1;
     const int ent = row_idx[e];
     const int k0 = (ent & kIdxMask) * kTileN;
     const bool partial = (ent >> kPartialBit) & 1;
-    const bool has_next = e + 1 < e_end;
-    if (has_next) stage((row_idx[e + 1] & kIdxMask) * kTileN, buf ^ 1);
-    const uint16_t* ck = sk[buf];
-    const uint16_t* cv = sv[buf];
-    const bool need_mask = partial || (q0 + 15 >= g.n_q) || (k0 + kTileN > g.n_kv) ||
-                           !tile_all_visible(g, q0, q_hi_wave, k0, k0 + kTileN - 1);
-    floatx4 ds[4];
+    if (e + 1 < e_end) stage((row_idx[e + 1] & kIdxMask) * kTileN, buf ^ 1);
+    const uint16_t* ck = stile + buf * TILE;
+    const uint16_t* cv = stile + (2 + buf) * TILE;
+    const int kw0 = k0 + 32 * kh;              // the wave's first kv row
+    // left out where none of the wave's rows sees one of its keys
+    if (!tile_unseen(g, q0w, q0w + 31, kw0, 32)) {
+      const bool need_mask = partial || (q0w + 31 >= g.n_q) || (kw0 + 32 > g.n_kv) ||
+                             !tile_all_visible(g, q0w, q0w + 31, kw0, kw0 + 31);
+      floatx16 s = splat16(PRE ? lse2 : 0.f), dp = splat16(ndlt);
+      // operands read kAhead products ahead, in a pinned order (as in dK/dV)
+      auto row_op = [&](int i) { return at.rows(i & 1 ? cv : ck, kh, i >> 1); };
+      uint4 op[kAhead];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      floatx4 s = floatx4{0.f, 0.f, 0.f, 0.f};
-      floatx4 dp = floatx4{ndlt, ndlt, ndlt, ndlt};
-      const int r = rho(t, col);
-      mfma_priority_hi<(D <= 64)>();
+      for (int i = 0; i < kAhead && i < 2 * KS; ++i) op[i] = row_op(i);
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int d0 = 32 * ks + 8 * grp;
-        const uint4 ak = (d0 < D) ? lds_row8<D>(ck, r, d0) : make_uint4(0, 0, 0, 0);
-        const uint4 av = (d0 < D) ? lds_row8<D>(cv, r, d0) : make_uint4(0, 0, 0, 0);
-        s = T::mfma(ak, qf[ks], s);
-        dp = T::mfma(av, df[ks], dp);
+      for (int i = 0; i < 2 * KS; ++i) {
+        if (i & 1) dp = T::mfma32(op[i % kAhead], df[i >> 1], dp);
+        else s = T::mfma32(op[i % kAhead], qf[i >> 1], s);
+        if (i + kAhead < 2 * KS) op[i % kAhead] = row_op(i + kAhead);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      mfma_priority_lo<(D <= 64)>();
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], g.scale_log2, -lse2));
-        ds[t][i] = PRE ? pv * dp[i] : pv * (dp[i] * g.scale);
+      for (int r = 0; r < 16; ++r) {
+        const float p = __builtin_amdgcn_exp2f(PRE ? s[r] * g.scale_log2 : __builtin_fmaf(s[r], g.scale_log2, -lse2));
+        dp[r] = PRE ? p * dp[r] : p * (dp[r] * g.scale);
+      }
+      if (need_mask) {     // masked elements: dS = 0 (bit select, as in the dK/dV kernel)
+        const uint64_t bits = row_valid_bits(opaque_blocks(g), q0w + (lane_now() & 31), k0, partial);
+        const LaneBits32 vis(kh ? (uint32_t)(bits >> 32) : (uint32_t)bits, lane_now() >> 5);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dp[r] = __int_as_float(__float_as_int(dp[r]) & vis.mask(r));
+      }
+      const uint4 pk[2] = {pack8<T>(dp, 0), pack8<T>(dp, 1)};
+      auto col_op = [&](int i) { return at.cols(ck, 2 * kh + i / DT, i % DT); };
+      uint4 ot[kAhead];
+#pragma unroll
+      for (int i = 0; i < kAhead && i < 2 * DT; ++i) ot[i] = col_op(i);
+#pragma unroll
+      for (int i = 0; i < 2 * DT; ++i) {
+        dq[i % DT] = T::mfma32(ot[i % kAhead], pk[i / DT], dq[i % DT]);
+        if (i + kAhead < 2 * DT) ot[i % kAhead] = col_op(i + kAhead);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if (need_mask) {     // masked elements: dS = 0 (bit select, as in the dK/dV kernel)
-      const LaneBits vis(row_valid_bits(g, my_q, k0, partial), grp);
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ds[t][i] = vis.pick(t, i, ds[t][i], 0.f);
-    }
-    mfma_priority_hi<(D <= 64)>();
-#pragma unroll
-    for (int st = 0; st < 2; ++st) {
-      const uint4 b = pack8<T>(ds[2 * st], ds[2 * st + 1]);
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) dq[dt] = T::mfma(lds_tr8<D>(ck, 32 * st, 16 * dt, lane), b, dq[dt]);
-    }
-    mfma_priority_lo<(D <= 64)>();
     dma_wait();        // the next tile's LDS-DMA has landed before the barrier
     __syncthreads();
   }
-  if (my_q < g.n_q) {
+  // the kv halves' sums meet in LDS (the K buffers are free: every wave passed
+  // the loop's last barrier): kh = 1 waves store, kh = 0 waves add theirs
+  floatx4* red = (floatx4*)stile + qh * (DT * 4 * 64);
+  const int lane_e = lane_now(), hi_e = lane_e >> 5;
+  if (kh == 1) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      uint2 w;
-      w.x = pack2<T>(dq[dt][0], dq[dt][1]);
-      w.y = pack2<T>(dq[dt][2], dq[dt][3]);
-      *(uint2*)(dQ + qb + (size_t)my_q * D + 16 * dt + 4 * grp) = w;
-    }
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        red[(dt * 4 + q) * 64 + lane_e] = floatx4{dq[dt][4 * q], dq[dt][4 * q + 1], dq[dt][4 * q + 2], dq[dt][4 * q + 3]};
   }
+  __syncthreads();
+  if (kh == 1) return;
+  const float post = PRE ? g.post : 1.f;
+  const int my_q = q0w + (lane_e & 31);
+  if (my_q >= g.n_q) return;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int q = 0; q < (D >= 32 ? 4 : 2); ++q) {      // D = 16: elements past 15 do not exist
+      const floatx4 r = red[(dt * 4 + q) * 64 + lane_e];
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (dq[dt][4 * q + i] + r[i]) * post;
+      *(uint2*)(dQ + qb + (size_t)my_q * D + 32 * dt + 8 * q + 4 * hi_e) =
+          make_uint2(pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3]));
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -948,7 +999,6 @@ __global__ __launch_bounds__(256, 4) void dq_kernel_q64(
     const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ row_idx, int n_qt,
     const int32_t* __restrict__ dq_order) {
   constexpr int D = 64, KS = 2, DT = 4;
-  using Tile = RowTile<D>;
   __shared__ __align__(16) uint16_t sk[2][64 * D];
   __shared__ __align__(16) uint16_t sv[2][64 * D];
 
@@ -986,10 +1036,10 @@ __global__ __launch_bounds__(256, 4) void dq_kernel_q64(
     }
     lse2[b] = ok ? lse_base2(LSE[(size_t)bh * g.n_q + my_q]) : 0.f;
     // stored negated (and scaled with PRE), as in dq_kernel_16
-    ndlt[b] = PRE ? -wave_sum16x4(part) * g.scale : -wave_sum16x4(part);
+    ndlt[b] = PRE ? -wave_sum16x4(part) * g.pre : -wave_sum16x4(part);
     if constexpr (PRE) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) df[b][ks] = scale8<T>(df[b][ks], g.scale);
+      for (int ks = 0; ks < KS; ++ks) df[b][ks] = scale8<T>(df[b][ks], g.pre);
     }
     if (ok && grp == 0 && kh == 0) {     // the two kv-half waves hold the same rows
       Delta[(size_t)bh * g.n_q + my_q] = ndlt[b];
@@ -1007,17 +1057,8 @@ __global__ __launch_bounds__(256, 4) void dq_kernel_q64(
   DmaTile<D> dma;
   dma.init(tid);
   auto stage = [&](int k0, int buf) {
-    if (k0 + kTileN <= g.n_kv) {
-      dma.load(K + kb, k0, sk[buf]);
-      dma.load(V + kb, k0, sv[buf]);
-    } else {
-      Tile t;
-      t.load(K + kb, k0, g.n_kv, tid);
-      t.store(sk[buf], tid);
-      t.load(V + kb, k0, g.n_kv, tid);
-      t.store(sv[buf], tid);
-      dma_wait();   // nothing of this branch pending where it rejoins the DMA path
-    }
+    dma.load(K + kb, k0, g.n_kv, sk[buf]);
+    dma.load(V + kb, k0, g.n_kv, sv[buf]);
   };
   if (e_beg < e_end) stage((row_idx[e_beg] & kIdxMask) * kTileN, 0);
   dma_wait();
@@ -1032,6 +1073,8 @@ __global__ __launch_bounds__(256, 4) void dq_kernel_q64(
     const uint16_t* ck = sk[buf];
     const uint16_t* cv = sv[buf];
     const int kw0 = k0 + 32 * kh;              // the wave's first kv row
+    // left out where none of the wave's rows sees one of its keys
+    if (!tile_unseen(g, q0w, q0w + 31, kw0, 32)) {
     const bool need_mask = partial || (q0w + 31 >= g.n_q) || (kw0 + 32 > g.n_kv) ||
                            !tile_all_visible(g, q0w, q_hi_wave, kw0, kw0 + 31);
     floatx4 ds[2][2];                          // [subtile 2 kh + u][q block]
@@ -1092,6 +1135,7 @@ __global__ __launch_bounds__(256, 4) void dq_kernel_q64(
       for (int b = 0; b < 2; ++b) dq[b][dt] = T::mfma(a, pb[b], dq[b][dt]);
     }
     mfma_priority_lo<true>();
+    }
     dma_wait();        // the next tile's LDS-DMA has landed before the barrier
     __syncthreads();
   }
@@ -1116,10 +1160,9 @@ __global__ __launch_bounds__(256, 4) void dq_kernel_q64(
     if (my_q >= g.n_q) continue;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
-      const floatx4 o = red[(b * DT + dt) * 64 + lane_e];
-      uint2 w;
-      w.x = pack2<T>(dq[b][dt][0] + o[0], dq[b][dt][1] + o[1]);
-      w.y = pack2<T>(dq[b][dt][2] + o[2], dq[b][dt][3] + o[3]);
+      floatx4 o = dq[b][dt] + red[(b * DT + dt) * 64 + lane_e];
+      if constexpr (PRE) o *= g.post;
+      const uint2 w = make_uint2(pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]));
       *(uint2*)(dQ + qb + (size_t)my_q * D + 16 * dt + 4 * grp_e) = w;
     }
   }
@@ -1308,22 +1351,21 @@ void launch_bwd16_as(const Geom& g, const void* q, const void* k, const void* v,
                      const int32_t* col_ptr, const int32_t* col_idx, const KvWork& w, hipStream_t stream) {
   const int BH = g.B * g.H, BHkv = g.B * g.H_kv;
   const float* lse2 = delta + (size_t)BH * g.n_q;
-  if constexpr (D == 64)
+  if constexpr (D == 64) {
     hipLaunchKernelGGL((dq_kernel_q64<T, PRE>), dim3(n_qt * BH), dim3(256), 0, stream, g,
                        (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)o,
                        (const uint16_t*)dout, (uint16_t*)dq, lse, delta, row_ptr, row_idx, n_qt, dq_order);
-  else
-    hipLaunchKernelGGL((dq_kernel_16<T, D, PRE>), dim3(n_qt * BH), dim3(256), 0, stream, g,
-                       (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)o,
-                       (const uint16_t*)dout, (uint16_t*)dq, lse, delta, row_ptr, row_idx, n_qt, dq_order);
-  if constexpr (D == 64)
     hipLaunchKernelGGL((dkdv_kernel_q64<T, PRE>), dim3(w.n_items * BHkv), dim3(256), 0, stream, g,
                        (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)dout,
                        (uint16_t*)dk, (uint16_t*)dv, lse2, delta, col_ptr, col_idx, w);
-  else
+  } else {
+    hipLaunchKernelGGL((dq_kernel_16<T, D, PRE>), dim3(n_qt * BH), dim3(256), 0, stream, g,
+                       (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)o,
+                       (const uint16_t*)dout, (uint16_t*)dq, lse, delta, row_ptr, row_idx, n_qt, dq_order);
     hipLaunchKernelGGL((dkdv_kernel_16<T, D, PRE>), dim3(w.n_items * BHkv), dim3(256), 0, stream, g,
                        (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)dout,
                        (uint16_t*)dk, (uint16_t*)dv, lse2, delta, col_ptr, col_idx, w);
+  }
 }
 
 template <typename T, int D>

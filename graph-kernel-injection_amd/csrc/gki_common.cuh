@@ -249,6 +249,8 @@ struct Lane32 {
     tr[0] = 2 * lds_off<D, true>(r, c);
     tr[1] = 2 * lds_off<D, true>(r + 8, c);
   }
+  // From here on the compiler takes the offsets for new values.
+  __device__ inline void pin() { asm volatile("" : "+v"(row), "+v"(tr[0]), "+v"(tr[1])); }
   // Row operand: rows 32 t + (l & 31), columns 16 ks + 8 (l >> 5) .. +7.
   __device__ inline uint4 rows(const uint16_t* tile, int t, int ks) const {
     return *(const uint4*)((const char*)tile + 64 * D * t + (row ^ (32 * ks)));
@@ -544,14 +546,18 @@ struct Geom {
   float qk_scale_log2;
   uint32_t q_and, q_xor;
   // 16-bit backward: dS = P (dP - Delta) scale, cast to 16 bits before the
-  // dK / dQ products. For a power-of-two scale in [2^-4, 1] (1/8 at
-  // head_dim 64) the kernels multiply the V (dK/dV) or dO (dQ) operand and
-  // -Delta by it once: every product and partial sum of the dP accumulator
-  // is then the same value times the scale (exact in fp32), so it ends as
-  // (dP - Delta) scale and dS costs one multiply (prescale = 1). Only a 16-bit
-  // operand that the scale takes below the smallest normal rounds (by at most
-  // half its subnormal spacing, 2^-25 for fp16). Otherwise prescale = 0.
+  // dK / dQ products. For a scale in [2^-4, 2) (bf16: [2^-30, 2^30)) the kernels
+  // multiply the V (dK/dV) or dO (dQ) operand and -Delta by `pre`, the power of
+  // two at or below it, once: every product and partial sum of the dP accumulator is then
+  // the same value times a power of two (exact in fp32), so it ends as
+  // (dP - Delta) pre and dS / post costs one multiply; the rest of the scale,
+  // post = scale / pre in [1, 2) (1 at head_dim 64, sqrt 2 at 128), multiplies
+  // the fp32 dK / dQ sums once (prescale = 1). dS / post rounds to 16 bits with
+  // the relative error of dS. Only a 16-bit operand that `pre` takes below the
+  // smallest normal rounds (by at most half its subnormal spacing, 2^-25 for
+  // fp16). Otherwise prescale = 0: the scaled dS is cast, pre = post = 1.
   int prescale;
+  float pre, post;
   int causal, sink, window;
   // original block mask (used only for tiles flagged partial)
   const int32_t* mask;
@@ -722,11 +728,19 @@ __device__ inline bool tile_all_visible(const Geom& g, int q_lo, int q_hi, int k
   return (k_hi < g.sink) || (k_lo >= qb - g.window + 1);
 }
 
-// True when no row of [q_lo, q_hi] sees a key of the tile [k0, k0 + kTileN) under
-// the token rule (never for a tile the rule does not apply to).
-__host__ __device__ inline bool tile_unseen(const Geom& g, int q_lo, int q_hi, int k0) {
+// The geometry with block sizes the compiler cannot follow back: the divisions
+// of a rarely taken mask branch are then not hoisted into registers held
+// through a kernel's tile loop.
+__device__ inline Geom opaque_blocks(Geom g) {
+  asm volatile("" : "+s"(g.bm), "+s"(g.bn));
+  return g;
+}
+
+// True when no row of [q_lo, q_hi] sees one of the n_k keys from k0 on under the
+// token rule (never where the rule does not apply).
+__host__ __device__ inline bool tile_unseen(const Geom& g, int q_lo, int q_hi, int k0, int n_k) {
   return g.causal != 0 && (k0 > q_hi + g.q_off ||
-                           (k0 >= g.sink && k0 + kTileN <= q_lo + g.q_off - word_window(g) + 1));
+                           (k0 >= g.sink && k0 + n_k <= q_lo + g.q_off - word_window(g) + 1));
 }
 
 // XCD-aware remap: hardware dispatches workgroup b to XCD b % 8. Give each XCD

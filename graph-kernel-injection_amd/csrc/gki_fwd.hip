@@ -221,7 +221,7 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 4 : 2) void fwd_kernel_16(
       // Left out where no row of this wave sees a key of the tile (a listed tile
       // is one that some of the workgroup's 128 rows sees): 2.5% of a forward
       // over 18-tile rows, 0.7% over 67 (head_dim 64).
-      if (!tile_unseen(g, qw, qw + 31, tile_k0(ent))) {
+      if (!tile_unseen(g, qw, qw + 31, tile_k0(ent), kTileN)) {
         floatx16 s[2];
         uint4 p[4];
         mfma_priority_hi<true>();

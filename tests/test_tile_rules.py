@@ -45,9 +45,9 @@ def test_unseen_tiles_are_exactly_those_without_a_visible_key(rules_exe):
         window = int(rng.choice([0, 1, 31, 64, 100, 700, 2**31 - 1]))
         vis = so.token_mask(n_q, n_kv, sink, min(window, n_q + n_kv + 1)) if causal else np.ones((n_q, n_kv), bool)
         for q_lo in range(0, n_q, 32):
-            for k0 in range(0, n_kv, TILE):
-                lines.append(f"{n_q} {n_kv} {int(causal)} {sink} {window} {q_lo} {q_lo + 31} {k0}")
-                want.append((not causal, bool(vis[q_lo:q_lo + 32, k0:k0 + TILE].any()), q_lo + 32 <= n_q))
+            for k0, n_k in [(k, n) for n in (TILE, TILE // 2) for k in range(0, n_kv, n)]:
+                lines.append(f"{n_q} {n_kv} {int(causal)} {sink} {window} {q_lo} {q_lo + 31} {k0} {n_k}")
+                want.append((not causal, bool(vis[q_lo:q_lo + 32, k0:k0 + n_k].any()), q_lo + 32 <= n_q))
     out = subprocess.run([rules_exe], input="\n".join(lines) + "\n", capture_output=True, text=True, check=True,
                          timeout=120).stdout.split()
     assert len(out) == len(want)

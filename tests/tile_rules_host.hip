@@ -1,7 +1,7 @@
 // Host driver for tests/test_tile_rules.py: the kernels' tile rules
 // (gki_common.cuh) on the CPU.
 //
-// stdin lines: n_q n_kv causal sink window q_lo q_hi k0
+// stdin lines: n_q n_kv causal sink window q_lo q_hi k0 n_k
 // stdout: tile_unseen, per line.
 #include <cstdio>
 
@@ -9,11 +9,11 @@
 
 int main() {
   gki::Geom g{};
-  int q_lo, q_hi, k0;
-  while (std::scanf("%d %d %d %d %d %d %d %d", &g.n_q, &g.n_kv, &g.causal, &g.sink, &g.window, &q_lo, &q_hi,
-                    &k0) == 8) {
+  int q_lo, q_hi, k0, n_k;
+  while (std::scanf("%d %d %d %d %d %d %d %d %d", &g.n_q, &g.n_kv, &g.causal, &g.sink, &g.window, &q_lo, &q_hi,
+                    &k0, &n_k) == 9) {
     g.q_off = g.n_kv - g.n_q;
-    std::printf("%d\n", (int)gki::tile_unseen(g, q_lo, q_hi, k0));
+    std::printf("%d\n", (int)gki::tile_unseen(g, q_lo, q_hi, k0, n_k));
   }
   return 0;
 }
