@@ -398,12 +398,13 @@ struct DmaTile {
       off[p] = row * D + ((pch ^ lds_swz<D, ROW32>(row)) << 3);
     }
   }
-  // Rows r0 .. r0+63 (r0 < n_rows) of a matrix of n_rows rows through a buffer resource over
+  // Rows r0 .. r0+63 of a matrix of n_rows rows through a buffer resource over
   // those that exist: the tile base is uniform, so a tile costs no per-lane
   // address arithmetic, and the resource's range check makes the rows past the
   // last one zeros in LDS (no separate path for a ragged tile).
   __device__ inline void load(const uint16_t* base, int r0, int n_rows, const uint16_t* lds) const {
-    const i32x4 rsrc = buffer_rsrc(base + (size_t)r0 * D, (n_rows - r0 < 64 ? n_rows - r0 : 64) * D * 2);
+    const int left = n_rows - r0;
+    const i32x4 rsrc = buffer_rsrc(base + (size_t)r0 * D, (left < 0 ? 0 : left < 64 ? left : 64) * D * 2);
     const uint32_t l0 = lds_addr(lds);
 #pragma unroll
     for (int p = 0; p < NP; ++p) {

@@ -347,6 +347,187 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 4 : 2) void fwd_kernel_16(
 }
 
 // ---------------------------------------------------------------------------
+// The same for grids too short for the card (kSplitGrid): the 128-row q tile of
+// the schedule is two workgroups of 64 rows, and a workgroup's eight waves are
+// two blocks of 32 rows x 4 shares of the keys. A step stages two kv tiles of
+// the list (double-buffered) and share x takes 32 keys of them: tile x >> 1, half
+// x & 1. Each share keeps a softmax state; they merge through LDS at the end, in
+// order (share x the 32-element slice x of O). Bound by the latency of a wave's
+// chain (products, softmax, products, barrier) per step: the split makes it a
+// quarter as long per tile and puts twice the workgroups on the card. Kernel
+// times, us: 500 queries behind 8500 keys, B1 H32, D128 (128 tiles) 46.8 -> 30.6;
+// B1 H8 N1000 D64 (64) 20.7 -> 12.9; B1 H4 N1000 D128 (32) 18.2 -> 13.6.
+// ---------------------------------------------------------------------------
+template <typename T, int D>
+__global__ __launch_bounds__(512, 2) void fwd_split_16(
+    Geom g, const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
+    const uint16_t* __restrict__ V, uint16_t* __restrict__ O, float* __restrict__ LSE,
+    const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ row_idx, int n_qt,
+    const int32_t* __restrict__ wg_order) {
+  constexpr int KS = D / 16;
+  constexpr int DT = D >= 32 ? D / 32 : 1;
+  constexpr int QB = 2, KB = 4, NW = QB * KB;  // row blocks, key shares, waves
+  constexpr int TPS = KB / 2;                  // kv tiles per step
+  constexpr int kAhead = 4;                    // operands read ahead
+  constexpr int TILE = kTileN * D;
+  // K, V of the steps' tiles; at the end every wave's O (fp32)
+  constexpr int OF = DT * 16 * 64;             // floats of a wave's O
+  constexpr int LDS16 = 2 * TPS * 2 * TILE > NW * OF * 2 ? 2 * TPS * 2 * TILE : NW * OF * 2;
+  __shared__ __align__(16) uint16_t stile[LDS16];
+  __shared__ float sm[NW][32], sl[NW][32];
+
+  int part;
+  const int wg = work_part_of(blockIdx.x, n_qt * g.B * g.H, 4 / QB, wg_order, part);
+  if (wg < 0) return;
+  const int bh = wg / n_qt, qt = wg - bh * n_qt;
+  const size_t qb = (size_t)bh * g.n_q * D;
+  const size_t kb = (size_t)kv_bh(g, bh) * g.n_kv * D;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, hi = lane >> 5, col = lane & 31;
+  const Lane32<D> at(lane);
+  const int blk = wave % QB, share = wave / QB;
+  const int qw = qt * kTileMF + 32 * (part * QB + blk);   // first row of this wave
+  if (qt * kTileMF + 32 * QB * part >= g.n_q) return;     // a part past the last row
+
+  const int e_beg = row_ptr[qt], n = row_ptr[qt + 1] - e_beg;
+  const int32_t* const ents = row_idx + e_beg;
+  DmaTile<D, NW, true> dma;
+  dma.init(tid);
+  auto tile_k0 = [&](int ent) { return (ent & kIdxMask) * kTileN; };
+  // the tiles of step s into buffer s & 1: K, V, K, V
+  auto stage = [&](int s) {
+#pragma unroll
+    for (int j = 0; j < TPS; ++j)
+      if (TPS * s + j < n) {
+        const int k0 = tile_k0(ents[TPS * s + j]);
+        uint16_t* const dst = stile + (2 * TPS * (s & 1) + 2 * j) * TILE;
+        dma.load(K + kb, k0, g.n_kv, dst);
+        dma.load(V + kb, k0, g.n_kv, dst + TILE);
+      }
+  };
+  uint4 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const uint4 v = q_words(g, row16_or_zero<D>(Q + qb, qw + col, g.n_q, 16 * ks + 8 * hi));
+    qf[ks] = qw + col < g.n_q ? v : make_uint4(0, 0, 0, 0);
+  }
+  floatx16 o[DT];
+#pragma unroll
+  for (int i = 0; i < DT; ++i) o[i] = splat16(0.f);
+  // the row sum of the fp32 P over the lane's keys; the lazy reference max as in
+  // fwd_kernel_16
+  float lsum = 0.f;
+  const float slack = kRescaleSlack * __builtin_amdgcn_rcpf(g.qk_scale_log2);
+  float nm = 0.f, thr = kNegInf;
+
+  const int steps = (n + TPS - 1) / TPS;
+  dma_wait();          // the Q loads, before any LDS-DMA is in flight
+  if (steps > 0) stage(0);
+  const int tj = share >> 1, th = share & 1;
+  for (int st = 0; st < steps; ++st) {
+    dma_wait();
+    __syncthreads();   // step st is in LDS, and every wave is done with the step before
+    if (st + 1 < steps) stage(st + 1);
+    const int e = TPS * st + tj;
+    if (e < n) {
+      const int ent = ents[e];
+      const int k0 = tile_k0(ent), kw = k0 + 32 * th;
+      const bool partial = (ent >> kPartialBit) & 1;
+      const uint16_t* ck = stile + (2 * TPS * (st & 1) + 2 * tj) * TILE + 32 * D * th;
+      const uint16_t* cv = ck + TILE;
+      if (!tile_unseen(g, qw, qw + 31, kw, 32)) {
+        // operands read kAhead products ahead, in a pinned order
+        floatx16 s = splat16(0.f);
+        uint4 op[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead && i < KS; ++i) op[i] = at.rows(ck, 0, i);
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+          s = T::mfma32(op[i % kAhead], qf[i], s);
+          if (i + kAhead < KS) op[i % kAhead] = at.rows(ck, 0, i + kAhead);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // V^T operands of the first products, in flight through the softmax
+        uint4 ov[kAhead];
+#pragma unroll
+        for (int i = 0; i < kAhead && i < 2 * DT; ++i) ov[i] = at.cols(cv, i / DT, i % DT);
+        if (partial || qw + 31 >= g.n_q || kw + 32 > g.n_kv || !tile_all_visible(g, qw, qw + 31, kw, kw + 31)) {
+          const uint64_t bits = row_valid_bits(opaque_blocks(g), qw + (lane_now() & 31), k0, partial);
+          const LaneBits32 vis(th ? (uint32_t)(bits >> 32) : (uint32_t)bits, lane_now() >> 5);
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[r] = vis.pick(r, s[r], kNegInf);
+        }
+        float mx = kNegInf;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+        if (__any(mx > thr)) {
+          const float mr = half_max(mx);
+          const bool grow = mr > thr;
+          const float nm1 = grow ? -mr * g.qk_scale_log2 : nm;
+          const float alpha = __builtin_amdgcn_exp2f(fminf(nm1 - nm, 0.f));
+          nm = nm1;
+          thr = grow ? mr + slack : thr;
+          lsum *= alpha;
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], g.qk_scale_log2, nm));
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) lsum += (s[r] + s[r + 1]) + (s[r + 2] + s[r + 3]);
+        const uint4 p[2] = {pack8<T>(s, 0), pack8<T>(s, 1)};
+#pragma unroll
+        for (int i = 0; i < 2 * DT; ++i) {
+          o[i % DT] = T::mfma32(ov[i % kAhead], p[i / DT], o[i % DT]);
+          if (i + kAhead < 2 * DT) ov[i % kAhead] = at.cols(cv, (i + kAhead) / DT, (i + kAhead) % DT);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  }
+  __syncthreads();
+
+  // Merge (every wave is done with the staging buffers, nothing is in flight). A
+  // share that saw no key of a row has lsum = 0 there and weighs nothing.
+  float* red = (float*)stile + (size_t)wave * OF;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *(floatx4*)(red + ((dt * 4 + q) * 64 + lane) * 4) =
+          floatx4{o[dt][4 * q], o[dt][4 * q + 1], o[dt][4 * q + 2], o[dt][4 * q + 3]};
+  lsum = half_sum(lsum);
+  if (hi == 0) {
+    sm[wave][col] = lsum > 0.f ? -nm : kNegInf;
+    sl[wave][col] = lsum;
+  }
+  __syncthreads();
+  float M = kNegInf, L = 0.f, f[KB];
+#pragma unroll
+  for (int x = 0; x < KB; ++x) M = fmaxf(M, sm[x * QB + blk][col]);
+#pragma unroll
+  for (int x = 0; x < KB; ++x) {
+    f[x] = M == kNegInf ? 0.f : __builtin_amdgcn_exp2f(sm[x * QB + blk][col] - M);
+    L += sl[x * QB + blk][col] * f[x];
+  }
+  const bool valid = L > 0.f;
+  const float inv = valid ? 1.f / L : 1.f;
+  const int my_q = qw + col;
+  if (my_q >= g.n_q) return;
+  for (int dt = share; dt < DT; dt += KB)
+#pragma unroll
+    for (int q = 0; q < (D >= 32 ? 4 : 2); ++q) {       // D = 16: rows past 15 do not exist
+      floatx4 a = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int x = 0; x < KB; ++x)
+        a += *(const floatx4*)((const float*)stile + (size_t)(x * QB + blk) * OF + ((dt * 4 + q) * 64 + lane) * 4) * f[x];
+      *(uint2*)(O + qb + (size_t)my_q * D + 32 * dt + 8 * q + 4 * hi) =
+          make_uint2(pack2<T>(a[0] * inv, a[1] * inv), pack2<T>(a[2] * inv, a[3] * inv));
+    }
+  if (share == 0 && hi == 0) LSE[(size_t)bh * g.n_q + my_q] = valid ? lse_natural(M, L) : 0.f;
+}
+
+// ---------------------------------------------------------------------------
 // fp32 path (v_mfma_f32_16x16x4f32, 64-row tiles): K and V row-major in LDS
 // (swz_f32), staged by LDS-DMA, double-buffered, one barrier per 32 or 64 keys.
 // Bound by the fp32 matrix cores (154 TFLOP/s reached by a large product): B1
@@ -571,6 +752,26 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : D * (QB == 
 template <int D>
 constexpr bool kFwdPipe = D >= 128;
 
+// Grids of at most this many 128-row tiles (one per CU) run fwd_split_16, in us
+// against fwd_kernel_16: 256 tiles D128 (33 kv tiles each) 37.0 -> 32.6, D64 (6)
+// 12.2 -> 11.8; at 512 tiles it is behind (D128 40 -> 57, D64 24 -> 28).
+constexpr int kSplitGrid = 256;
+template <typename T, int D>
+void launch_fwd16(const Geom& g, const void* q, const void* k, const void* v, void* o, float* lse,
+                  const int32_t* row_ptr, const int32_t* row_idx, int n_qt, const int32_t* wg_order,
+                  hipStream_t stream) {
+  const int grid = n_qt * g.B * g.H;
+#define GKI_FWD16(KERNEL, GRID, THREADS)                                                           \
+  hipLaunchKernelGGL(KERNEL, dim3(GRID), dim3(THREADS), 0, stream, g, (const uint16_t*)q,          \
+                     (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o, lse, row_ptr, row_idx,  \
+                     n_qt, wg_order)
+  if (grid <= kSplitGrid)
+    GKI_FWD16((fwd_split_16<T, D>), work_parts_grid(grid, 2), 512);
+  else
+    GKI_FWD16((fwd_kernel_16<T, D, kFwdPipe<D>>), grid, kFwdThreads);
+#undef GKI_FWD16
+}
+
 template <int D>
 int launch_fwd(int dtype, const Geom& g, const void* q, const void* k, const void* v, void* o,
                float* lse, const int32_t* row_ptr, const int32_t* row_idx, int n_qt,
@@ -586,13 +787,9 @@ int launch_fwd(int dtype, const Geom& g, const void* q, const void* k, const voi
     else GKI_FWD32(4);
 #undef GKI_FWD32
   } else if (dtype == kF16) {
-    hipLaunchKernelGGL((fwd_kernel_16<F16, D, kFwdPipe<D>>), dim3(grid), dim3(kFwdThreads), 0, stream, g,
-                       (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o, lse,
-                       row_ptr, row_idx, n_qt, wg_order);
+    launch_fwd16<F16, D>(g, q, k, v, o, lse, row_ptr, row_idx, n_qt, wg_order, stream);
   } else {
-    hipLaunchKernelGGL((fwd_kernel_16<BF16, D, kFwdPipe<D>>), dim3(grid), dim3(kFwdThreads), 0, stream, g,
-                       (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o, lse,
-                       row_ptr, row_idx, n_qt, wg_order);
+    launch_fwd16<BF16, D>(g, q, k, v, o, lse, row_ptr, row_idx, n_qt, wg_order, stream);
   }
   return check_launch("gki_bsa_fwd");
 }

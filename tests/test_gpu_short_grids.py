@@ -1,0 +1,43 @@
+"""Forward grids too short for the card (GPU): 16-bit grids of up to 256 128-row
+tiles share each tile's keys among a workgroup's waves, longer ones do not. At
+the edges -- one kv tile, an odd number of them, a last half of 64 rows that
+does not exist, rows that see nothing, both sides of the 256-tile line -- each
+against the fp64 oracle, with the bars of the parity tests."""
+
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import sparse_triton_kernel as stk
+from oracle import streaming_oracle as so
+
+DEV = "cuda"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,H,n_q,n_kv,D,sink,window", [
+    (1, 1, 5, 5, 16, 0, 3),             # one tile, a sliver of its rows
+    (1, 2, 64, 64, 32, 4, 64),          # the second 64 rows of the tile do not exist
+    (1, 2, 65, 129, 64, 1, 200),        # three kv tiles: an odd number, the last of one key
+    (1, 1, 130, 700, 128, 4, 40),       # a ragged chunk behind a long cache
+    (2, 2, 200, 100, 64, 0, 30),        # more queries than keys: rows that see nothing
+    (2, 64, 250, 250, 64, 4, 100),      # 256 tiles
+    (3, 43, 250, 250, 32, 4, 100),      # 258: one workgroup per tile
+])
+def test_short_grid_matches_oracle(B, H, n_q, n_kv, D, sink, window, dtype):
+    print(f"[case] B{B} H{H} nq{n_q} nkv{n_kv} D{D} S{sink} W{window} {dtype}", flush=True)
+    gen = torch.Generator().manual_seed(n_q + D)
+    q, k, v = (torch.randn(B, H, n, D, generator=gen).to(dtype) for n in (n_q, n_kv, n_kv))
+    mask = stk.make_streaming_mask(n_q, n_kv, stk.StreamingMaskSpec(sink, window), 64, 64, device=DEV)
+    out = stk.block_sparse_attention(q.to(DEV), k.to(DEV), v.to(DEV), mask, is_causal=True, sink_size=sink,
+                                     window_size=window)
+    eff = so.effective_mask(mask.cpu().numpy(), n_q, n_kv, 64, 64, True, sink, window)
+    ref, _ = so.attention_fwd(*(t.double().numpy() for t in (q, k, v)), eff, 1 / math.sqrt(D))
+    err = np.abs(out.double().cpu().numpy() - ref)
+    assert np.isfinite(err).all()
+    assert (err <= 2e-2 + 1e-2 * np.abs(ref)).all(), err.max()
