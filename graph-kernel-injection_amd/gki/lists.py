@@ -167,7 +167,7 @@ class _ScheduleCache:
     so a retired mask's storage cannot be recycled under a live class.
     """
 
-    def __init__(self, capacity: int = 64, max_classes: int = 16) -> None:
+    def __init__(self, capacity: int = 96, max_classes: int = 16) -> None:
         self._sched: "OrderedDict[tuple, object]" = OrderedDict()
         self._classes: "OrderedDict[int, Tuple[torch.Tensor, int, tuple]]" = OrderedDict()
         self._alias: dict = {}       # id(tensor) -> (weakref, version, class id)
@@ -281,6 +281,18 @@ def fwd_order(mask: torch.Tensor, sched: FwdSchedule, bh: int) -> torch.Tensor:
     cached with the schedule."""
     return _CACHE.get(mask, sched.key + ("order", bh),
                       lambda: _grid_order(sched.lists.row_ptr, sched.n_qt, bh, mask.device))
+
+
+def fwd_plan(mask: torch.Tensor, n_q: int, n_kv: int, block_m: int, block_n: int, is_causal: bool, sink: int,
+             window: int, fp32: bool, bh: int) -> Tuple[FwdSchedule, torch.Tensor]:
+    """``fwd_schedule`` and its ``fwd_order`` in one lookup (a forward call is
+    short enough for the second one to show)."""
+
+    def build() -> Tuple[FwdSchedule, torch.Tensor]:
+        sched = fwd_schedule(mask, n_q, n_kv, block_m, block_n, is_causal, sink, window, fp32)
+        return sched, fwd_order(mask, sched, bh)
+
+    return _CACHE.get(mask, ("fwd plan", n_q, n_kv, block_m, block_n, is_causal, sink, window, fp32, bh), build)
 
 
 def dkdv_items(col_ptr_host: torch.Tensor, group: int, bh_kv: int, max_chunk: int = 0):

@@ -24,7 +24,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from .lists import _CACHE, bwd_schedule, decode_schedule, fwd_order, fwd_schedule
+from .lists import _CACHE, bwd_schedule, decode_schedule, fwd_plan
 
 _DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 _HEAD_DIMS = (16, 32, 64, 128)
@@ -61,10 +61,17 @@ def _current_stream(dev: torch.device) -> int:
     return raw(dev.index) if raw is not None else torch.cuda.current_stream(dev).cuda_stream
 
 
+def _is_current(dev: torch.device) -> bool:
+    """Whether ``dev`` already is the current device (torch's query without its
+    Python wrappers when available)."""
+    raw = getattr(torch._C, "_cuda_getDevice", None)
+    return dev.index == (raw() if raw is not None else torch.cuda.current_device())
+
+
 def _on_device(dev: torch.device):
     """``dev`` as the current device for the launches (a no-op context when it
     already is)."""
-    return contextlib.nullcontext() if dev.index == torch.cuda.current_device() else torch.cuda.device(dev)
+    return contextlib.nullcontext() if _is_current(dev) else torch.cuda.device(dev)
 
 
 def _decode_splits(n_tokens: int, bh: int) -> int:
@@ -155,59 +162,66 @@ def _attention_forward(q, k, v, block_mask, softmax_scale, block_m, block_n, is_
     dev = q.device
     block_mask = _device_mask(block_mask, dev)
 
-    o = torch.empty_like(q)
-    lse = None
-    q_offset = N_KV - N_Q
     dtype = _DTYPE_CODE[q.dtype]
-    common = (block_mask.data_ptr(), n_qb, n_kb, block_m, block_n, float(softmax_scale),
-              int(bool(is_causal)), int(sink_size), int(window_size))
+    launch = (lib, q, k, v, block_mask, dtype, B, H, H_kv, N_Q, N_KV, D, n_qb, n_kb, block_m, block_n,
+              float(softmax_scale), bool(is_causal), int(sink_size), int(window_size), need_lse)
+    if _is_current(dev):
+        o, lse = _launch_forward(*launch)
+    else:
+        with torch.cuda.device(dev):
+            o, lse = _launch_forward(*launch)
+    return o, lse, q, k, v, block_mask, N_KV - N_Q
 
-    with _on_device(dev):
-        stream = _current_stream(dev)
-        ts = _lib.tile_sizes()
-        if N_Q <= ts["decode_max_q"] and D in _DECODE_HEAD_DIMS:
-            sched = decode_schedule(block_mask, N_Q, N_KV, block_m, block_n, bool(is_causal),
-                                    int(sink_size), int(window_size))
-            _, n_splits, ws_floats = _decode_plan(lib, dtype, B, H, H_kv, N_Q, D, sched.n_tokens,
-                                                  bool(sched.ring))
-            n_lse = B * H * N_Q
-            if need_lse:
-                lse = torch.empty((B, H, N_Q), dtype=torch.float32, device=dev)
-                lse_ptr = lse.data_ptr()
-                ws_ptr = 0
-                if ws_floats:
-                    ws = torch.empty(ws_floats, dtype=torch.float32, device=dev)
-                    ws_ptr = ws.data_ptr()
-            else:
-                # one allocation: the LSE rows (padded to 256 bytes), then the workspace
-                pad = (n_lse + 63) & ~63
-                scratch = torch.empty(pad + ws_floats, dtype=torch.float32, device=dev)
-                lse_ptr = scratch.data_ptr()
-                ws_ptr = lse_ptr + 4 * pad if ws_floats else 0
-            if sched.ring:
-                # the stream is the StreamingLLM one: positions computed in
-                # the kernel (no list read), same stream and arithmetic
-                _lib.check(lib.gki_rolling_decode(
-                    q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse_ptr,
-                    dtype, B, H, H_kv, N_Q, D, int(sink_size), int(window_size), sched.ring,
-                    N_KV, float(softmax_scale), ws_ptr, n_splits, stream), "gki_rolling_decode")
-            else:
-                _lib.check(lib.gki_bsa_decode(
-                    q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse_ptr, dtype,
-                    B, H, H_kv, N_Q, N_KV, D, sched.tokens.data_ptr(), sched.n_tokens, *common,
-                    ws_ptr, n_splits, stream), "gki_bsa_decode")
-        else:
+
+def _launch_forward(lib, q, k, v, block_mask, dtype, B, H, H_kv, N_Q, N_KV, D, n_qb, n_kb, block_m, block_n,
+                    scale, causal, sink, window, need_lse):
+    """The forward launch on q's device, which is current: (o, lse or None)."""
+    dev = q.device
+    stream = _current_stream(dev)
+    o = torch.empty_like(q)
+    if N_Q <= _lib.tile_sizes()["decode_max_q"] and D in _DECODE_HEAD_DIMS:
+        sched = decode_schedule(block_mask, N_Q, N_KV, block_m, block_n, causal, sink, window)
+        _, n_splits, ws_floats = _decode_plan(lib, dtype, B, H, H_kv, N_Q, D, sched.n_tokens, bool(sched.ring))
+        lse = None
+        if need_lse:
             lse = torch.empty((B, H, N_Q), dtype=torch.float32, device=dev)
-            sched = fwd_schedule(block_mask, N_Q, N_KV, block_m, block_n, bool(is_causal),
-                                 int(sink_size), int(window_size), q.dtype == torch.float32)
-            order = fwd_order(block_mask, sched, B * H)
-            _lib.check(lib.gki_bsa_fwd(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), dtype,
-                B, H, H_kv, N_Q, N_KV, D, sched.lists.row_ptr.data_ptr(),
-                sched.lists.row_buf.data_ptr(), sched.n_qt, order.data_ptr(), *common, stream),
-                "gki_bsa_fwd")
-
-    return o, lse, q, k, v, block_mask, q_offset
+            lse_ptr = lse.data_ptr()
+            ws_ptr = 0
+            if ws_floats:
+                ws = torch.empty(ws_floats, dtype=torch.float32, device=dev)
+                ws_ptr = ws.data_ptr()
+        else:
+            # one allocation: the LSE rows (padded to 256 bytes), then the workspace
+            pad = (B * H * N_Q + 63) & ~63
+            scratch = torch.empty(pad + ws_floats, dtype=torch.float32, device=dev)
+            lse_ptr = scratch.data_ptr()
+            ws_ptr = lse_ptr + 4 * pad if ws_floats else 0
+        if sched.ring:
+            # the stream is the StreamingLLM one: positions computed in
+            # the kernel (no list read), same stream and arithmetic
+            rc = lib.gki_rolling_decode(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse_ptr, dtype, B, H, H_kv, N_Q, D,
+                sink, window, sched.ring, N_KV, scale, ws_ptr, n_splits, stream)
+            if rc:
+                _lib.check(rc, "gki_rolling_decode")
+        else:
+            rc = lib.gki_bsa_decode(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse_ptr, dtype,
+                B, H, H_kv, N_Q, N_KV, D, sched.tokens.data_ptr(), sched.n_tokens, block_mask.data_ptr(), n_qb,
+                n_kb, block_m, block_n, scale, causal, sink, window, ws_ptr, n_splits, stream)
+            if rc:
+                _lib.check(rc, "gki_bsa_decode")
+        return o, lse
+    lse = torch.empty((B, H, N_Q), dtype=torch.float32, device=dev)
+    sched, order = fwd_plan(block_mask, N_Q, N_KV, block_m, block_n, causal, sink, window, dtype == 0, B * H)
+    lists = sched.lists
+    rc = lib.gki_bsa_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), dtype,
+        B, H, H_kv, N_Q, N_KV, D, lists.row_ptr.data_ptr(), lists.row_buf.data_ptr(), sched.n_qt,
+        order.data_ptr(), block_mask.data_ptr(), n_qb, n_kb, block_m, block_n, scale, causal, sink, window, stream)
+    if rc:
+        _lib.check(rc, "gki_bsa_fwd")
+    return o, lse
 
 
 class _BlockSparseFlashAttention(torch.autograd.Function):
@@ -315,12 +329,13 @@ def block_sparse_attention(
     """
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(q.shape[-1])
-    args = (q.contiguous(), k.contiguous(), v.contiguous(), block_mask, float(softmax_scale),
-            int(block_m), int(block_n), bool(is_causal), int(sink_size), int(window_size))
     if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)):
         # nothing to differentiate (inference, a decode step): the same forward
         # without the autograd node and its saved tensors
-        return _attention_forward(*args, enable_gqa, need_lse=False)[0]
+        return _attention_forward(q, k, v, block_mask, softmax_scale, block_m, block_n, is_causal, sink_size,
+                                  window_size, enable_gqa, need_lse=False)[0]
+    args = (q.contiguous(), k.contiguous(), v.contiguous(), block_mask, float(softmax_scale),
+            int(block_m), int(block_n), bool(is_causal), int(sink_size), int(window_size))
     if enable_gqa:
         args += (True,)
     return _BlockSparseFlashAttention.apply(*args)
