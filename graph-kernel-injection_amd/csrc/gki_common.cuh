@@ -143,13 +143,8 @@ __device__ inline uint4 scale8(const uint4& v, float s) {
                     pack2<T>(f[6], f[7]));
 }
 
-// Pack 8 fp32 values into 8 16-bit elements (one 16x16x32 MFMA operand).
-template <typename T>
-__device__ inline uint4 pack8(const float* v) {
-  return make_uint4(pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3]), pack2<T>(v[4], v[5]),
-                    pack2<T>(v[6], v[7]));
-}
-// Same, from the accumulators of two 16x16 subtiles (rows 0-3 then 4-7).
+// Accumulators of two 16x16 subtiles (rows 0-3 then 4-7) packed to eight 16-bit
+// elements: one 16x16x32 MFMA operand.
 template <typename T>
 __device__ inline uint4 pack8(const floatx4& lo, const floatx4& hi) {
   return make_uint4(pack2<T>(lo[0], lo[1]), pack2<T>(lo[2], lo[3]), pack2<T>(hi[0], hi[1]),
@@ -222,9 +217,9 @@ __device__ inline uint4 lds_tr8(const uint16_t* tile, int k0, int n0, int lane) 
   return make_uint4(a.x, a.y, b.x, b.y);
 }
 // 16-byte row read (8 elements starting at a multiple-of-8 column).
-template <int D, bool ROW32 = false>
+template <int D>
 __device__ inline uint4 lds_row8(const uint16_t* tile, int row, int col) {
-  return *(const uint4*)(tile + lds_off<D, ROW32>(row, col));
+  return *(const uint4*)(tile + lds_off<D>(row, col));
 }
 
 // Operands of v_mfma_f32_32x32x16 (lane l: row or column l & 31, elements
@@ -274,44 +269,6 @@ __device__ inline int lane_now() {
 }
 // Row (of 32) of register r in lane half hi of a 32x32 accumulator.
 __device__ inline int acc32_row(int r, int hi) { return 8 * (r >> 2) + 4 * hi + (r & 3); }
-
-// Stage a 64-row tile of a row-major [n, D] 16-bit matrix: each thread moves
-// P 16-byte chunks, consecutive threads covering consecutive bytes of a row.
-// The loads go through a buffer resource over the rows that exist, so rows at
-// or past n_rows read as zero without a per-element predicate, and the lane
-// offsets are 32-bit (chunk c of the tile sits at byte 16 c).
-template <int D, int NT = 256, bool ROW32 = false>
-struct RowTile {
-  static constexpr int CPR = D / 8;          // 16-byte chunks per row
-  static constexpr int CH = 64 * CPR;
-  static constexpr int P = (CH + NT - 1) / NT;
-  uint4 reg[P];
-  // base and r0 are uniform at every call site (kernel arguments and a tile
-  // index from the schedule); reading them through readfirstlane lets the
-  // compiler keep the resource in scalar registers (no per-lane loop).
-  __device__ inline void load(const uint16_t* base, int r0, int n_rows, int tid) {
-    const int rows = max(0, min(64, n_rows - r0));
-    const uint64_t a = (uint64_t)(uintptr_t)(base + (size_t)r0 * D);
-    const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) |
-                       ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32);
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(uintptr_t)u, (short)0, __builtin_amdgcn_readfirstlane(rows * D * 2), 0x00020000);
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      const int c = tid + NT * p;
-      reg[p] = make_uint4(0, 0, 0, 0);
-      if (CH % NT == 0 || c < CH)
-        reg[p] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, 16 * c, 0, 0));
-    }
-  }
-  __device__ inline void store(uint16_t* lds, int tid) const {
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      const int c = tid + NT * p;
-      if (c < CH) *(uint4*)(lds + lds_off<D, ROW32>(c / CPR, (c % CPR) * 8)) = reg[p];
-    }
-  }
-};
 
 // 16 bytes at (row, d0) of a row-major [n_rows, D] 16-bit matrix, zero when
 // row >= n_rows or d0 >= D (n_rows >= 1). The load is unconditional, from a
@@ -381,7 +338,6 @@ __device__ inline void dma_wait() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 // belongs at its LDS position. The workgroup's NW waves cover the tile's D/8
 // blocks of 1 KB (block NW p + wave for p = 0, 1, ...); `off` is the lane's
 // element offset inside the tile for each block it moves (computed once).
-// Only for tiles whose 64 rows are all in bounds.
 template <int D, int NW = 4, bool ROW32 = false>
 struct DmaTile {
   static constexpr int NB = D / 8;                     // 1 KB blocks per tile
@@ -405,16 +361,6 @@ struct DmaTile {
   __device__ inline void load(const uint16_t* base, int r0, int n_rows, const uint16_t* lds) const {
     const int left = n_rows - r0;
     const i32x4 rsrc = buffer_rsrc(base + (size_t)r0 * D, (left < 0 ? 0 : left < 64 ? left : 64) * D * 2);
-    const uint32_t l0 = lds_addr(lds);
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int blk = NW * p + wave;
-      if (NB % NW == 0 || blk < NB) dma_buf16(rsrc, 2 * off[p], l0 + blk * 1024);
-    }
-  }
-  // The same for a tile known to be whole.
-  __device__ inline void load(const uint16_t* base, int r0, const uint16_t* lds) const {
-    const i32x4 rsrc = buffer_rsrc(base + (size_t)r0 * D, 64 * D * 2);
     const uint32_t l0 = lds_addr(lds);
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
