@@ -41,3 +41,34 @@ def test_short_grid_matches_oracle(B, H, n_q, n_kv, D, sink, window, dtype):
     err = np.abs(out.double().cpu().numpy() - ref)
     assert np.isfinite(err).all()
     assert (err <= 2e-2 + 1e-2 * np.abs(ref)).all(), err.max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("B,H,H_kv,n_q,n_kv,sink,window", [
+    (2, 4, 4, 130, 130, 4, 50),          # 24 64-row tiles: four workgroups each (dK/dV too, but at D 128)
+    (3, 48, 48, 128, 190, 1, 70),        # 288: two each
+    (3, 96, 48, 190, 100, 0, 40),        # 864: one each; grouped-query, rows that see nothing
+])
+def test_fp32_grids_match_oracle(B, H, H_kv, n_q, n_kv, sink, window, D):
+    """fp32 forward and backward at each number of workgroups per tile, held to
+    1e-5 (N(0, 1) inputs, as the parity tests)."""
+    print(f"[case] B{B} H{H}/{H_kv} nq{n_q} nkv{n_kv} D{D} fp32", flush=True)
+    gen = torch.Generator().manual_seed(H + D)
+    q, do = (torch.randn(B, H, n_q, D, generator=gen) for _ in range(2))
+    k, v = (torch.randn(B, H_kv, n_kv, D, generator=gen) for _ in range(2))
+    mask = stk.make_streaming_mask(n_q, n_kv, stk.StreamingMaskSpec(sink, window), 64, 64, device=DEV)
+    leaves = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
+    out = stk.block_sparse_attention(*leaves, mask, is_causal=True, sink_size=sink, window_size=window,
+                                     enable_gqa=H != H_kv)
+    out.backward(do.to(DEV))
+    eff = so.effective_mask(mask.cpu().numpy(), n_q, n_kv, 64, 64, True, sink, window)
+    group = H // H_kv
+    qn, kn, vn, dn = (t.double().numpy() for t in (q, k, v, do))
+    kx, vx = so.expand_kv_heads(kn, group), so.expand_kv_heads(vn, group)
+    o, _ = so.attention_fwd(qn, kx, vx, eff, 1 / math.sqrt(D))
+    dq, dk, dv = so.attention_bwd(qn, kx, vx, dn, eff, 1 / math.sqrt(D))
+    refs = (o, dq, so.reduce_kv_grad(dk, group), so.reduce_kv_grad(dv, group))
+    for name, got, ref in zip(("O", "dQ", "dK", "dV"), [out] + [t.grad for t in leaves], refs):
+        err = np.abs(got.detach().double().cpu().numpy() - ref)
+        assert np.isfinite(err).all() and err.max() <= 1e-5, (name, err.max())
