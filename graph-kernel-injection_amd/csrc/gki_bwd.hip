@@ -141,15 +141,16 @@ __global__ __launch_bounds__(256) void dkdv_reduce_kernel(Geom g, KvWork w,
 // At head_dim 64 the card's power is the bound (1.9-2.1 GHz under the backward)
 // and this form, 7% fewer cycles at a 10% lower clock, ran 2-3% slower than the
 // 16x16x32 quadrants below.
-// PRE: Geom::prescale. A template parameter, so neither form carries a branch.
-template <typename T, int D, bool PRE>
-__global__ __launch_bounds__(256, D <= 32 ? 4 : D == 64 ? 3 : PRE ? 2 : 1) void dkdv_kernel_16(
+// FORM: Geom::bwd_form. A template parameter, so no form carries a branch.
+template <typename T, int D, int FORM>
+__global__ __launch_bounds__(256, D <= 32 ? 4 : FORM != kBwdPlain ? 2 : 1) void dkdv_kernel_16(
     Geom g, const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ dO, uint16_t* __restrict__ dK,
     uint16_t* __restrict__ dV, const float* __restrict__ LSE2, const float* __restrict__ Delta,
     const int32_t* __restrict__ col_ptr, const int32_t* __restrict__ col_idx, KvWork w) {
-  // LSE2: -LSE / scale rows when PRE, else base-2 LSE rows; Delta: -Delta rows
+  // LSE2: -LSE / scale rows when ROW, else base-2 LSE rows; Delta: -Delta rows
   // (times pre when PRE); both written by the dQ kernel, which runs first
+  constexpr bool ROW = FORM != kBwdPlain, PRE = FORM == kBwdPre;
   constexpr int kAhead = 3;                    // operands read ahead (255 VGPRs at head_dim 128)
   constexpr int KS = D / 16;                   // k-steps of the contractions over d
   constexpr int DT = D >= 32 ? D / 32 : 1;     // 32-row tiles of dK^T / dV^T
@@ -239,7 +240,7 @@ __global__ __launch_bounds__(256, D <= 32 ? 4 : D == 64 ? 3 : PRE ? 2 : 1) void 
                              !tile_all_visible(g, qw0, qw0 + 31, k_w, kv_hi_wave);
       // register r of lane (hi, col): q row qw0 + acc32_row(r, hi), kv row k_w + col.
       // The accumulators start at the row terms of their q rows: dP at -Delta, so
-      // that it ends as dP - Delta (times pre when PRE), and with PRE S at
+      // that it ends as dP - Delta (times pre when PRE), and with ROW S at
       // -LSE / scale, so that P = exp2(S scale log2 e).
       floatx16 s, dp;
       const float* rd = &sdlt[buf][32 * qh + 4 * hi];
@@ -247,8 +248,8 @@ __global__ __launch_bounds__(256, D <= 32 ? 4 : D == 64 ? 3 : PRE ? 2 : 1) void 
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const float4 l = *(const float4*)(rl + 8 * q), v = *(const float4*)(rd + 8 * q);
-        s[4 * q] = PRE ? l.x : 0.f, s[4 * q + 1] = PRE ? l.y : 0.f;
-        s[4 * q + 2] = PRE ? l.z : 0.f, s[4 * q + 3] = PRE ? l.w : 0.f;
+        s[4 * q] = ROW ? l.x : 0.f, s[4 * q + 1] = ROW ? l.y : 0.f;
+        s[4 * q + 2] = ROW ? l.z : 0.f, s[4 * q + 3] = ROW ? l.w : 0.f;
         dp[4 * q] = v.x, dp[4 * q + 1] = v.y, dp[4 * q + 2] = v.z, dp[4 * q + 3] = v.w;
       }
       // S and dP in turn, each operand read kAhead products ahead (the order is
@@ -264,11 +265,11 @@ __global__ __launch_bounds__(256, D <= 32 ? 4 : D == 64 ? 3 : PRE ? 2 : 1) void 
         if (i + kAhead < 2 * KS) op[i % kAhead] = row_op(i + kAhead);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if constexpr (PRE) {
+      if constexpr (ROW) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           s[r] = __builtin_amdgcn_exp2f(s[r] * g.scale_log2);
-          dp[r] *= s[r];
+          dp[r] = PRE ? s[r] * dp[r] : s[r] * (dp[r] * g.scale);
         }
       } else {
 #pragma unroll
@@ -377,7 +378,7 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ dO, uint16_t* __restrict__ dK,
     uint16_t* __restrict__ dV, const float* __restrict__ LSE2, const float* __restrict__ Delta,
     const int32_t* __restrict__ col_ptr, const int32_t* __restrict__ col_idx, KvWork w) {
-  // LSE2: base-2 LSE rows; Delta: -Delta rows (times the scale when PRE),
+  // LSE2: base-2 LSE rows; Delta: -Delta rows (times pre when PRE),
   // both written by the dQ kernel, which runs first
   constexpr int D = 64, KS = 2, DT = 4;
   __shared__ __align__(16) uint16_t sq[2][64 * D];
@@ -821,13 +822,14 @@ __global__ __launch_bounds__(256, D >= 128 || (D == 64 && KB == 1) ? 1 : 2) void
 // halves' fp32 sums meet once, through LDS, at the end (the kh = 0 wave adds
 // the kh = 1 wave's, a fixed order).
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool PRE>
-__global__ __launch_bounds__(256, D > 64 ? 2 : D == 64 ? 3 : 4) void dq_kernel_16(
+template <typename T, int D, int FORM>
+__global__ __launch_bounds__(256, D > 64 ? 2 : 4) void dq_kernel_16(
     Geom g, const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO,
     uint16_t* __restrict__ dQ, const float* __restrict__ LSE, float* __restrict__ Delta,
     const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ row_idx, int n_qt,
     const int32_t* __restrict__ dq_order) {
+  constexpr bool ROW = FORM != kBwdPlain, PRE = FORM == kBwdPre;
   constexpr int kAhead = 4;                    // operands read ahead
   constexpr int KS = D / 16;
   constexpr int DT = D >= 32 ? D / 32 : 1;
@@ -871,10 +873,10 @@ __global__ __launch_bounds__(256, D > 64 ? 2 : D == 64 ? 3 : 4) void dq_kernel_1
         for (int i = 0; i < 8; ++i) part += T::to_float(ho[i]) * T::to_float(hd[i]);
       }
     }
-    // the row's start of S: -LSE / scale with PRE, else (added after) the LSE in
+    // the row's start of S: -LSE / scale with ROW, else (added after) the LSE in
     // base 2; one rounding, once per row
     const float lse = ok ? LSE[(size_t)bh * g.n_q + my_q] : 0.f;
-    lse2 = PRE ? (float)(-(double)lse / (double)g.scale) : lse_base2(lse);
+    lse2 = ROW ? (float)(-(double)lse / (double)g.scale) : lse_base2(lse);
     // Stored negated: both kernels start their dP accumulators at -Delta, so
     // they end as dP - Delta. With PRE the dO operand and -Delta carry pre.
     ndlt = PRE ? -half_sum(part) * g.pre : -half_sum(part);
@@ -914,7 +916,7 @@ __global__ __launch_bounds__(256, D > 64 ? 2 : D == 64 ? 3 : 4) void dq_kernel_1
     if (!tile_unseen(g, q0w, q0w + 31, kw0, 32)) {
       const bool need_mask = partial || (q0w + 31 >= g.n_q) || (kw0 + 32 > g.n_kv) ||
                              !tile_all_visible(g, q0w, q0w + 31, kw0, kw0 + 31);
-      floatx16 s = splat16(PRE ? lse2 : 0.f), dp = splat16(ndlt);
+      floatx16 s = splat16(ROW ? lse2 : 0.f), dp = splat16(ndlt);
       // operands read kAhead products ahead, in a pinned order (as in dK/dV)
       auto row_op = [&](int i) { return at.rows(i & 1 ? cv : ck, kh, i >> 1); };
       uint4 op[kAhead];
@@ -929,7 +931,7 @@ __global__ __launch_bounds__(256, D > 64 ? 2 : D == 64 ? 3 : 4) void dq_kernel_1
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float p = __builtin_amdgcn_exp2f(PRE ? s[r] * g.scale_log2 : __builtin_fmaf(s[r], g.scale_log2, -lse2));
+        const float p = __builtin_amdgcn_exp2f(ROW ? s[r] * g.scale_log2 : __builtin_fmaf(s[r], g.scale_log2, -lse2));
         dp[r] = PRE ? p * dp[r] : p * (dp[r] * g.scale);
       }
       if (need_mask) {     // masked elements: dS = 0 (bit select, as in the dK/dV kernel)
@@ -1344,7 +1346,7 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : 2) void dq_
 
 // dQ first: it also produces -Delta and the base-2 LSE rows, which dK/dV reads
 // from the two halves of the row-term workspace
-template <typename T, int D, bool PRE>
+template <typename T, int D, int FORM>
 void launch_bwd16_as(const Geom& g, const void* q, const void* k, const void* v, const void* o,
                      const void* dout, const float* lse, void* dq, void* dk, void* dv, float* delta,
                      const int32_t* row_ptr, const int32_t* row_idx, int n_qt, const int32_t* dq_order,
@@ -1352,6 +1354,7 @@ void launch_bwd16_as(const Geom& g, const void* q, const void* k, const void* v,
   const int BH = g.B * g.H, BHkv = g.B * g.H_kv;
   const float* lse2 = delta + (size_t)BH * g.n_q;
   if constexpr (D == 64) {
+    constexpr bool PRE = FORM == kBwdPre;
     hipLaunchKernelGGL((dq_kernel_q64<T, PRE>), dim3(n_qt * BH), dim3(256), 0, stream, g,
                        (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)o,
                        (const uint16_t*)dout, (uint16_t*)dq, lse, delta, row_ptr, row_idx, n_qt, dq_order);
@@ -1359,10 +1362,10 @@ void launch_bwd16_as(const Geom& g, const void* q, const void* k, const void* v,
                        (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)dout,
                        (uint16_t*)dk, (uint16_t*)dv, lse2, delta, col_ptr, col_idx, w);
   } else {
-    hipLaunchKernelGGL((dq_kernel_16<T, D, PRE>), dim3(n_qt * BH), dim3(256), 0, stream, g,
+    hipLaunchKernelGGL((dq_kernel_16<T, D, FORM>), dim3(n_qt * BH), dim3(256), 0, stream, g,
                        (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)o,
                        (const uint16_t*)dout, (uint16_t*)dq, lse, delta, row_ptr, row_idx, n_qt, dq_order);
-    hipLaunchKernelGGL((dkdv_kernel_16<T, D, PRE>), dim3(w.n_items * BHkv), dim3(256), 0, stream, g,
+    hipLaunchKernelGGL((dkdv_kernel_16<T, D, FORM>), dim3(w.n_items * BHkv), dim3(256), 0, stream, g,
                        (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)dout,
                        (uint16_t*)dk, (uint16_t*)dv, lse2, delta, col_ptr, col_idx, w);
   }
@@ -1373,12 +1376,14 @@ void launch_bwd16(const Geom& g, const void* q, const void* k, const void* v, co
                   const void* dout, const float* lse, void* dq, void* dk, void* dv, float* delta,
                   const int32_t* row_ptr, const int32_t* row_idx, int n_qt, const int32_t* dq_order,
                   const int32_t* col_ptr, const int32_t* col_idx, const KvWork& w, hipStream_t stream) {
-  if (g.prescale)
-    launch_bwd16_as<T, D, true>(g, q, k, v, o, dout, lse, dq, dk, dv, delta, row_ptr, row_idx, n_qt,
-                                dq_order, col_ptr, col_idx, w, stream);
-  else
-    launch_bwd16_as<T, D, false>(g, q, k, v, o, dout, lse, dq, dk, dv, delta, row_ptr, row_idx, n_qt,
-                                 dq_order, col_ptr, col_idx, w, stream);
+#define GKI_BWD16(FORM)                                                                             \
+  launch_bwd16_as<T, D, FORM>(g, q, k, v, o, dout, lse, dq, dk, dv, delta, row_ptr, row_idx, n_qt,  \
+                              dq_order, col_ptr, col_idx, w, stream)
+  // head_dim 64 forms P by an fma of the base-2 LSE, so its first two forms are one
+  if (g.bwd_form == kBwdPre) GKI_BWD16(kBwdPre);
+  else if (g.bwd_form == kBwdRow && D != 64) GKI_BWD16((D != 64 ? kBwdRow : kBwdPlain));
+  else GKI_BWD16(kBwdPlain);
+#undef GKI_BWD16
 }
 
 template <int D>

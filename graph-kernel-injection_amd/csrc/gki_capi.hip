@@ -74,7 +74,7 @@ void set_scale(Geom& g, float scale) {
   g.q_and = scale == 0.f ? 0u : 0xFFFFFFFFu;
   g.q_xor = scale < 0.f ? 0x80008000u : 0u;
   g.qk_scale_log2 = scale == 0.f ? kLog2e : (scale < 0.f ? -scale : scale) * kLog2e;
-  g.prescale = 0;   // reference order; make_geom sets it where exact
+  g.bwd_form = kBwdPlain;   // make_geom sets it
   g.pre = g.post = 1.f;
 }
 
@@ -106,17 +106,8 @@ int make_geom(Geom& g, int dtype, int B, int H, int H_kv, int n_q, int n_kv, int
   g.n_kv = n_kv;
   g.q_off = n_kv - n_q;
   set_scale(g, scale);
-  // 16-bit backward: the power-of-two part of a positive scale moves into
-  // the dP operand (exact products; see Geom::prescale), over the range
-  // where it keeps the operand's elements normal in its type
-  int e2 = 0;
-  std::frexp(scale, &e2);                        // scale in [2^(e2-1), 2^e2)
-  const int e_lo = dtype == kF16 ? -3 : -29, e_hi = dtype == kF16 ? 1 : 30;
-  g.prescale = dtype != kF32 && scale > 0.f && e2 >= e_lo && e2 <= e_hi;
-  if (g.prescale) {
-    g.pre = std::ldexp(1.f, e2 - 1);
-    g.post = scale / g.pre;                      // exact: a power of two
-  }
+  g.bwd_form = bwd_form_of(dtype, scale, g.pre);
+  if (g.bwd_form == kBwdPre) g.post = scale / g.pre;   // exact: a power of two
   g.causal = causal ? 1 : 0;
   g.sink = sink;
   g.window = window;

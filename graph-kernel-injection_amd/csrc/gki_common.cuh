@@ -7,6 +7,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
+
 #include <string>
 
 namespace gki {
@@ -485,6 +487,28 @@ __device__ inline int rho(int t, int j) {
 }
 
 // Geometry + masking parameters shared by all attention kernels.
+// Forms of the 16-bit backward (Geom::bwd_form).
+enum BwdForm : int { kBwdPlain = 0, kBwdRow = 1, kBwdPre = 2 };
+
+// The form a scale takes, and its power of two. An operand times `pre` must
+// keep its bits. fp16 has five exponent bits and gradients of 1e-3 .. 1e-5 are
+// ordinary (training without loss scaling), dS of a long row smaller still: only
+// scales that are powers of two take kBwdPre (head_dim 16 and 64; dS is then cast
+// as it is), down to 2^-4. For any other scale a dO of 1e-4 lost up to 2.9 times
+// the accuracy in dQ with the operand scaled by 2^-4 and dS cast as dS / post.
+// bf16 has the exponents of fp32: 2^-10 costs bits below 1.2e-35 only, and dS /
+// post rounds as dS.
+__host__ inline int bwd_form_of(int dtype, float scale, float& pre) {
+  pre = 1.f;
+  int e2 = 0;
+  const float mant = std::frexp(scale, &e2);           // |scale| in [2^(e2-1), 2^e2)
+  if (dtype == kF32 || mant == 0.f || e2 < -29 || e2 > 30) return kBwdPlain;
+  const bool two = mant == 0.5f || mant == -0.5f;
+  if (dtype == kBF16 ? e2 < -9 || e2 > 1 : !two || e2 < -3 || e2 > 1) return kBwdRow;
+  pre = std::ldexp(mant < 0.f ? -1.f : 1.f, e2 - 1);
+  return kBwdPre;
+}
+
 struct Geom {
   int B, H;
   int H_kv, group;    // K/V heads and q heads per K/V head (grouped-query attention; 1 = MHA)
@@ -500,17 +524,18 @@ struct Geom {
   float qk_scale_log2;
   uint32_t q_and, q_xor;
   // 16-bit backward: dS = P (dP - Delta) scale, cast to 16 bits before the
-  // dK / dQ products. For a scale in [2^-4, 2) (bf16: [2^-30, 2^30)) the kernels
-  // multiply the V (dK/dV) or dO (dQ) operand and -Delta by `pre`, the power of
-  // two at or below it, once: every product and partial sum of the dP accumulator is then
-  // the same value times a power of two (exact in fp32), so it ends as
-  // (dP - Delta) pre and dS / post costs one multiply; the rest of the scale,
-  // post = scale / pre in [1, 2) (1 at head_dim 64, sqrt 2 at 128), multiplies
-  // the fp32 dK / dQ sums once (prescale = 1). dS / post rounds to 16 bits with
-  // the relative error of dS. Only a 16-bit operand that `pre` takes below the
-  // smallest normal rounds (by at most half its subnormal spacing, 2^-25 for
-  // fp16). Otherwise prescale = 0: the scaled dS is cast, pre = post = 1.
-  int prescale;
+  // dK / dQ products (bwd_form):
+  //  kBwdPre   the kernels multiply the V (dK/dV) or dO (dQ) operand and -Delta
+  //    by `pre`, a power of two, once: every product and partial sum of the dP
+  //    accumulator is the same value times it (exact in fp32), so it ends as
+  //    (dP - Delta) pre and dS / post costs one multiply; post = scale / pre (1, or
+  //    in (1, 2) for bf16) multiplies the fp32 dK / dQ sums once. Only a 16-bit
+  //    operand that `pre` takes below the smallest normal rounds.
+  //  kBwdRow   the scaled dS is formed and cast as in the reference; the row
+  //    terms still start the accumulators (-LSE / scale, -Delta).
+  //  kBwdPlain for scales that cannot divide the LSE (0, |scale| outside
+  //    [2^-30, 2^30)): as kBwdRow with the LSE subtracted in the exponent.
+  int bwd_form;
   float pre, post;
   int causal, sink, window;
   // original block mask (used only for tiles flagged partial)

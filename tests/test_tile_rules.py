@@ -1,4 +1,5 @@
-"""The rule by which a wave leaves a kv tile out (CPU).
+"""The kernels' rules on the CPU: the tiles a wave leaves out, the form of the
+16-bit backward that a scale takes.
 
 `tile_unseen` (graph-kernel-injection_amd/csrc/gki_common.cuh) must never hold
 for a tile of which some row sees a key under the oracle's token rule, and
@@ -7,6 +8,7 @@ holds whenever no in-range row sees one (else work would be done for nothing).
 
 from __future__ import annotations
 
+import math
 import os
 import shutil
 import subprocess
@@ -34,6 +36,38 @@ def rules_exe(tmp_path_factory):
     return exe
 
 
+def _run(exe, what, lines):
+    return subprocess.run([exe, what], input="\n".join(lines) + "\n", capture_output=True, text=True, check=True,
+                          timeout=120).stdout.split()
+
+
+PLAIN, ROW, PRE = 0, 1, 2
+FP32, FP16, BF16 = 0, 1, 2
+
+
+def test_the_backward_scales_an_operand_only_where_its_type_has_the_bits(rules_exe):
+    """fp16 (five exponent bits): only by the exact powers of two 2^-4 .. 1 that
+    leave no remainder for dS; bf16: by the power of two at or below |scale| in
+    [2^-10, 2). Elsewhere dS is scaled in fp32."""
+    scales = [0.0] + [s * m * 2.0**e for e in range(-40, 40) for m in (1.0, math.sqrt(2), 1.999) for s in (1, -1)]
+    for dtype in (FP32, FP16, BF16):
+        out = _run(rules_exe, "form", [f"{dtype} {s!r}" for s in scales])
+        for s, form, pre in zip(scales, map(int, out[::2]), map(float.fromhex, out[1::2])):
+            mag = abs(np.float32(s))
+            two = mag > 0 and math.frexp(mag)[0] == 0.5
+            if dtype == FP32 or mag == 0 or not 2.0**-30 <= mag < 2.0**30:
+                want = PLAIN
+            elif dtype == FP16:
+                want = PRE if two and 2.0**-4 <= mag <= 1 else ROW
+            else:
+                want = PRE if 2.0**-10 <= mag < 2 else ROW
+            assert form == want, (dtype, s, form)
+            if form == PRE:
+                assert math.frexp(abs(pre))[0] == 0.5 and 1 <= s / pre < 2 and (dtype == BF16 or s == pre)
+            else:
+                assert pre == 1
+
+
 def test_unseen_tiles_are_exactly_those_without_a_visible_key(rules_exe):
     rng = np.random.default_rng(5)
     lines, want = [], []
@@ -48,8 +82,7 @@ def test_unseen_tiles_are_exactly_those_without_a_visible_key(rules_exe):
             for k0, n_k in [(k, n) for n in (TILE, TILE // 2) for k in range(0, n_kv, n)]:
                 lines.append(f"{n_q} {n_kv} {int(causal)} {sink} {window} {q_lo} {q_lo + 31} {k0} {n_k}")
                 want.append((not causal, bool(vis[q_lo:q_lo + 32, k0:k0 + n_k].any()), q_lo + 32 <= n_q))
-    out = subprocess.run([rules_exe], input="\n".join(lines) + "\n", capture_output=True, text=True, check=True,
-                         timeout=120).stdout.split()
+    out = _run(rules_exe, "unseen", lines)
     assert len(out) == len(want)
     skipped = 0
     for line, got, (never, seen, whole) in zip(lines, out, want):

@@ -1,19 +1,32 @@
-// Host driver for tests/test_tile_rules.py: the kernels' tile rules
-// (gki_common.cuh) on the CPU.
+// Host driver for the CPU tests of the kernels' rules (gki_common.cuh).
 //
-// stdin lines: n_q n_kv causal sink window q_lo q_hi k0 n_k
-// stdout: tile_unseen, per line.
+// argv[1] "unseen": stdin lines n_q n_kv causal sink window q_lo q_hi k0 n_k,
+//   stdout tile_unseen per line;
+// "form": lines dtype scale, stdout bwd_form_of and its power of two.
 #include <cstdio>
+#include <cstring>
 
 #include "gki_common.cuh"
 
-int main() {
-  gki::Geom g{};
-  int q_lo, q_hi, k0, n_k;
-  while (std::scanf("%d %d %d %d %d %d %d %d %d", &g.n_q, &g.n_kv, &g.causal, &g.sink, &g.window, &q_lo, &q_hi,
-                    &k0, &n_k) == 9) {
-    g.q_off = g.n_kv - g.n_q;
-    std::printf("%d\n", (int)gki::tile_unseen(g, q_lo, q_hi, k0, n_k));
+int main(int argc, char** argv) {
+  const char* what = argc > 1 ? argv[1] : "";
+  if (!std::strcmp(what, "unseen")) {
+    gki::Geom g{};
+    int q_lo, q_hi, k0, n_k;
+    while (std::scanf("%d %d %d %d %d %d %d %d %d", &g.n_q, &g.n_kv, &g.causal, &g.sink, &g.window, &q_lo, &q_hi,
+                      &k0, &n_k) == 9) {
+      g.q_off = g.n_kv - g.n_q;
+      std::printf("%d\n", (int)gki::tile_unseen(g, q_lo, q_hi, k0, n_k));
+    }
+  } else if (!std::strcmp(what, "form")) {
+    int dtype;
+    float scale, pre;
+    while (std::scanf("%d %f", &dtype, &scale) == 2) {
+      const int form = gki::bwd_form_of(dtype, scale, pre);
+      std::printf("%d %a\n", form, pre);
+    }
+  } else {
+    return 1;
   }
   return 0;
 }
