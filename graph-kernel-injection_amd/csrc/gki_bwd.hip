@@ -47,6 +47,10 @@ __device__ inline void two_sum_fold(floatx4& sum, floatx4& comp, const floatx4& 
   }
 }
 
+__device__ inline uint4 and4(const uint4& v, uint32_t m) {
+  return make_uint4(v.x & m, v.y & m, v.z & m, v.w & m);
+}
+
 // Work item of workgroup b in the dK / dV grid: the items of one (b, kv head)
 // are consecutive, XCD-remapped so that neighbouring kv tiles of a head (which
 // share most q tiles) run on one XCD and meet in its L2.
@@ -148,7 +152,7 @@ __global__ __launch_bounds__(256, D <= 32 ? 4 : FORM != kBwdPlain ? 2 : 1) void 
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ dO, uint16_t* __restrict__ dK,
     uint16_t* __restrict__ dV, const float* __restrict__ LSE2, const float* __restrict__ Delta,
     const int32_t* __restrict__ col_ptr, const int32_t* __restrict__ col_idx, KvWork w) {
-  // LSE2: -LSE / scale rows when ROW, else base-2 LSE rows; Delta: -Delta rows
+  // LSE2: -LSE / row_scale rows when ROW, else base-2 LSE rows; Delta: -Delta rows
   // (times pre when PRE); both written by the dQ kernel, which runs first
   constexpr bool ROW = FORM != kBwdPlain, PRE = FORM == kBwdPre;
   constexpr int kAhead = 3;                    // operands read ahead (255 VGPRs at head_dim 128)
@@ -186,6 +190,7 @@ __global__ __launch_bounds__(256, D <= 32 ? 4 : FORM != kBwdPlain ? 2 : 1) void 
       const size_t o = kb + (size_t)my_kv * D + 16 * ks + 8 * hi;
       kf[ks] = ok ? *(const uint4*)(K + o) : make_uint4(0, 0, 0, 0);
       vf[ks] = ok ? *(const uint4*)(V + o) : make_uint4(0, 0, 0, 0);
+      if constexpr (FORM == kBwdRow) kf[ks] = and4(kf[ks], g.q_and);
       if constexpr (PRE) vf[ks] = scale8<T>(vf[ks], g.pre);
     }
   }
@@ -268,7 +273,7 @@ __global__ __launch_bounds__(256, D <= 32 ? 4 : FORM != kBwdPlain ? 2 : 1) void 
       if constexpr (ROW) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          s[r] = __builtin_amdgcn_exp2f(s[r] * g.scale_log2);
+          s[r] = __builtin_amdgcn_exp2f(s[r] * g.row_scale_log2);
           dp[r] = PRE ? s[r] * dp[r] : s[r] * (dp[r] * g.scale);
         }
       } else {
@@ -873,16 +878,17 @@ __global__ __launch_bounds__(256, D > 64 ? 2 : 4) void dq_kernel_16(
         for (int i = 0; i < 8; ++i) part += T::to_float(ho[i]) * T::to_float(hd[i]);
       }
     }
-    // the row's start of S: -LSE / scale with ROW, else (added after) the LSE in
+    // the row's start of S: -LSE / row_scale with ROW, else (added after) the LSE in
     // base 2; one rounding, once per row
     const float lse = ok ? LSE[(size_t)bh * g.n_q + my_q] : 0.f;
-    lse2 = ROW ? (float)(-(double)lse / (double)g.scale) : lse_base2(lse);
+    lse2 = ROW ? (float)(-(double)lse / (double)g.row_scale) : lse_base2(lse);
     // Stored negated: both kernels start their dP accumulators at -Delta, so
     // they end as dP - Delta. With PRE the dO operand and -Delta carry pre.
     ndlt = PRE ? -half_sum(part) * g.pre : -half_sum(part);
-    if constexpr (PRE) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) df[ks] = scale8<T>(df[ks], g.pre);
+    for (int ks = 0; ks < KS; ++ks) {
+      if constexpr (FORM == kBwdRow) qf[ks] = and4(qf[ks], g.q_and);
+      if constexpr (PRE) df[ks] = scale8<T>(df[ks], g.pre);
     }
     if (ok && hi == 0 && kh == 0) {            // the two kv-half waves hold the same rows
       Delta[(size_t)bh * g.n_q + my_q] = ndlt;
@@ -931,7 +937,7 @@ __global__ __launch_bounds__(256, D > 64 ? 2 : 4) void dq_kernel_16(
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float p = __builtin_amdgcn_exp2f(ROW ? s[r] * g.scale_log2 : __builtin_fmaf(s[r], g.scale_log2, -lse2));
+        const float p = __builtin_amdgcn_exp2f(ROW ? s[r] * g.row_scale_log2 : __builtin_fmaf(s[r], g.scale_log2, -lse2));
         dp[r] = PRE ? p * dp[r] : p * (dp[r] * g.scale);
       }
       if (need_mask) {     // masked elements: dS = 0 (bit select, as in the dK/dV kernel)

@@ -76,6 +76,8 @@ void set_scale(Geom& g, float scale) {
   g.qk_scale_log2 = scale == 0.f ? kLog2e : (scale < 0.f ? -scale : scale) * kLog2e;
   g.bwd_form = kBwdPlain;   // make_geom sets it
   g.pre = g.post = 1.f;
+  g.row_scale = scale == 0.f ? 1.f : scale;
+  g.row_scale_log2 = g.row_scale * kLog2e;
 }
 
 int make_geom(Geom& g, int dtype, int B, int H, int H_kv, int n_q, int n_kv, int head_dim,

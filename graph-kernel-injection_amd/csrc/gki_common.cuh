@@ -502,7 +502,8 @@ __host__ inline int bwd_form_of(int dtype, float scale, float& pre) {
   pre = 1.f;
   int e2 = 0;
   const float mant = std::frexp(scale, &e2);           // |scale| in [2^(e2-1), 2^e2)
-  if (dtype == kF32 || mant == 0.f || e2 < -29 || e2 > 30) return kBwdPlain;
+  if (dtype != kF32 && mant == 0.f) return kBwdRow;
+  if (dtype == kF32 || e2 < -29 || e2 > 30) return kBwdPlain;
   const bool two = mant == 0.5f || mant == -0.5f;
   if (dtype == kBF16 ? e2 < -9 || e2 > 1 : !two || e2 < -3 || e2 > 1) return kBwdRow;
   pre = std::ldexp(mant < 0.f ? -1.f : 1.f, e2 - 1);
@@ -532,11 +533,12 @@ struct Geom {
   //    in (1, 2) for bf16) multiplies the fp32 dK / dQ sums once. Only a 16-bit
   //    operand that `pre` takes below the smallest normal rounds.
   //  kBwdRow   the scaled dS is formed and cast as in the reference; the row
-  //    terms still start the accumulators (-LSE / scale, -Delta).
-  //  kBwdPlain for scales that cannot divide the LSE (0, |scale| outside
+  //    terms still start the accumulators (-LSE / scale, -Delta). Scale 0: the
+  //    operand of S is zeroed (q_and) and row_scale 1 divides the LSE.
+  //  kBwdPlain for scales too small or large to divide the LSE (|scale| outside
   //    [2^-30, 2^30)): as kBwdRow with the LSE subtracted in the exponent.
   int bwd_form;
-  float pre, post;
+  float pre, post, row_scale, row_scale_log2;
   int causal, sink, window;
   // original block mask (used only for tiles flagged partial)
   const int32_t* mask;
