@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256, D <= 32 ? 4 : FORM != kBwdPlain ? 2 : 1) void 
     uint16_t* __restrict__ dV, const float* __restrict__ LSE2, const float* __restrict__ Delta,
     const int32_t* __restrict__ col_ptr, const int32_t* __restrict__ col_idx, KvWork w) {
   // LSE2: -LSE / row_scale rows when ROW, else base-2 LSE rows; Delta: -Delta rows
-  // (times pre when PRE); both written by the dQ kernel, which runs first
+  // (times the scale when PRE); both written by the dQ kernel, which runs first
   constexpr bool ROW = FORM != kBwdPlain, PRE = FORM == kBwdPre;
   constexpr int kAhead = 3;                    // operands read ahead (255 VGPRs at head_dim 128)
   constexpr int KS = D / 16;                   // k-steps of the contractions over d
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(256, D <= 32 ? 4 : FORM != kBwdPlain ? 2 : 1) void 
       kf[ks] = ok ? *(const uint4*)(K + o) : make_uint4(0, 0, 0, 0);
       vf[ks] = ok ? *(const uint4*)(V + o) : make_uint4(0, 0, 0, 0);
       if constexpr (FORM == kBwdRow) kf[ks] = and4(kf[ks], g.q_and);
-      if constexpr (PRE) vf[ks] = scale8<T>(vf[ks], g.pre);
+      if constexpr (PRE) vf[ks] = scale8<T>(vf[ks], g.scale);
     }
   }
   floatx16 dk[DT], dv[DT];
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(256, D <= 32 ? 4 : FORM != kBwdPlain ? 2 : 1) void 
                              !tile_all_visible(g, qw0, qw0 + 31, k_w, kv_hi_wave);
       // register r of lane (hi, col): q row qw0 + acc32_row(r, hi), kv row k_w + col.
       // The accumulators start at the row terms of their q rows: dP at -Delta, so
-      // that it ends as dP - Delta (times pre when PRE), and with ROW S at
+      // that it ends as dP - Delta (times the scale when PRE), and with ROW S at
       // -LSE / scale, so that P = exp2(S scale log2 e).
       floatx16 s, dp;
       const float* rd = &sdlt[buf][32 * qh + 4 * hi];
@@ -337,7 +337,6 @@ __global__ __launch_bounds__(256, D <= 32 ? 4 : FORM != kBwdPlain ? 2 : 1) void 
   }
   __syncthreads();
   if (qh == 1) return;
-  const float post = PRE ? g.post : 1.f;
   const bool split = item.pslot >= 0;          // a split column: fp32 partials for the reduce
   const int row = 32 * kh + (lane_e & 31);     // of the kv tile
   if (!split && kt * kTileN + row >= g.n_kv) return;
@@ -351,7 +350,7 @@ __global__ __launch_bounds__(256, D <= 32 ? 4 : FORM != kBwdPlain ? 2 : 1) void 
       floatx4 a, b;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        a[i] = (dk[dt][4 * q + i] + rk[i]) * post;
+        a[i] = dk[dt][4 * q + i] + rk[i];
         b[i] = dv[dt][4 * q + i] + rv[i];
       }
       const int d0 = 32 * dt + 8 * q + 4 * hi_e;
@@ -383,7 +382,7 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
     const uint16_t* __restrict__ V, const uint16_t* __restrict__ dO, uint16_t* __restrict__ dK,
     uint16_t* __restrict__ dV, const float* __restrict__ LSE2, const float* __restrict__ Delta,
     const int32_t* __restrict__ col_ptr, const int32_t* __restrict__ col_idx, KvWork w) {
-  // LSE2: base-2 LSE rows; Delta: -Delta rows (times pre when PRE),
+  // LSE2: base-2 LSE rows; Delta: -Delta rows (times the scale when PRE),
   // both written by the dQ kernel, which runs first
   constexpr int D = 64, KS = 2, DT = 4;
   __shared__ __align__(16) uint16_t sq[2][64 * D];
@@ -414,7 +413,7 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
       const bool ok = has_work && my_kv < g.n_kv;
       kf[b][ks] = ok ? *(const uint4*)(K + kb + (size_t)my_kv * D + d0) : make_uint4(0, 0, 0, 0);
       vf[b][ks] = ok ? *(const uint4*)(V + kb + (size_t)my_kv * D + d0) : make_uint4(0, 0, 0, 0);
-      if constexpr (PRE) vf[b][ks] = scale8<T>(vf[b][ks], g.pre);
+      if constexpr (PRE) vf[b][ks] = scale8<T>(vf[b][ks], g.scale);
     }
   }
   floatx4 dk[2][DT], dv[2][DT];
@@ -556,7 +555,6 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       dk[b][dt] += red[((2 * b + 0) * DT + dt) * 64 + lane];
-      if constexpr (PRE) dk[b][dt] *= g.post;
       dv[b][dt] += red[((2 * b + 1) * DT + dt) * 64 + lane];
     }
   // accumulators: lane holds kv rows k_w + 16 b + 4 grp + i, column 16 dt + col
@@ -883,12 +881,12 @@ __global__ __launch_bounds__(256, D > 64 ? 2 : 4) void dq_kernel_16(
     const float lse = ok ? LSE[(size_t)bh * g.n_q + my_q] : 0.f;
     lse2 = ROW ? (float)(-(double)lse / (double)g.row_scale) : lse_base2(lse);
     // Stored negated: both kernels start their dP accumulators at -Delta, so
-    // they end as dP - Delta. With PRE the dO operand and -Delta carry pre.
-    ndlt = PRE ? -half_sum(part) * g.pre : -half_sum(part);
+    // they end as dP - Delta. With PRE the dO operand and -Delta carry the scale.
+    ndlt = PRE ? -half_sum(part) * g.scale : -half_sum(part);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       if constexpr (FORM == kBwdRow) qf[ks] = and4(qf[ks], g.q_and);
-      if constexpr (PRE) df[ks] = scale8<T>(df[ks], g.pre);
+      if constexpr (PRE) df[ks] = scale8<T>(df[ks], g.scale);
     }
     if (ok && hi == 0 && kh == 0) {            // the two kv-half waves hold the same rows
       Delta[(size_t)bh * g.n_q + my_q] = ndlt;
@@ -974,7 +972,6 @@ __global__ __launch_bounds__(256, D > 64 ? 2 : 4) void dq_kernel_16(
   }
   __syncthreads();
   if (kh == 1) return;
-  const float post = PRE ? g.post : 1.f;
   const int my_q = q0w + (lane_e & 31);
   if (my_q >= g.n_q) return;
 #pragma unroll
@@ -984,7 +981,7 @@ __global__ __launch_bounds__(256, D > 64 ? 2 : 4) void dq_kernel_16(
       const floatx4 r = red[(dt * 4 + q) * 64 + lane_e];
       float v[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = (dq[dt][4 * q + i] + r[i]) * post;
+      for (int i = 0; i < 4; ++i) v[i] = dq[dt][4 * q + i] + r[i];
       *(uint2*)(dQ + qb + (size_t)my_q * D + 32 * dt + 8 * q + 4 * hi_e) =
           make_uint2(pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3]));
     }
@@ -1044,10 +1041,10 @@ __global__ __launch_bounds__(256, 4) void dq_kernel_q64(
     }
     lse2[b] = ok ? lse_base2(LSE[(size_t)bh * g.n_q + my_q]) : 0.f;
     // stored negated (and scaled with PRE), as in dq_kernel_16
-    ndlt[b] = PRE ? -wave_sum16x4(part) * g.pre : -wave_sum16x4(part);
+    ndlt[b] = PRE ? -wave_sum16x4(part) * g.scale : -wave_sum16x4(part);
     if constexpr (PRE) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) df[b][ks] = scale8<T>(df[b][ks], g.pre);
+      for (int ks = 0; ks < KS; ++ks) df[b][ks] = scale8<T>(df[b][ks], g.scale);
     }
     if (ok && grp == 0 && kh == 0) {     // the two kv-half waves hold the same rows
       Delta[(size_t)bh * g.n_q + my_q] = ndlt[b];
@@ -1168,8 +1165,7 @@ __global__ __launch_bounds__(256, 4) void dq_kernel_q64(
     if (my_q >= g.n_q) continue;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
-      floatx4 o = dq[b][dt] + red[(b * DT + dt) * 64 + lane_e];
-      if constexpr (PRE) o *= g.post;
+      const floatx4 o = dq[b][dt] + red[(b * DT + dt) * 64 + lane_e];
       const uint2 w = make_uint2(pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3]));
       *(uint2*)(dQ + qb + (size_t)my_q * D + 16 * dt + 4 * grp_e) = w;
     }

@@ -75,7 +75,6 @@ void set_scale(Geom& g, float scale) {
   g.q_xor = scale < 0.f ? 0x80008000u : 0u;
   g.qk_scale_log2 = scale == 0.f ? kLog2e : (scale < 0.f ? -scale : scale) * kLog2e;
   g.bwd_form = kBwdPlain;   // make_geom sets it
-  g.pre = g.post = 1.f;
   g.row_scale = scale == 0.f ? 1.f : scale;
   g.row_scale_log2 = g.row_scale * kLog2e;
 }
@@ -108,8 +107,7 @@ int make_geom(Geom& g, int dtype, int B, int H, int H_kv, int n_q, int n_kv, int
   g.n_kv = n_kv;
   g.q_off = n_kv - n_q;
   set_scale(g, scale);
-  g.bwd_form = bwd_form_of(dtype, scale, g.pre);
-  if (g.bwd_form == kBwdPre) g.post = scale / g.pre;   // exact: a power of two
+  g.bwd_form = bwd_form_of(dtype, scale);
   g.causal = causal ? 1 : 0;
   g.sink = sink;
   g.window = window;

@@ -490,24 +490,18 @@ __device__ inline int rho(int t, int j) {
 // Forms of the 16-bit backward (Geom::bwd_form).
 enum BwdForm : int { kBwdPlain = 0, kBwdRow = 1, kBwdPre = 2 };
 
-// The form a scale takes, and its power of two. An operand times `pre` must
-// keep its bits. fp16 has five exponent bits and gradients of 1e-3 .. 1e-5 are
-// ordinary (training without loss scaling), dS of a long row smaller still: only
-// scales that are powers of two take kBwdPre (head_dim 16 and 64; dS is then cast
-// as it is), down to 2^-4. For any other scale a dO of 1e-4 lost up to 2.9 times
-// the accuracy in dQ with the operand scaled by 2^-4 and dS cast as dS / post.
-// bf16 has the exponents of fp32: 2^-10 costs bits below 1.2e-35 only, and dS /
-// post rounds as dS.
-__host__ inline int bwd_form_of(int dtype, float scale, float& pre) {
-  pre = 1.f;
+// The form a scale takes: dS is cast to 16 bits after the scale, as in the
+// reference, so an operand can carry it only where it is a power of two (head_dim
+// 16 and 64 by default). Taking a power of two out of other scales (dS / post cast,
+// post in [1, 2) multiplied into the sums) saved 0-2% of a bf16 backward and cost
+// fp16 gradients accuracy: a dO of 1e-4, ordinary without loss scaling, up to 2.9
+// times in dQ, as operand and dS / post sink among the subnormal numbers.
+__host__ inline int bwd_form_of(int dtype, float scale) {
   int e2 = 0;
   const float mant = std::frexp(scale, &e2);           // |scale| in [2^(e2-1), 2^e2)
   if (dtype != kF32 && mant == 0.f) return kBwdRow;
   if (dtype == kF32 || e2 < -29 || e2 > 30) return kBwdPlain;
-  const bool two = mant == 0.5f || mant == -0.5f;
-  if (dtype == kBF16 ? e2 < -9 || e2 > 1 : !two || e2 < -3 || e2 > 1) return kBwdRow;
-  pre = std::ldexp(mant < 0.f ? -1.f : 1.f, e2 - 1);
-  return kBwdPre;
+  return (mant == 0.5f || mant == -0.5f) && e2 >= -3 && e2 <= 1 ? kBwdPre : kBwdRow;
 }
 
 struct Geom {
@@ -526,19 +520,19 @@ struct Geom {
   uint32_t q_and, q_xor;
   // 16-bit backward: dS = P (dP - Delta) scale, cast to 16 bits before the
   // dK / dQ products (bwd_form):
-  //  kBwdPre   the kernels multiply the V (dK/dV) or dO (dQ) operand and -Delta
-  //    by `pre`, a power of two, once: every product and partial sum of the dP
-  //    accumulator is the same value times it (exact in fp32), so it ends as
-  //    (dP - Delta) pre and dS / post costs one multiply; post = scale / pre (1, or
-  //    in (1, 2) for bf16) multiplies the fp32 dK / dQ sums once. Only a 16-bit
-  //    operand that `pre` takes below the smallest normal rounds.
-  //  kBwdRow   the scaled dS is formed and cast as in the reference; the row
-  //    terms still start the accumulators (-LSE / scale, -Delta). Scale 0: the
-  //    operand of S is zeroed (q_and) and row_scale 1 divides the LSE.
+  //  kBwdPre   scale +-2^-4 .. 1: the kernels multiply the V (dK/dV) or dO (dQ)
+  //    operand and -Delta by it once; every product and partial sum of the dP
+  //    accumulator is then the same value times it (exact in fp32), so it ends
+  //    as (dP - Delta) scale and dS costs one multiply. Only a 16-bit operand
+  //    that the scale takes below the smallest normal rounds (by at most half
+  //    its subnormal spacing, 2^-25 for fp16).
+  //  kBwdRow   dS is scaled per element; the row terms still start the
+  //    accumulators (-LSE / scale, -Delta). Scale 0: the operand of S is zeroed
+  //    (q_and) and row_scale 1 divides the LSE.
   //  kBwdPlain for scales too small or large to divide the LSE (|scale| outside
   //    [2^-30, 2^30)): as kBwdRow with the LSE subtracted in the exponent.
   int bwd_form;
-  float pre, post, row_scale, row_scale_log2;
+  float row_scale, row_scale_log2;
   int causal, sink, window;
   // original block mask (used only for tiles flagged partial)
   const int32_t* mask;

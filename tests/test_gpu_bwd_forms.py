@@ -33,8 +33,8 @@ def _gradients64(q, k, v, do, vis, scale, o=None, cast=None):
 @pytest.mark.parametrize("scale", [0.0, -0.3, 0.3, 3.0, 0.25, -0.125, 1 / 128, 1e-3, 1e-12])
 def test_every_form_and_head_dim_matches_64_bits(scale, D, dtype):
     """Each scale class at each head dim, on ragged tiles and rows that see nothing
-    (more queries than keys): no further from 64 bits than 1.2 times the reference's
-    rounding (dS / post rounds elsewhere than dS), plus 2^-14 for the order of sums."""
+    (more queries than keys): no further from 64 bits than the reference's
+    rounding puts them, 2% and 2^-14 left for the order of sums."""
     print(f"[case] scale {scale} D{D} {dtype}", flush=True)
     B, H, n_q, n_kv, S, W = 1, 2, 300, 270, 4, 64
     gen = torch.Generator().manual_seed(D + 1)
@@ -53,7 +53,7 @@ def test_every_form_and_head_dim_matches_64_bits(scale, D, dtype):
             continue
         err, bar = (float((x - want).norm() / want.norm()) for x in (got, ref))
         print(f"  {name} {err:.3e} (the reference's rounding {bar:.3e})", flush=True)
-        assert err <= 1.2 * bar + 2.0**-14, (name, err, bar)
+        assert err <= 1.02 * bar + 2.0**-14, (name, err, bar)
 
 
 @pytest.mark.parametrize("D,scale", [(32, None), (128, None), (16, 0.2), (64, 0.1)])

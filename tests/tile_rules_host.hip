@@ -2,7 +2,7 @@
 //
 // argv[1] "unseen": stdin lines n_q n_kv causal sink window q_lo q_hi k0 n_k,
 //   stdout tile_unseen per line;
-// "form": lines dtype scale, stdout bwd_form_of and its power of two.
+// "form": lines dtype scale, stdout bwd_form_of.
 #include <cstdio>
 #include <cstring>
 
@@ -20,11 +20,8 @@ int main(int argc, char** argv) {
     }
   } else if (!std::strcmp(what, "form")) {
     int dtype;
-    float scale, pre;
-    while (std::scanf("%d %f", &dtype, &scale) == 2) {
-      const int form = gki::bwd_form_of(dtype, scale, pre);
-      std::printf("%d %a\n", form, pre);
-    }
+    float scale;
+    while (std::scanf("%d %f", &dtype, &scale) == 2) std::printf("%d\n", gki::bwd_form_of(dtype, scale));
   } else {
     return 1;
   }
