@@ -1,0 +1,48 @@
+"""How fp32 sums are held (GPU): inputs built so that a plain sum over more rows
+than it should span, or a chain of too many terms, loses a part that shows."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import sparse_triton_kernel as stk
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+D = 64
+H = 600      # grids past those whose tiles are shared among workgroups
+
+
+def _zeros():
+    return torch.zeros(1, H, 64, D, device=DEV)
+
+
+def _grads(q, k, v, do, **kw):
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+    out = stk.block_sparse_attention(*leaves, torch.ones(1, 1, dtype=torch.int32, device=DEV), **kw)
+    return out, torch.autograd.grad(out, leaves, do)
+
+
+def test_dv_folds_every_16_rows():
+    """q = 0: P = 1/64 everywhere. Column 0 of dV sums 1.5 (row 0) and 16 x 2^-27 (rows
+    16 .. 31), column 1 the 1.5 alone: 2^-23 apart, one unit, when those 16 rows are
+    summed apart from the first, and equal when four of them (2^-25) at a time are
+    added to it."""
+    q, k, v, do = (_zeros() for _ in range(4))
+    do[..., 0, :2] = 1.5 * 64
+    do[..., 16:32, 0] = 64 * 2.0**-27
+    dv = _grads(q, k, v, do)[1][2]
+    assert ((dv[..., 0] - dv[..., 1]) >= 2.0**-23).all()
+
+
+def test_dq_folds_every_16_keys():
+    """The same over keys: P = 1/64, dP alternates +-512 (Delta = 0), dS = +-1."""
+    q, k, v, do = (_zeros() for _ in range(4))
+    sign = 1.0 - 2.0 * (torch.arange(64, device=DEV) % 2)
+    v[..., 0] = sign
+    do[..., 0] = 512.0                       # times V, P and the scale 1/8: dS = +-1
+    k[..., 0, :2] = 1.5
+    k[..., 16:32, 0] = sign[16:32] * 2.0**-27
+    dq = _grads(q, k, v, do)[1][0]
+    assert ((dq[..., 0] - dq[..., 1]) >= 2.0**-23).all()
