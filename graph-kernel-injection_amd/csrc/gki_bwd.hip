@@ -1218,7 +1218,7 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : 2) void dq_
   const int my_q = q0 + col;
 
   floatx4 qf[DJ], df[DJ];
-  float dlt = 0.f;
+  float part_d[DJ];
 #pragma unroll
   for (int j = 0; j < DJ; ++j) {
     const bool ok = my_q < g.n_q;
@@ -1226,10 +1226,15 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : 2) void dq_
     qf[j] = ok ? *(const floatx4*)(Q + at) : floatx4{0.f, 0.f, 0.f, 0.f};
     df[j] = ok ? *(const floatx4*)(dO + at) : floatx4{0.f, 0.f, 0.f, 0.f};
     const floatx4 ov = ok ? *(const floatx4*)(O + at) : floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dlt = __builtin_fmaf(ov[i], df[j][i], dlt);
+    part_d[j] = __builtin_fmaf(ov[3], df[j][3], __builtin_fmaf(ov[2], df[j][2],
+                               __builtin_fmaf(ov[1], df[j][1], ov[0] * df[j][0])));
   }
-  dlt = wave_sum16x4(dlt);
+  // pairwise: the rounding of one chain of D / 4 terms showed in dP - Delta
+#pragma unroll
+  for (int n = DJ / 2; n > 0; n /= 2)
+#pragma unroll
+    for (int j = 0; j < n; ++j) part_d[j] += part_d[j + n];
+  const float dlt = wave_sum16x4(part_d[0]);
   const float lse = my_q < g.n_q ? LSE[(size_t)bh * g.n_q + my_q] : 0.f;   // natural
   if (my_q < g.n_q && grp == 0 && share == 0) Delta[(size_t)bh * g.n_q + my_q] = dlt;
   floatx4 dq[DV][DE], cq[DV][DE];      // running sum and its compensation (two_sum_fold)

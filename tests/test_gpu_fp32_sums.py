@@ -46,3 +46,23 @@ def test_dq_folds_every_16_keys():
     k[..., 16:32, 0] = sign[16:32] * 2.0**-27
     dq = _grads(q, k, v, do)[1][0]
     assert ((dq[..., 0] - dq[..., 1]) >= 2.0**-23).all()
+
+
+def test_delta_is_summed_pairwise():
+    """Window 1: P = 1, O = V, so dP - Delta is 0 but for rounding, and dQ (K = 1 in
+    column 0) shows it. The products of a row: 1, then 25 of 2^-25, which a chain
+    from the 1 on loses one by one (25 x 2^-25 in Delta, against at most six
+    roundings of 2^-24 in the two sums where each is a tree over terms that are
+    exact). The small ones sit where the accumulators of dP keep them apart from the 1."""
+    n, d = 64, 128
+    q, k, v, do = (torch.zeros(1, 8, n, d, device=DEV) for _ in range(4))
+    small = [16 * j + i for j in range(1, 8) for i in range(4) if (4 * j + i) % 8]
+    assert len(small) == 25
+    v[..., 0], do[..., 0], k[..., 0] = 1.0, 1.0, 1.0
+    v[..., small], do[..., small] = 2.0**-13, 2.0**-12
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+    out = stk.block_sparse_attention(*leaves, torch.ones(1, 1, dtype=torch.int32, device=DEV), softmax_scale=1.0,
+                                     is_causal=True, sink_size=0, window_size=1)
+    assert torch.equal(out, v)
+    dq = torch.autograd.grad(out, leaves, do)[0]
+    assert float(dq.abs().max()) <= 6 * 2.0**-24
