@@ -586,7 +586,9 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : D * (QB == 
   for (int v = 0; v < DV; ++v)
 #pragma unroll
     for (int e = 0; e < DE; ++e) o[v][e] = floatx4{0.f, 0.f, 0.f, 0.f};
-  float m = kNegInf, l = 0.f;
+  // the row sum with its rounding error kept apart: an addition per 32 keys left
+  // the LSE of a 1024-key row 9% above one rounding (8% per 64 keys, now 6%)
+  float m = kNegInf, l = 0.f, lc = 0.f;
 
   const int e_beg = row_ptr[qt], n_step = (row_ptr[qt + 1] - e_beg) * HALVES;
   DmaTileF32<D, TR> dma;
@@ -650,6 +652,7 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : D * (QB == 
       const float alpha = m_new == kNegInf ? 1.f : __builtin_amdgcn_exp2f((m - m_new) * kLog2e);
       m = m_new;
       l *= alpha;
+      lc *= alpha;
 #pragma unroll
       for (int v = 0; v < DV; ++v)
 #pragma unroll
@@ -671,7 +674,9 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : D * (QB == 
     float rs = 0.f;
 #pragma unroll
     for (int t = 0; t < SUBS; ++t) rs += (p[t][0] + p[t][1]) + (p[t][2] + p[t][3]);
-    l += rs;
+    const float l_new = l + rs;
+    lc += rs - (l_new - l);
+    l = l_new;
 #pragma unroll
     for (int t = 0; t < SUBS; ++t)
 #pragma unroll
@@ -688,14 +693,17 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : D * (QB == 
     __syncthreads();
   }
 
-  l = wave_sum16x4(l);
+  l = wave_sum16x4(l + lc);
+  double l_tot = l;
   if constexpr (KB > 1) {
     // shares 1 .. KB - 1 hand (o, m, l) over through LDS (free: every wave
-    // passed the last barrier); share 0 merges them in order
-    float* red = sk[0];
+    // passed the last barrier); share 0 merges them in order, by one factor each
+    static_assert((KB - 1) * QB * (D + 2) * 16 <= 2 * TR * D, "the shares' sums fit one staging array");
+    float* red = &sk[0][0];
     const int blk = wave % QB;
+    auto part_of = [&](int w) { return red + ((size_t)(w - 1) * QB + blk) * (D + 2) * 16; };
     if (share > 0) {
-      float* dst = red + ((size_t)(share - 1) * QB + blk) * (D + 2) * 16 + lane;
+      float* dst = part_of(share) + lane;
 #pragma unroll
       for (int v = 0; v < DV; ++v)
 #pragma unroll
@@ -709,23 +717,34 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : D * (QB == 
     }
     __syncthreads();
     if (share > 0) return;
+    float f[KB];
+    const float m_own = m;
 #pragma unroll
-    for (int w = 1; w < KB; ++w) {
-      const float* src = red + ((size_t)(w - 1) * QB + blk) * (D + 2) * 16;
-      const float mw = src[16 * D + col], lw = src[16 * D + 16 + col];
-      const float m_new = fmaxf(m, mw), m_use = m_new == kNegInf ? 0.f : m_new;
-      const float fa = __builtin_amdgcn_exp2f((m - m_use) * kLog2e);
-      const float fb = __builtin_amdgcn_exp2f((mw - m_use) * kLog2e);
-      l = l * fa + lw * fb;
-      m = m_new;
+    for (int w = 1; w < KB; ++w) m = fmaxf(m, part_of(w)[16 * D + col]);
+    const float m_use = m == kNegInf ? 0.f : m;
+    f[0] = __builtin_amdgcn_exp2f((m_own - m_use) * kLog2e);
 #pragma unroll
-      for (int v = 0; v < DV; ++v)
+    for (int w = 1; w < KB; ++w) f[w] = __builtin_amdgcn_exp2f((part_of(w)[16 * D + col] - m_use) * kLog2e);
+    // the row sum in 64 bits, a lane group per share: 32-bit factors would round it
+    // by as much as the stored LSE is rounded
+    const int ws = grp % KB;
+    const float* of = part_of(ws ? ws : 1) + 16 * D + col;
+    l_tot = (double)(ws ? of[16] : l) * exp((double)(ws ? of[0] : m_own) - (double)m_use);
+    l_tot += __shfl_xor(l_tot, 16);
+    if constexpr (KB == 4) l_tot += __shfl_xor(l_tot, 32);
+    l = (float)l_tot;
 #pragma unroll
-        for (int e = 0; e < DE; ++e)
+    for (int v = 0; v < DV; ++v)
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            o[v][e][i] = o[v][e][i] * fa + src[64 * ((v * DE + e) * 4 + i) + lane] * fb;
-    }
+      for (int e = 0; e < DE; ++e)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float a = o[v][e][i] * f[0];
+#pragma unroll
+          for (int w = 1; w < KB; ++w)
+            a += part_of(w)[64 * ((v * DE + e) * 4 + i) + lane] * f[w];
+          o[v][e][i] = a;
+        }
   }
   const bool valid = l > 0.f;
   if (my_q < g.n_q) {
@@ -742,7 +761,7 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : D * (QB == 
           for (int e = 0; e < DE; ++e) dst[e] = o[v][e][i] / den;
         }
       }
-    if (grp == 0) LSE[(size_t)bh * g.n_q + my_q] = valid ? (float)((double)m + log((double)l)) : 0.f;
+    if (grp == 0) LSE[(size_t)bh * g.n_q + my_q] = valid ? (float)((double)m + log(l_tot)) : 0.f;
   }
 }
 
