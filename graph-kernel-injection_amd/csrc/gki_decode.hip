@@ -36,9 +36,11 @@
 namespace gki {
 namespace {
 
-// Slack of the decode's lazy reference max, in log2 units: p = exp2(s - m) <= 2^8.
+// Slack of the decode's lazy reference max, in its units (log2, natural for fp32):
+// p <= 2^8 either way, so that P V overflows only where 256 V does.
 constexpr float kDecodeSlack = 8.f;
-
+template <typename T>
+constexpr float kDecodeSlackOf = T::is_f32 ? kDecodeSlack * 0.69314718f : kDecodeSlack;
 
 // The tokens of kv tile `kt` that some of the n_q rows can see, as at most two
 // ascending runs [lo1, hi1), [lo2, hi2): the sink run and the window run (one
@@ -267,7 +269,7 @@ __device__ inline void decode_consume(const Geom& g, const DecodeRound<T, D, NU>
     // below 2^slack and the rescale (a cross-lane max, one exp2, VEC + 1
     // multiplies) is skipped in almost every round. acc / l is exact for any
     // reference max.
-    if (__any(mx > m[r] + kDecodeSlack)) {
+    if (__any(mx > m[r] + kDecodeSlackOf<T>)) {
       mx = cross_group_max<LPT>(mx);           // scores are uniform within a token row
       const float m_new = fmaxf(m[r], mx);
       const float alpha = decode_exp<T>(m[r] - m_new);   // m = -inf: 0

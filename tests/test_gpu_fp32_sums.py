@@ -88,3 +88,21 @@ def test_lse_is_rounded_once(heads):
     err, least = (float((x.double() - want).pow(2).mean().sqrt()) for x in (lse.reshape(want.shape), want.float()))
     print(f"[lse] heads {heads}: rms {err:.4e}, of one rounding {least:.4e}, ratio {err / least:.4f}", flush=True)
     assert err <= 1.07 * least
+
+
+def test_decode_weights_stay_below_2_8():
+    """The fp32 decode's reference max lags by 8 log2 units at most: blocks of 32 keys
+    that score 0 or 7 (p up to e^7 = 1096 against a lagging max of 0) times V = 3e34
+    stay finite, and O is V."""
+    b, h, n = 2, 16, 4096
+    gen = torch.Generator().manual_seed(5)
+    block = torch.randint(0, 2, (b, h, n // 32, 1), generator=gen).float() * 7
+    q, k = torch.zeros(b, h, 1, D), torch.zeros(b, h, n, D)
+    q[..., 0] = 1.0
+    k[..., 0] = block.expand(-1, -1, -1, 32).reshape(b, h, n)
+    v = torch.full((b, h, n, D), 3e34)
+    mask = stk.make_streaming_mask(1, n, stk.StreamingMaskSpec(4, 4000), 1, 64, device=DEV)
+    o = stk.block_sparse_attention(q.to(DEV), k.to(DEV), v.to(DEV), mask, softmax_scale=1.0, block_m=1,
+                                   is_causal=True, sink_size=4, window_size=4000)
+    assert torch.isfinite(o).all()
+    assert float((o / 3e34 - 1).abs().max()) <= 1e-5
