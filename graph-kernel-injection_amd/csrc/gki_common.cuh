@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include <string>
@@ -716,6 +717,34 @@ __device__ inline Geom opaque_blocks(Geom g) {
 __host__ __device__ inline bool tile_unseen(const Geom& g, int q_lo, int q_hi, int k0, int n_k) {
   return g.causal != 0 && (k0 > q_hi + g.q_off ||
                            (k0 >= g.sink && k0 + n_k <= q_lo + g.q_off - word_window(g) + 1));
+}
+
+// ---------------------------------------------------------------------------
+// Rules of the launches (host).
+// ---------------------------------------------------------------------------
+// About the kv tiles that a tile of `rows` q rows visits: the window's and the
+// sinks' under the token rule, half of them under a block mask (not known here).
+inline int row_kv_tiles(const Geom& g, int rows) {
+  const int64_t n_kt = (g.n_kv + kTileN - 1) / kTileN;
+  if (!g.causal) return (int)((n_kt + 1) / 2);
+  const int64_t keys = std::min<int64_t>((int64_t)g.window + rows - 1, g.n_kv);
+  return (int)std::min(n_kt, (keys + kTileN - 2) / kTileN + 1 + ((int64_t)g.sink + kTileN - 1) / kTileN);
+}
+
+// Does a 16-bit forward grid of `tiles` 128-row q tiles share each tile's keys
+// among the waves of two workgroups (fwd_split_16)? Where these all run at once,
+// one per CU (its 128 KB of LDS at head_dim 128 hold one), whatever the lists; at
+// head_dim <= 64, whose CU holds two, up to twice that if the chain that is cut
+// into four is long (8 kv tiles). us, one workgroup per tile against two:
+//   D128  128 tiles of 1 / 19 kv tiles  8.86, 27.7 -> 8.87, 22.0
+//         160                           8.99, 27.8 -> 15.3, 38.1
+//   D64   128                           6.80, 22.3 -> 6.55, 14.5
+//         256 tiles of 1 / 3 / 7        7.40, 9.59, 12.6 -> 8.94, 10.0, 12.6
+//         256 of 9 / 15, of 1 to 8      16.1, 21.2, 12.3 -> 14.9, 19.1, 10.9
+//         288 of 3 / 19                 11.1, 29.3 -> 14.4, 29.7
+//   D16   256 of 3 / 7 / 9 / 19         7.04, 9.40, 11.7, 17.9 -> 7.59, 9.57, 10.9, 16.3
+inline bool fwd_shares_keys(int head_dim, int tiles, int kv_tiles) {
+  return tiles <= 128 || (head_dim <= 64 && tiles <= 256 && kv_tiles >= 8);
 }
 
 // XCD-aware remap: hardware dispatches workgroup b to XCD b % 8. Give each XCD

@@ -347,7 +347,7 @@ __global__ __launch_bounds__(kFwdThreads, D <= 64 ? 4 : 2) void fwd_kernel_16(
 }
 
 // ---------------------------------------------------------------------------
-// The same for grids too short for the card (kSplitGrid): the 128-row q tile of
+// The same for grids too short for the card (fwd_shares_keys): the 128-row q tile of
 // the schedule is two workgroups of 64 rows, and a workgroup's eight waves are
 // two blocks of 32 rows x 4 shares of the keys. A step stages two kv tiles of
 // the list (double-buffered) and share x takes 32 keys of them: tile x >> 1, half
@@ -771,10 +771,6 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : D * (QB == 
 template <int D>
 constexpr bool kFwdPipe = D >= 128;
 
-// Grids of at most this many 128-row tiles (one per CU) run fwd_split_16, in us
-// against fwd_kernel_16: 256 tiles D128 (33 kv tiles each) 37.0 -> 32.6, D64 (6)
-// 12.2 -> 11.8; at 512 tiles it is behind (D128 40 -> 57, D64 24 -> 28).
-constexpr int kSplitGrid = 256;
 template <typename T, int D>
 void launch_fwd16(const Geom& g, const void* q, const void* k, const void* v, void* o, float* lse,
                   const int32_t* row_ptr, const int32_t* row_idx, int n_qt, const int32_t* wg_order,
@@ -784,7 +780,7 @@ void launch_fwd16(const Geom& g, const void* q, const void* k, const void* v, vo
   hipLaunchKernelGGL(KERNEL, dim3(GRID), dim3(THREADS), 0, stream, g, (const uint16_t*)q,          \
                      (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)o, lse, row_ptr, row_idx,  \
                      n_qt, wg_order)
-  if (grid <= kSplitGrid)
+  if (fwd_shares_keys(D, grid, row_kv_tiles(g, kTileMF)))
     GKI_FWD16((fwd_split_16<T, D>), work_parts_grid(grid, 2), 512);
   else
     GKI_FWD16((fwd_kernel_16<T, D, kFwdPipe<D>>), grid, kFwdThreads);

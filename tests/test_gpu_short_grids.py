@@ -1,8 +1,8 @@
-"""Forward grids too short for the card (GPU): 16-bit grids of up to 256 128-row
-tiles share each tile's keys among a workgroup's waves, longer ones do not. At
-the edges -- one kv tile, an odd number of them, a last half of 64 rows that
-does not exist, rows that see nothing, both sides of the 256-tile line -- each
-against the fp64 oracle, with the bars of the parity tests."""
+"""Forward grids too short for the card (GPU): 16-bit grids of up to 128 128-row
+tiles (256 of long lists at head_dim <= 64) share each tile's keys among the waves
+of two workgroups, longer ones do not. At the edges -- one kv tile, an odd number of
+them, a last half of 64 rows that does not exist, rows that see nothing, both sides
+of the lines -- each against the fp64 oracle, with the bars of the parity tests."""
 
 from __future__ import annotations
 
@@ -26,8 +26,14 @@ DEV = "cuda"
     (1, 2, 65, 129, 64, 1, 200),        # three kv tiles: an odd number, the last of one key
     (1, 1, 130, 700, 128, 4, 40),       # a ragged chunk behind a long cache
     (2, 2, 200, 100, 64, 0, 30),        # more queries than keys: rows that see nothing
-    (2, 64, 250, 250, 64, 4, 100),      # 256 tiles
-    (3, 43, 250, 250, 32, 4, 100),      # 258: one workgroup per tile
+    (2, 32, 250, 250, 64, 4, 100),      # 128 tiles
+    (1, 64, 250, 250, 128, 4, 100),     # the same, one workgroup per CU
+    (2, 64, 250, 250, 64, 4, 100),      # 256 tiles of short lists: one workgroup per tile
+    (2, 64, 250, 850, 64, 4, 500),      # 256 of long ones: two
+    (2, 64, 250, 850, 16, 4, 500),
+    (3, 43, 250, 850, 32, 4, 500),      # 258: one
+    (1, 65, 250, 850, 128, 4, 500),     # 130 at head_dim 128: one
+    (3, 43, 250, 250, 32, 4, 100),
 ])
 def test_short_grid_matches_oracle(B, H, n_q, n_kv, D, sink, window, dtype):
     print(f"[case] B{B} H{H} nq{n_q} nkv{n_kv} D{D} S{sink} W{window} {dtype}", flush=True)

@@ -1,5 +1,5 @@
 """The kernels' rules on the CPU: the tiles a wave leaves out, the form of the
-16-bit backward that a scale takes.
+16-bit backward that a scale takes, the form of the forward that a grid takes.
 
 `tile_unseen` (graph-kernel-injection_amd/csrc/gki_common.cuh) must never hold
 for a tile of which some row sees a key under the oracle's token rule, and
@@ -58,6 +58,38 @@ def test_an_operand_of_the_backward_carries_exact_scales_only(rules_exe):
             else:
                 want = PRE if 2.0**-4 <= mag <= 1 and math.frexp(mag)[0] == 0.5 else ROW
             assert form == want, (dtype, s, form)
+
+
+def test_kv_tiles_of_a_row_are_bounded(rules_exe):
+    """row_kv_tiles: never less than the longest list of the token rule, at most one
+    (an unaligned window) and the sinks' tiles above it in the middle of a long row."""
+    rng = np.random.default_rng(3)
+    cases = [(int(rng.integers(1, 700)), int(rng.integers(1, 900)), int(rng.choice([0, 1, 4, 100])),
+              int(rng.choice([0, 1, 31, 64, 200, 2**31 - 1])), rows) for _ in range(100) for rows in (64, 128)]
+    out = _run(rules_exe, "grid", [f"64 1 {n_q} {n_kv} 1 {s} {w} {rows}" for n_q, n_kv, s, w, rows in cases])
+    for (n_q, n_kv, sink, window, rows), got in zip(cases, map(int, out[::2])):
+        tiles = so.tile_classes(np.ones((-(-n_q // 64), -(-n_kv // 64)), np.int32), n_q, n_kv, 64, 64, rows, TILE, True,
+                                sink, min(window, n_q + n_kv))
+        longest = int((tiles != 0).sum(1).max())
+        assert longest <= got <= -(-n_kv // TILE)
+        if n_q < n_kv // 3 and n_q % rows == 0 and window < n_kv // 3:
+            assert got <= longest + 1 + -(-sink // TILE)
+    assert _run(rules_exe, "grid", ["64 1 100 1000 0 0 0 64", "64 1 9 64 0 0 0 64"])[::2] == ["8", "1"]
+
+
+def test_grids_whose_tiles_share_their_keys(rules_exe):
+    """Two workgroups of shares per tile while all run at once (128 tiles); up to 256
+    tiles of long lists where a CU holds two; head_dim 128 never past one per CU."""
+    def lines(d, tiles, n_kv, window, causal=1):
+        return f"{d} {tiles} 128 {n_kv} {causal} 4 {window} 128"
+
+    got = {}
+    cases = [(d, tiles, n_kv, window) for d in (16, 32, 64, 128) for tiles in (1, 128, 129, 256, 257, 4096)
+             for n_kv, window in ((64, 64), (1024, 64), (1024, 256), (1024, 400), (9000, 2048))]
+    for case, form in zip(cases, _run(rules_exe, "grid", [lines(*c) for c in cases])[1::2]):
+        got[case] = form == "1"
+    for (d, tiles, n_kv, window), split in got.items():
+        assert split == (tiles <= 128 or (d <= 64 and tiles <= 256 and window >= 256)), (d, tiles, n_kv, window)
 
 
 def test_unseen_tiles_are_exactly_those_without_a_visible_key(rules_exe):
