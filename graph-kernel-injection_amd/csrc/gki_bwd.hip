@@ -1422,11 +1422,13 @@ int launch_bwd(int dtype, const Geom& g, const void* q, const void* k, const voi
   hipLaunchKernelGGL((dkdv_kernel_32<D, KB>), dim3(work_parts_grid(kgrid, 4 / KB)), dim3(256), 0,   \
                      stream, g, (const float*)q, (const float*)k, (const float*)v,                  \
                      (const float*)dout, (float*)dk, (float*)dv, lse, delta, col_ptr, col_idx, w)
-    if (qgrid <= kF32SplitGrid4) GKI_DQ32(1);
-    else if (qgrid <= kF32SplitGrid2) GKI_DQ32(2);
+    const int qblocks = f32_row_blocks(D, qgrid, row_kv_tiles(g, kTileM));
+    if (qblocks == 1) GKI_DQ32(1);
+    else if (qblocks == 2) GKI_DQ32(2);
     else GKI_DQ32(4);
-    if (D <= 64 && kgrid <= kF32SplitGrid4) GKI_DKDV32((D <= 64 ? 1 : 2));   // 128: would spill
-    else if (kgrid <= kF32SplitGrid2) GKI_DKDV32(2);
+    const int kblocks = f32_kv_blocks(D, kgrid);
+    if (D <= 64 && kblocks == 1) GKI_DKDV32((D <= 64 ? 1 : 2));
+    else if (kblocks <= 2) GKI_DKDV32(2);
     else GKI_DKDV32(4);
 #undef GKI_DQ32
 #undef GKI_DKDV32

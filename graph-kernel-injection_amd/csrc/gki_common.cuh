@@ -458,11 +458,6 @@ constexpr int kTileN = 64;       // kv rows of every tile
 constexpr int kTileMF = 128;     // q rows of the forward tile (4 waves x 32 rows)
 constexpr int kDecodeTileM = 16;
 constexpr int kDecodeMaxQ = 4;
-// fp32 grids of at most this many 64-row tiles (one or two per CU) run them as
-// four / two workgroups of 16 / 32 rows whose waves share out the keys: B1 H4
-// N1024 D64 (64 tiles) forward 29 -> 11.6 us, dQ 43 -> 16.5 us. On full grids
-// (2048 tiles) two shares are level with none.
-constexpr int kF32SplitGrid4 = 256, kF32SplitGrid2 = 512;
 // dK/dV work items: at least kDkdvMinChunk iterations each, and about
 // kDkdvTargetItems items over the whole grid when the column walks are long.
 constexpr int kDkdvMinChunk = 32;
@@ -745,6 +740,39 @@ inline int row_kv_tiles(const Geom& g, int rows) {
 //   D16   256 of 3 / 7 / 9 / 19         7.04, 9.40, 11.7, 17.9 -> 7.59, 9.57, 10.9, 16.3
 inline bool fwd_shares_keys(int head_dim, int tiles, int kv_tiles) {
   return tiles <= 128 || (head_dim <= 64 && tiles <= 256 && kv_tiles >= 8);
+}
+
+// fp32: 16-row blocks per workgroup (1, 2 or 4 of a 64-row tile's four; the waves
+// share out the keys in fours, in twos, not at all) of a forward or dQ grid of
+// `tiles` tiles. One or two where these workgroups (16 KB x head_dim / 16 of LDS
+// each for one block, half of it for two) run at once; no shares of one or two kv
+// tiles. Forward us with 1 / 2 / 4 blocks, 3 and 19 kv tiles a row:
+//   D128   64 tiles  13.1 / 15.7 / 22.0, 46.7 / 62.8 / 101
+//         128        24.3 / 17.0 / 23.5, 87.1 / 64.5 / 102
+//         256, 512   46.3 / 25.8 / 26.1, 89.1 / 46.2 / 40.2 (3 kv tiles)
+//   D64   128        11.3 / 11.5 / 15.1, 34.8 / 41.7 / 61.9
+//         192        18.2 / 15.7 / 15.7, 61.0 / 56.9 / 62.0
+//         384, 512   29.4 / 21.8 / 23.3, 38.3 / 27.0 / 25.2 (3 kv tiles)
+//   D32   256        12.4 / 12.0 / 11.7, 38.2 / 42.2 / 44.0
+//         256 tiles of one kv tile: 7.68 / 7.24 / 6.59 (D128 27.7 / 14.5 / 13.6)
+// dQ (backward, dK/dV the same): D128 64, 128, 256 tiles 69.9 / 79.3 / 103, 122 /
+// 109 / 133, 188 / 157 / 161; D64 128, 256, 512 61.0 / 62.0 / 74.7, 86.9 / 84.8 /
+// 88.1, 195 / 187 / 184.
+inline int f32_row_blocks(int head_dim, int tiles, int kv_tiles) {
+  if (tiles > 128 && kv_tiles <= 2) return 4;
+  return tiles <= (head_dim <= 32 ? 256 : head_dim == 64 ? 128 : 64) ? 1 : tiles <= 384 ? 2 : 4;
+}
+
+// The same for the kv blocks of a dK/dV grid of `items` work items (one block would
+// spill at head_dim 128). Backward us with 1 / 2 / 4 blocks:
+//   D128  94, 188, 504 items     - / 54.7 / 64.1, 77.8 / 69.9, 154 / 138
+//   D64   36, 94, 188, 376, 504  25.1 / 27.0 / 32.8, 39.6 / 33.5 / 39.2, 51.0 / 41.7 /
+//                                41.7, 82.5 / 62.7 / 60.7, 105 / 72.1 / 68.5
+//   D32   36, 94, 188, 376, 504  17.7 / 19.4 / 22.6, 23.4 / 23.2 / 26.2, 27.1 / 27.0 /
+//                                27.4, 40.1 / 36.4 / 37.7, 49.6 / 44.0 / 42.3
+inline int f32_kv_blocks(int head_dim, int items) {
+  if (head_dim >= 128) return items <= 128 ? 2 : 4;
+  return items <= (head_dim == 64 ? 64 : 128) ? 1 : items <= (head_dim == 64 ? 256 : 384) ? 2 : 4;
 }
 
 // XCD-aware remap: hardware dispatches workgroup b to XCD b % 8. Give each XCD

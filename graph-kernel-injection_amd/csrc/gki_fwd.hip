@@ -797,8 +797,9 @@ int launch_fwd(int dtype, const Geom& g, const void* q, const void* k, const voi
   hipLaunchKernelGGL((fwd_kernel_32<D, QB>), dim3(work_parts_grid(grid, 4 / QB)), dim3(256), 0,     \
                      stream, g, (const float*)q, (const float*)k, (const float*)v, (float*)o, lse,  \
                      row_ptr, row_idx, n_qt, wg_order)
-    if (grid <= kF32SplitGrid4) GKI_FWD32(1);
-    else if (grid <= kF32SplitGrid2) GKI_FWD32(2);
+    const int blocks = f32_row_blocks(D, grid, row_kv_tiles(g, kTileM));
+    if (blocks == 1) GKI_FWD32(1);
+    else if (blocks == 2) GKI_FWD32(2);
     else GKI_FWD32(4);
 #undef GKI_FWD32
   } else if (dtype == kF16) {

@@ -67,14 +67,14 @@ def test_kv_tiles_of_a_row_are_bounded(rules_exe):
     cases = [(int(rng.integers(1, 700)), int(rng.integers(1, 900)), int(rng.choice([0, 1, 4, 100])),
               int(rng.choice([0, 1, 31, 64, 200, 2**31 - 1])), rows) for _ in range(100) for rows in (64, 128)]
     out = _run(rules_exe, "grid", [f"64 1 {n_q} {n_kv} 1 {s} {w} {rows}" for n_q, n_kv, s, w, rows in cases])
-    for (n_q, n_kv, sink, window, rows), got in zip(cases, map(int, out[::2])):
+    for (n_q, n_kv, sink, window, rows), got in zip(cases, map(int, out[::4])):
         tiles = so.tile_classes(np.ones((-(-n_q // 64), -(-n_kv // 64)), np.int32), n_q, n_kv, 64, 64, rows, TILE, True,
                                 sink, min(window, n_q + n_kv))
         longest = int((tiles != 0).sum(1).max())
         assert longest <= got <= -(-n_kv // TILE)
         if n_q < n_kv // 3 and n_q % rows == 0 and window < n_kv // 3:
             assert got <= longest + 1 + -(-sink // TILE)
-    assert _run(rules_exe, "grid", ["64 1 100 1000 0 0 0 64", "64 1 9 64 0 0 0 64"])[::2] == ["8", "1"]
+    assert _run(rules_exe, "grid", ["64 1 100 1000 0 0 0 64", "64 1 9 64 0 0 0 64"])[::4] == ["8", "1"]
 
 
 def test_grids_whose_tiles_share_their_keys(rules_exe):
@@ -86,10 +86,25 @@ def test_grids_whose_tiles_share_their_keys(rules_exe):
     got = {}
     cases = [(d, tiles, n_kv, window) for d in (16, 32, 64, 128) for tiles in (1, 128, 129, 256, 257, 4096)
              for n_kv, window in ((64, 64), (1024, 64), (1024, 256), (1024, 400), (9000, 2048))]
-    for case, form in zip(cases, _run(rules_exe, "grid", [lines(*c) for c in cases])[1::2]):
+    for case, form in zip(cases, _run(rules_exe, "grid", [lines(*c) for c in cases])[1::4]):
         got[case] = form == "1"
     for (d, tiles, n_kv, window), split in got.items():
         assert split == (tiles <= 128 or (d <= 64 and tiles <= 256 and window >= 256)), (d, tiles, n_kv, window)
+
+
+def test_fp32_blocks_per_workgroup(rules_exe):
+    """Four, two, one workgroups per tile or item while they fit the card, fewer for
+    the wider heads; one from 129 tiles on where a row sees one or two kv tiles."""
+    def blocks(d, n, n_kv=9000):
+        out = _run(rules_exe, "grid", [f"{d} {n} 64 {n_kv} 1 4 2048 64"])
+        return int(out[2]), int(out[3])
+
+    for d, one, k_one, k_two in ((16, 256, 128, 384), (32, 256, 128, 384), (64, 128, 64, 256), (128, 64, 0, 128)):
+        for n in (1, 64, 65, 128, 129, 256, 257, 384, 385, 512, 100000):
+            rows, kv = blocks(d, n)
+            assert rows == (1 if n <= one else 2 if n <= 384 else 4), (d, n)
+            assert kv == (1 if n <= k_one else 2 if n <= k_two else 4), (d, n)
+            assert blocks(d, n, 128)[0] == (4 if n > 128 else rows), (d, n)
 
 
 def test_unseen_tiles_are_exactly_those_without_a_visible_key(rules_exe):

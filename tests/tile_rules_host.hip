@@ -30,7 +30,8 @@ int main(int argc, char** argv) {
     while (std::scanf("%d %d %d %d %d %d %d %d", &head_dim, &tiles, &g.n_q, &g.n_kv, &g.causal, &g.sink, &g.window,
                       &rows) == 8) {
       const int kv = gki::row_kv_tiles(g, rows);
-      std::printf("%d %d\n", kv, (int)gki::fwd_shares_keys(head_dim, tiles, kv));
+      std::printf("%d %d %d %d\n", kv, (int)gki::fwd_shares_keys(head_dim, tiles, kv),
+                  gki::f32_row_blocks(head_dim, tiles, kv), gki::f32_kv_blocks(head_dim, tiles));
     }
   } else {
     return 1;
