@@ -326,6 +326,26 @@ def spread_chunk(col_ptr_host: torch.Tensor, group: int, bh_kv: int, target: int
     return max(2, -(-total // target))
 
 
+def _typical_walk(lens: torch.Tensor) -> int:
+    """The 90th percentile of the column walks: what most columns take, the sink
+    column's walk over every q tile left aside."""
+    return int(lens.sort().values[(9 * (lens.numel() - 1)) // 10])
+
+
+def long_walk_chunk(col_ptr_host: torch.Tensor, group: int) -> int:
+    """Iterations per fp32 dK/dV work item of a grid that fills the card: columns
+    stay whole but for those longer than a typical walk and a quarter (and 5
+    iterations). A sink column of 32 iterations among walks of 5 is a chain that
+    outlasts the grid.
+
+    Measured (fp32 backward us, columns whole up to 32 -> cut so): B1 N2048 W256 H64
+    (walks of 5 and 32) D16 400 -> 140, D32 461 -> 247, D64 725 -> 465, D128 1444 ->
+    1044 (cut at 8: 145, 253, 466, 1014); B1 H64 N512 W64 (2 and 8) D64 118 -> 87 (at 8
+    128); B1 H16 N8192 W1024 (17 and 128) D64 1306 -> 1303 (at 25 1312)."""
+    typical = _typical_walk((col_ptr_host[1:] - col_ptr_host[:-1]).to(torch.int64) * group)
+    return max(5, typical + typical // 4)
+
+
 def balanced_chunk(col_ptr_host: torch.Tensor, group: int, bh_kv: int) -> int:
     """Iterations per 16-bit dK/dV work item: a typical column walk (the 90th
     percentile, between 32 and 80) stays whole, so that only the long ones (the
@@ -345,7 +365,7 @@ def balanced_chunk(col_ptr_host: torch.Tensor, group: int, bh_kv: int) -> int:
     total = int(lens.sum()) * bh_kv
     if n == 0 or total == 0:
         return 0
-    typical = int(lens.sort().values[(9 * (n - 1)) // 10])
+    typical = _typical_walk(lens)
     chunk = min(80, max(32, typical), max(8, -(-total // 512)))
     return max(chunk, -(-total // 8192))
 
@@ -358,7 +378,8 @@ def bwd_schedule(mask: torch.Tensor, n_q: int, n_kv: int, block_m: int, block_n:
     dK/dV work list for ``group`` q heads per kv head over ``bh_kv`` = B * H_kv
     (b, kv head) pairs (items of at most ``max_chunk`` iterations when positive;
     with ``spread_to``, short grids are cut into about that many items, see
-    ``spread_chunk``; with ``balance``, the items are ``balanced_chunk`` long)."""
+    ``spread_chunk``, and the long columns of others, see ``long_walk_chunk``; with
+    ``balance``, the items are ``balanced_chunk`` long)."""
     ts = _lib.tile_sizes()
     tm, tn = ts["bwd_tile_m"], ts["tile_n"]
 
@@ -367,6 +388,8 @@ def bwd_schedule(mask: torch.Tensor, n_q: int, n_kv: int, block_m: int, block_n:
         lists = _lists_of(tiles)
         col_ptr = lists.col_ptr.cpu()
         chunk = max_chunk or spread_chunk(col_ptr, group, bh_kv, spread_to)
+        if spread_to and not chunk:
+            chunk = long_walk_chunk(col_ptr, group)
         bh_items = bh_kv
         if balance and not chunk:
             chunk = balanced_chunk(col_ptr, group, bh_kv)

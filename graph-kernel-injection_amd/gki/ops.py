@@ -31,8 +31,8 @@ _HEAD_DIMS = (16, 32, 64, 128)
 _DECODE_HEAD_DIMS = (64, 128)
 # decode workgroups to aim for: one 768-thread group on each of the 256 CUs
 _DECODE_TARGET_WGS = 256
-# fp32 dK/dV work items wanted when the kv-tile columns are fewer: the fp32
-# kernel runs one workgroup per CU, two per CU of the 256 keep them all busy
+# fp32 dK/dV work items wanted when the kv-tile columns are fewer: two per CU of the
+# 256 keep them all busy
 _FP32_DKDV_TARGET_ITEMS = 512
 
 

@@ -7,7 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from gki.lists import balanced_chunk, dkdv_items
+from gki.lists import balanced_chunk, dkdv_items, long_walk_chunk
 
 
 def _ptr(lens):
@@ -39,3 +39,13 @@ def test_chunk_and_list(lens, group, bh, want):
         assert (slot >= 0) == (lens[kt] * group > chunk)
         slots += slot >= 0
     assert at == {k: n * group for k, n in enumerate(lens)} and slots == n_pslots
+
+
+@pytest.mark.parametrize("lens,group,want", [
+    ([32] + [5] * 31, 1, 6),          # only the long one is cut
+    ([128] + [17] * 127, 1, 21),      # a quarter above a typical walk
+    ([16] + [9] * 30, 4, 45),         # grouped-query walks of 36
+    ([5, 3, 3, 2, 1], 1, 5), ([0, 0, 0], 1, 5), ([1], 1, 5),
+])
+def test_fp32_long_walks(lens, group, want):
+    assert long_walk_chunk(_ptr(lens), group) == want

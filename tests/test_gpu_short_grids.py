@@ -55,6 +55,7 @@ def test_short_grid_matches_oracle(B, H, n_q, n_kv, D, sink, window, dtype):
     (2, 4, 4, 130, 130, 4, 50),          # 24 64-row tiles: four workgroups each (dK/dV too, but at D 128)
     (3, 48, 48, 128, 190, 1, 70),        # 288: two each
     (3, 96, 48, 190, 100, 0, 40),        # 864: one each; grouped-query, rows that see nothing
+    (1, 48, 48, 700, 700, 4, 100),       # 528 kv columns: the sink column alone is cut
 ])
 def test_fp32_grids_match_oracle(B, H, H_kv, n_q, n_kv, sink, window, D):
     """fp32 forward and backward at each number of workgroups per tile, held to
