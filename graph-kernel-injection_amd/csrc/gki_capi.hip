@@ -315,25 +315,23 @@ int gki_bsa_bwd(const void* q, const void* k, const void* v, const void* o, cons
                       n_qt, dq_order, col_ptr, col_idx, w, (hipStream_t)stream);
 }
 
-int gki_dkdv_items(const int32_t* col_ptr, int32_t n_kt, int32_t group, int32_t bh_kv,
-                   int32_t max_chunk, int32_t* items, int32_t* n_items, int32_t* split,
-                   int32_t* n_split, int32_t* n_pslots) {
-  GKI_REQUIRE(col_ptr && n_items && n_split && n_pslots, 1, "gki_dkdv_items: null pointer");
-  GKI_REQUIRE(n_kt >= 1 && group >= 1 && bh_kv >= 1, 1,
-              "gki_dkdv_items: n_kt, group and bh_kv must be positive");
+namespace {
+
+// Iterations of one (b, kv head)'s columns, or -1 for column pointers that fall or
+// a walk past 2^30.
+int64_t column_iterations(const int32_t* col_ptr, int32_t n_kt, int32_t group) {
   int64_t total = 0;
   for (int kt = 0; kt < n_kt; ++kt) {
     const int64_t len = (int64_t)col_ptr[kt + 1] - col_ptr[kt];
-    GKI_REQUIRE(len >= 0 && len * group < (1ll << 30), 1, "gki_dkdv_items: bad column list");
+    if (len < 0 || len * group >= (1ll << 30)) return -1;
     total += len;
   }
-  total *= (int64_t)group * bh_kv;
-  // iterations per item: at least kDkdvMinChunk, and few enough that the whole
-  // grid has about kDkdvTargetItems items of work when columns are long; at
-  // most max_chunk when positive (more, shorter items: cuts columns at any
-  // length, e.g. to test the split path on short sequences)
-  int64_t chunk = std::max<int64_t>(kDkdvMinChunk, (total + kDkdvTargetItems - 1) / kDkdvTargetItems);
-  if (max_chunk > 0) chunk = std::min<int64_t>(chunk, max_chunk);
+  return total * group;
+}
+
+// Columns longer than `chunk` iterations cut into near-equal items no longer than it.
+void cut_columns(const int32_t* col_ptr, int32_t n_kt, int32_t group, int64_t chunk, int32_t* items,
+                 int32_t* n_items, int32_t* split, int32_t* n_split, int32_t* n_pslots) {
   int32_t ni = 0, ns = 0, np = 0;
   for (int kt = 0; kt < n_kt; ++kt) {
     const int64_t n_it = ((int64_t)col_ptr[kt + 1] - col_ptr[kt]) * group;
@@ -364,6 +362,36 @@ int gki_dkdv_items(const int32_t* col_ptr, int32_t n_kt, int32_t group, int32_t 
   *n_items = ni;
   *n_split = ns;
   *n_pslots = np;
+}
+
+}  // namespace
+
+int gki_dkdv_items(const int32_t* col_ptr, int32_t n_kt, int32_t group, int32_t bh_kv,
+                   int32_t max_chunk, int32_t* items, int32_t* n_items, int32_t* split,
+                   int32_t* n_split, int32_t* n_pslots) {
+  GKI_REQUIRE(col_ptr && n_items && n_split && n_pslots, 1, "gki_dkdv_items: null pointer");
+  GKI_REQUIRE(n_kt >= 1 && group >= 1 && bh_kv >= 1, 1,
+              "gki_dkdv_items: n_kt, group and bh_kv must be positive");
+  const int64_t its = column_iterations(col_ptr, n_kt, group);
+  GKI_REQUIRE(its >= 0, 1, "gki_dkdv_items: bad column list");
+  // iterations per item: at least kDkdvMinChunk, and few enough that the whole
+  // grid has about kDkdvTargetItems items of work when columns are long; at
+  // most max_chunk when positive (more, shorter items)
+  const int64_t total = its * bh_kv;
+  int64_t chunk = std::max<int64_t>(kDkdvMinChunk, (total + kDkdvTargetItems - 1) / kDkdvTargetItems);
+  if (max_chunk > 0) chunk = std::min<int64_t>(chunk, max_chunk);
+  cut_columns(col_ptr, n_kt, group, chunk, items, n_items, split, n_split, n_pslots);
+  return 0;
+}
+
+int gki_dkdv_items_cut(const int32_t* col_ptr, int32_t n_kt, int32_t group, int32_t chunk,
+                       int32_t* items, int32_t* n_items, int32_t* split, int32_t* n_split,
+                       int32_t* n_pslots) {
+  GKI_REQUIRE(col_ptr && n_items && n_split && n_pslots, 1, "gki_dkdv_items_cut: null pointer");
+  GKI_REQUIRE(n_kt >= 1 && group >= 1 && chunk >= 1, 1,
+              "gki_dkdv_items_cut: n_kt, group and chunk must be positive");
+  GKI_REQUIRE(column_iterations(col_ptr, n_kt, group) >= 0, 1, "gki_dkdv_items_cut: bad column list");
+  cut_columns(col_ptr, n_kt, group, chunk, items, n_items, split, n_split, n_pslots);
   return 0;
 }
 

@@ -295,24 +295,33 @@ def fwd_plan(mask: torch.Tensor, n_q: int, n_kv: int, block_m: int, block_n: int
     return _CACHE.get(mask, ("fwd plan", n_q, n_kv, block_m, block_n, is_causal, sink, window, fp32, bh), build)
 
 
-def dkdv_items(col_ptr_host: torch.Tensor, group: int, bh_kv: int, max_chunk: int = 0):
-    """The dK/dV work list of CSC column pointers (a host int32 tensor):
-    (items [n_items, 4], split [max(n_split, 1), 3], n_items, n_split, n_pslots),
-    host int32 tensors, from ``gki_dkdv_items`` (items of at most ``max_chunk``
-    iterations when positive)."""
-    lib = _lib.load()
+def _work_list(fn, name: str, col_ptr_host: torch.Tensor, *cut: int):
+    """(items [n_items, 4], split [max(n_split, 1), 3], n_items, n_split, n_pslots),
+    host int32 tensors, of column pointers cut by the library's ``fn``."""
     ptr = col_ptr_host.to(torch.int32).contiguous()
     n_kt = ptr.numel() - 1
     counts = [ctypes.c_int32() for _ in range(3)]
     refs = [ctypes.addressof(c) for c in counts]
-    _lib.check(lib.gki_dkdv_items(ptr.data_ptr(), n_kt, group, bh_kv, max_chunk, None, refs[0], None,
-                                  refs[1], refs[2]), "gki_dkdv_items")
-    n_items, n_split, _ = (c.value for c in counts)
+    _lib.check(fn(ptr.data_ptr(), n_kt, *cut, None, refs[0], None, refs[1], refs[2]), name)
+    n_items, n_split, n_pslots = (c.value for c in counts)
     items = torch.empty((n_items, 4), dtype=torch.int32)
     split = torch.zeros((max(n_split, 1), 3), dtype=torch.int32)
-    _lib.check(lib.gki_dkdv_items(ptr.data_ptr(), n_kt, group, bh_kv, max_chunk, items.data_ptr(),
-                                  refs[0], split.data_ptr(), refs[1], refs[2]), "gki_dkdv_items")
-    return items, split, counts[0].value, counts[1].value, counts[2].value
+    _lib.check(fn(ptr.data_ptr(), n_kt, *cut, items.data_ptr(), refs[0], split.data_ptr(), refs[1], refs[2]),
+               name)
+    return items, split, n_items, n_split, n_pslots
+
+
+def dkdv_items(col_ptr_host: torch.Tensor, group: int, bh_kv: int, max_chunk: int = 0):
+    """The dK/dV work list of CSC column pointers (a host int32 tensor) by the
+    library's own rule (items of at most ``max_chunk`` iterations when positive),
+    from ``gki_dkdv_items``."""
+    return _work_list(_lib.load().gki_dkdv_items, "gki_dkdv_items", col_ptr_host, group, bh_kv, max_chunk)
+
+
+def dkdv_items_cut(col_ptr_host: torch.Tensor, group: int, chunk: int):
+    """The dK/dV work list with items of at most ``chunk`` iterations, from
+    ``gki_dkdv_items_cut``."""
+    return _work_list(_lib.load().gki_dkdv_items_cut, "gki_dkdv_items_cut", col_ptr_host, group, chunk)
 
 
 def spread_chunk(col_ptr_host: torch.Tensor, group: int, bh_kv: int, target: int) -> int:
@@ -387,16 +396,14 @@ def bwd_schedule(mask: torch.Tensor, n_q: int, n_kv: int, block_m: int, block_n:
         tiles = tile_matrix(mask, n_q, n_kv, block_m, block_n, tm, tn, is_causal, sink, window)
         lists = _lists_of(tiles)
         col_ptr = lists.col_ptr.cpu()
-        chunk = max_chunk or spread_chunk(col_ptr, group, bh_kv, spread_to)
-        if spread_to and not chunk:
-            chunk = long_walk_chunk(col_ptr, group)
-        bh_items = bh_kv
-        if balance and not chunk:
-            chunk = balanced_chunk(col_ptr, group, bh_kv)
-            # the library's least chunk follows the whole grid's iterations (one
-            # item in 8192 of them): ask as for a grid of that many
-            bh_items = max(bh_kv, -(-8192 * chunk // max(1, int(col_ptr[-1]) * group)))
-        items, split, n_items, n_split, n_pslots = dkdv_items(col_ptr, group, bh_items, chunk)
+        if balance and not max_chunk:
+            cut = dkdv_items_cut(col_ptr, group, max(1, balanced_chunk(col_ptr, group, bh_kv)))
+        else:
+            chunk = max_chunk or spread_chunk(col_ptr, group, bh_kv, spread_to)
+            if spread_to and not chunk:
+                chunk = long_walk_chunk(col_ptr, group)
+            cut = dkdv_items(col_ptr, group, bh_kv, chunk)
+        items, split, n_items, n_split, n_pslots = cut
         dev = mask.device
         dq_order = _grid_order(lists.row_ptr, lists.n_rows, group * bh_kv, dev)
         return BwdSchedule(lists, items.to(dev), n_items, split.to(dev), n_split, n_pslots,

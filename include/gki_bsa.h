@@ -106,18 +106,21 @@ int gki_block_list_fill(const int32_t* m, int32_t n_rows, int32_t n_cols,
  * the chunk max(32, ceil(total iterations / 8192)) -- several near-equal items
  * whose fp32 partials gki_bsa_bwd sums in item order (deterministic; fp32
  * partials with a compensated sum). max_chunk > 0 caps the chunk (more,
- * shorter items: a caller may cut columns of any length, as the tests do to
- * run the split path on short sequences); 0 keeps the rule above. The Python
- * op passes max(2, ceil(total iterations / 512)) for fp32 inputs whose
- * B * H_kv * n_kt columns number under 512: the fp32 dK/dV kernel runs one
- * workgroup per CU, and short grids would leave CUs idle. Writes
- * items [n_items][4] = (kv tile, first iteration, end iteration, partial slot or
+ * shorter items); 0 keeps the rule above. Writes items [n_items][4] = (kv tile, first iteration, end iteration, partial slot or
  * -1) and split [n_split][3] = (kv tile, first slot, slot count), and the counts;
  * pass items = split = NULL to size them first. n_pslots partial slots per
  * (b, kv head) need 2 * 64 * head_dim floats each. */
 int gki_dkdv_items(const int32_t* col_ptr, int32_t n_kt, int32_t group, int32_t bh_kv,
                    int32_t max_chunk, int32_t* items, int32_t* n_items, int32_t* split,
                    int32_t* n_split, int32_t* n_pslots);
+
+/* The same with the items' greatest length given (chunk >= 1 iterations, any: the
+ * results do not depend on it beyond the order of fp32 partial sums). The Python
+ * op takes balanced_chunk of gki/lists.py for 16-bit inputs (spread_chunk and
+ * long_walk_chunk as max_chunk above for fp32). */
+int gki_dkdv_items_cut(const int32_t* col_ptr, int32_t n_kt, int32_t group, int32_t chunk,
+                       int32_t* items, int32_t* n_items, int32_t* split, int32_t* n_split,
+                       int32_t* n_pslots);
 
 /* Order of the forward (or dQ) grid's workgroups (host arrays; no reference
  * counterpart -- the reference's grids run their programs in index order,

@@ -7,7 +7,9 @@ from __future__ import annotations
 import pytest
 import torch
 
-from gki.lists import balanced_chunk, dkdv_items, long_walk_chunk
+from gki import _lib
+from gki.lists import balanced_chunk, dkdv_items, dkdv_items_cut, long_walk_chunk
+from oracle import streaming_oracle as so
 
 
 def _ptr(lens):
@@ -30,8 +32,7 @@ def test_chunk_and_list(lens, group, bh, want):
     assert chunk == want
     if not chunk:
         return
-    grid = max(bh, -(-8192 * chunk // (int(ptr[-1]) * group)))
-    items, split, n_items, n_split, n_pslots = dkdv_items(ptr, group, grid, chunk)
+    items, split, n_items, n_split, n_pslots = dkdv_items_cut(ptr, group, chunk)
     at, slots = {}, 0
     for kt, a, b, slot in items.tolist():
         assert a == at.get(kt, 0) and b - a <= chunk
@@ -49,3 +50,27 @@ def test_chunk_and_list(lens, group, bh, want):
 ])
 def test_fp32_long_walks(lens, group, want):
     assert long_walk_chunk(_ptr(lens), group) == want
+
+
+@pytest.mark.parametrize("chunk", [1, 5, 32, 80, 1 << 20])
+def test_cut_list_equals_the_oracle(chunk):
+    """Any length, also above the least one of the library's own rule."""
+    for lens, group in (([128] + [18] * 127, 8), ([0, 3, 0, 7], 1), ([1], 4)):
+        ptr = _ptr(lens)
+        items, split, n_items, n_split, n_pslots = dkdv_items_cut(ptr, group, chunk)
+        want = so.dkdv_items(ptr.numpy(), group, 1, chunk=chunk)
+        assert items.tolist() == want[0].tolist() and split[:n_split].tolist() == want[1].tolist()
+        assert (n_items, n_pslots) == (len(want[0]), want[2])
+        own = dkdv_items(ptr, group, 1, min(chunk, 32))
+        assert dkdv_items_cut(ptr, group, min(chunk, 32))[0].tolist() == own[0].tolist()
+
+
+def test_cut_refuses_what_the_rule_refuses():
+    lib, ptr = _lib.load(), _ptr([3, 4])
+    out = torch.zeros(3, dtype=torch.int32)
+    refs = [out.data_ptr() + 4 * i for i in range(3)]
+    falling = torch.tensor([0, 5, 3], dtype=torch.int32)
+    for col_ptr, n_kt, group, chunk in ((ptr, 2, 1, 0), (ptr, 2, 1, -1), (ptr, 2, 0, 8), (ptr, 0, 1, 8),
+                                        (falling, 2, 1, 8)):
+        assert lib.gki_dkdv_items_cut(col_ptr.data_ptr(), n_kt, group, chunk, None, refs[0], None, refs[1], refs[2]) == 1
+    assert lib.gki_dkdv_items_cut(None, 2, 1, 8, None, refs[0], None, refs[1], refs[2]) == 1

@@ -21,7 +21,7 @@ import fx_compiler_pass as fxp
 import sparse_triton_kernel as stk
 from gki import _lib, build_block_lists
 from gki.ops import _FP32_DKDV_TARGET_ITEMS
-from gki.lists import bwd_schedule, decode_schedule, fwd_order, fwd_schedule
+from gki.lists import balanced_chunk, bwd_schedule, decode_schedule, fwd_order, fwd_schedule, spread_chunk
 from oracle import chunked_reference as cr
 from oracle import streaming_oracle as so
 
@@ -426,14 +426,11 @@ def _forward_lse(q, k, v, mask, bm, bn, S, W):
                                          (torch.bfloat16, None), (torch.bfloat16, 1 << 20)])
 def test_dkdv_any_cut_of_the_work_list_matches_oracle(chunk, dtype):
     """gki_bsa_bwd through the C ABI with the dK/dV work list cut at any chunk
-    (1 iteration per item, 5, the library's default list -- the op's own for
-    16-bit inputs; fp32 ones spread short grids into 2+ iteration items --,
-    never): every cut gives the
+    (1 iteration per item, 5, the op's own list, never): every cut gives the
     oracle's gradients, grouped-query (4 q heads per kv head) so items also
     split inside a group. Inputs N(0, 1): the sink keys' walk covers 44
-    iterations (2816 q rows, |dV| up to ~9). The fp32 kernels add each
-    iteration's 64 rows into the running sums with a compensated (TwoSum)
-    addition and the reduce sums fp32 partials with Kahan summation: one fp32
+    iterations (2816 q rows, |dV| up to ~9). The fp32 kernels add 16 rows at a
+    time into the running sums with a compensated addition and the reduce sums fp32 partials with Kahan summation: one fp32
     accumulator over the whole walk reached 1.08e-5 of dV against the 1e-5 bar."""
     B, H_kv, group, N, D, S, W, bm = 1, 2, 4, 700, 64, 4, 128, 64
     H = H_kv * group
@@ -444,9 +441,13 @@ def test_dkdv_any_cut_of_the_work_list_matches_oracle(chunk, dtype):
     out = stk.block_sparse_attention(*leaves, mask, block_m=bm, block_n=bm, is_causal=True,
                                      sink_size=S, window_size=W, enable_gqa=True)
     lse = out.grad_fn.saved_tensors[4]
-    sched = bwd_schedule(mask, N, N, bm, bm, True, S, W, group=group, bh_kv=B * H_kv)
+    fp32 = dtype == torch.float32
+    sched = bwd_schedule(mask, N, N, bm, bm, True, S, W, group=group, bh_kv=B * H_kv,
+                         spread_to=_FP32_DKDV_TARGET_ITEMS if fp32 else 0, balance=not fp32)
     L = sched.lists
-    items, split, n_pslots = so.dkdv_items(L.col_ptr.cpu().numpy(), group, B * H_kv, chunk=chunk)
+    ptr = L.col_ptr.cpu()
+    own = spread_chunk(ptr, group, B * H_kv, _FP32_DKDV_TARGET_ITEMS) if fp32 else balanced_chunk(ptr, group, B * H_kv)
+    items, split, n_pslots = so.dkdv_items(ptr.numpy(), group, B * H_kv, chunk=chunk or own)
     if chunk is None:        # the op's own work list
         np.testing.assert_array_equal(sched.items.cpu().numpy(), items)
     assert (len(split) > 0) == (chunk is None or chunk < 1 << 20)
