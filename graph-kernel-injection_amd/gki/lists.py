@@ -355,40 +355,46 @@ def long_walk_chunk(col_ptr_host: torch.Tensor, group: int) -> int:
     return max(5, typical + typical // 4)
 
 
-def balanced_chunk(col_ptr_host: torch.Tensor, group: int, bh_kv: int) -> int:
-    """Iterations per 16-bit dK/dV work item: a typical column walk (the 90th
-    percentile, between 32 and 80) stays whole, so that only the long ones (the
-    sink column, large grouped-query groups) pay for fp32 partials and their
-    reduce; a grid of fewer than 512 such items (two workgroups on each of the
-    256 CUs) is cut finer, down to 8. Never less than the library's own chunk
-    for very long walks (about 8192 items in all).
+def balanced_chunk(col_ptr_host: torch.Tensor, group: int, bh_kv: int, head_dim: int = 128) -> int:
+    """Iterations per 16-bit dK/dV work item. Cutting costs fp32 partials and their
+    reduce, so a typical column walk of up to 80 iterations stays whole where the
+    columns alone fill the card (512 at head_dim 128, two workgroups per CU; 1024
+    below, where three or four fit) and only longer ones (the sink column) are cut.
+    Below head_dim 128 fewer columns of more than 48 go in items of 32, and fewer
+    than 512 columns are cut into about 512 items of at least 8. Never less than the
+    library's own chunk for very long walks (about 8192 items in all).
 
-    Measured (backward ms, 32-iteration items -> these): B1 H16 N8192 D128 W2048
-    0.511 -> 0.453, B1 H32 N16384 0.223 -> 0.191 x 10, B2 H32 on 8 kv heads N4096
-    W1024 0.553 -> 0.494 (walks of 72; items of 160 / 320: 0.500 / 0.642); B4 H16
-    N8192 D64 W1024 (walks of 17, a sink column of 128) is best at 32 (48: 0.590,
-    80: 0.605 against 0.584); a 32-block global column over 1024 short ones
-    (D32) 42 -> 23 us."""
+    Measured (backward us, 32-iteration items -> these): B1 H16 N8192 D128 W2048 511 ->
+    453; walks of 72, B2 H32/8 N4096 W1024 D128 665 -> 554 (160: 560), B1 of it 285 ->
+    257 (66: 289), D64 B8 1045 -> 945; of 144, B2 H64/8 N4096 D128 1046 -> 985 (160: 955).
+    512 columns at head_dim 64, walks of 72 and 144, at 32 / 40 / 80: B1 H32/8 N4096 153 /
+    154 / 146, H32/4 N8192 285 / 279 / 309, B2 H64/8 N2048 235 / 238 / 249; D32 H16/4
+    N8192 110 / 114 / 118. B4 H16 N8192 D64 W1024 (walks of 17, a sink column of 128) is
+    best at 32 (48: 590, 80: 605 against 584); a 32-block global column over 1024
+    short ones (D32) 42 -> 23."""
     lens = (col_ptr_host[1:] - col_ptr_host[:-1]).to(torch.int64) * group
-    n = lens.numel()
     total = int(lens.sum()) * bh_kv
-    if n == 0 or total == 0:
+    if total == 0:
         return 0
-    typical = _typical_walk(lens)
-    chunk = min(80, max(32, typical), max(8, -(-total // 512)))
+    typical, columns = _typical_walk(lens), lens.numel() * bh_kv
+    spread = max(8, -(-total // 512))
+    if columns >= 512:
+        spread = max(spread, typical)              # no typical walk in two for a little
+    whole, piece = (48, 32) if head_dim < 128 and 512 <= columns < 1024 else (80, 80)
+    chunk = min(max(32, typical) if typical <= whole else piece, spread)
     return max(chunk, -(-total // 8192))
 
 
 def bwd_schedule(mask: torch.Tensor, n_q: int, n_kv: int, block_m: int, block_n: int,
                  is_causal: bool, sink: int, window: int, group: int = 1,
                  bh_kv: int = 1, max_chunk: int = 0, spread_to: int = 0,
-                 balance: bool = False) -> BwdSchedule:
+                 balance: bool = False, head_dim: int = 128) -> BwdSchedule:
     """CSR + CSC schedules of the dQ and dK/dV kernels (64x64 tiles) and the
     dK/dV work list for ``group`` q heads per kv head over ``bh_kv`` = B * H_kv
     (b, kv head) pairs (items of at most ``max_chunk`` iterations when positive;
     with ``spread_to``, short grids are cut into about that many items, see
     ``spread_chunk``, and the long columns of others, see ``long_walk_chunk``; with
-    ``balance``, the items are ``balanced_chunk`` long)."""
+    ``balance``, the items are ``balanced_chunk`` long for ``head_dim``)."""
     ts = _lib.tile_sizes()
     tm, tn = ts["bwd_tile_m"], ts["tile_n"]
 
@@ -397,7 +403,7 @@ def bwd_schedule(mask: torch.Tensor, n_q: int, n_kv: int, block_m: int, block_n:
         lists = _lists_of(tiles)
         col_ptr = lists.col_ptr.cpu()
         if balance and not max_chunk:
-            cut = dkdv_items_cut(col_ptr, group, max(1, balanced_chunk(col_ptr, group, bh_kv)))
+            cut = dkdv_items_cut(col_ptr, group, max(1, balanced_chunk(col_ptr, group, bh_kv, head_dim)))
         else:
             chunk = max_chunk or spread_chunk(col_ptr, group, bh_kv, spread_to)
             if spread_to and not chunk:
@@ -410,7 +416,7 @@ def bwd_schedule(mask: torch.Tensor, n_q: int, n_kv: int, block_m: int, block_n:
                            lists.n_rows, lists.n_cols, dq_order)
 
     key = ("bwd", n_q, n_kv, block_m, block_n, tm, tn, bool(is_causal), sink, window, group, bh_kv,
-           max_chunk, spread_to, balance)
+           max_chunk, spread_to, balance, head_dim if balance else 0)
     return _CACHE.get(mask, key, build)
 
 

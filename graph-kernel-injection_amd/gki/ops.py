@@ -280,7 +280,7 @@ class _BlockSparseFlashAttention(torch.autograd.Function):
             spread = _FP32_DKDV_TARGET_ITEMS if q.dtype == torch.float32 else 0
             sched = bwd_schedule(block_mask, N_Q, N_KV, ctx.block_m, ctx.block_n, ctx.is_causal,
                                  ctx.sink_size, ctx.window_size, group=H // H_kv, bh_kv=B * H_kv,
-                                 spread_to=spread, balance=spread == 0)
+                                 spread_to=spread, balance=spread == 0, head_dim=D)
             L = sched.lists
             # fp32 dK / dV partials of the split kv tiles: [B*H_kv, n_pslots, 2, 64, D]
             tile_n = _lib.tile_sizes()["tile_n"]

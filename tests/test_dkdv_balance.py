@@ -20,6 +20,7 @@ def _ptr(lens):
     ([128] + [17] * 127, 1, 64, 32),          # short walks, one long: the least chunk
     ([256] + [33] * 255, 1, 16, 33),          # walks just past 32 stay whole
     ([64] + [18] * 63, 4, 16, 72),            # grouped-query walks of 72
+    ([20] + [18] * 63, 4, 8, 72),             # 512 of them; their mean is a little less
     ([128] + [18] * 127, 8, 4, 80),           # of 144: cut
     ([32] + [7] * 31, 1, 32, 16),             # a short grid: total / 512
     ([6] * 16, 1, 4, 8),                      # the shortest
@@ -50,6 +51,18 @@ def test_chunk_and_list(lens, group, bh, want):
 ])
 def test_fp32_long_walks(lens, group, want):
     assert long_walk_chunk(_ptr(lens), group) == want
+
+
+@pytest.mark.parametrize("lens,group,bh,want", [
+    ([64] + [18] * 63, 4, 8, 32),             # 512 columns of 72: in pieces
+    ([64] + [18] * 63, 4, 16, 72),            # 1024: whole
+    ([128] + [18] * 127, 8, 4, 32), ([128] + [18] * 127, 8, 8, 80),
+    ([64] + [33] * 63, 1, 8, 33),             # walks of up to 48: whole
+    ([64] + [18] * 63, 4, 4, 38),             # fewer columns: total / 512
+])
+def test_chunk_where_more_workgroups_fit(lens, group, bh, want):
+    for head_dim in (16, 32, 64):
+        assert balanced_chunk(_ptr(lens), group, bh, head_dim) == want
 
 
 @pytest.mark.parametrize("chunk", [1, 5, 32, 80, 1 << 20])

@@ -443,10 +443,10 @@ def test_dkdv_any_cut_of_the_work_list_matches_oracle(chunk, dtype):
     lse = out.grad_fn.saved_tensors[4]
     fp32 = dtype == torch.float32
     sched = bwd_schedule(mask, N, N, bm, bm, True, S, W, group=group, bh_kv=B * H_kv,
-                         spread_to=_FP32_DKDV_TARGET_ITEMS if fp32 else 0, balance=not fp32)
+                         spread_to=_FP32_DKDV_TARGET_ITEMS if fp32 else 0, balance=not fp32, head_dim=D)
     L = sched.lists
     ptr = L.col_ptr.cpu()
-    own = spread_chunk(ptr, group, B * H_kv, _FP32_DKDV_TARGET_ITEMS) if fp32 else balanced_chunk(ptr, group, B * H_kv)
+    own = spread_chunk(ptr, group, B * H_kv, _FP32_DKDV_TARGET_ITEMS) if fp32 else balanced_chunk(ptr, group, B * H_kv, D)
     items, split, n_pslots = so.dkdv_items(ptr.numpy(), group, B * H_kv, chunk=chunk or own)
     if chunk is None:        # the op's own work list
         np.testing.assert_array_equal(sched.items.cpu().numpy(), items)
