@@ -17,7 +17,8 @@ from oracle import streaming_oracle as so
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
-LSE_BAR = {torch.float16: 5e-4, torch.bfloat16: 2.5e-3}    # the row sum is of the 16-bit P
+# the row sum is of the 16-bit P, each within half a unit: ln(1 + 2^-11), ln(1 + 2^-8)
+LSE_BAR = {torch.float16: 5e-4, torch.bfloat16: 4e-3}
 
 
 def _check(B, H, H_kv, n_q, n_kv, D, dtype, sink, window, mask=None, bm=64, bn=64, scale=None, q_scale=1.0):

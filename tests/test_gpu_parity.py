@@ -400,10 +400,10 @@ def test_config2_prefill_bf16_full():
 def test_lse_vs_oracle(case, dtype, bar):
     """The saved log-sum-exp against the fp64 oracle's, absolute: fp32 sums fp32
     P (1e-5); the 16-bit kernels sum the 16-bit-rounded P that multiplies V
-    (fp32 P where a short grid's workgroups share a tile's keys), within 2^-12
-    (fp16) / 2^-9 (bf16) of each fp32 term, bounding the LSE error by
-    ln(1 + 2^-11) < 5e-4 and ln(1 + 2^-9) < 2.5e-3. Rows that see no key keep the
-    sentinel 0."""
+    (fp32 P where a short grid's workgroups share a tile's keys), within 2^-11
+    (fp16) / 2^-8 (bf16) of each fp32 term: an LSE error of ln(1 + 2^-11) < 5e-4
+    and, where one term makes the row, 3.9e-3 (2.5e-3 asked of these rows). Rows
+    that see no key keep the sentinel 0."""
     B, H, n_q, n_kv, D, bm, bn, S, W = case
     q, k, v, _ = _inputs((B, H, n_q, D), (B, H, n_kv, D), dtype, seed=57)
     mask = stk.make_streaming_mask(n_q, n_kv, stk.StreamingMaskSpec(S, W), bm, bn, device=DEV)
