@@ -361,7 +361,9 @@ def balanced_chunk(col_ptr_host: torch.Tensor, group: int, bh_kv: int, head_dim:
     columns alone fill the card (512 at head_dim 128, two workgroups per CU; 1024
     below, where three or four fit) and only longer ones (the sink column) are cut.
     Below head_dim 128 fewer columns of more than 48 go in items of 32, and fewer
-    than 512 columns are cut into about 512 items of at least 8. Never less than the
+    than 512 columns are cut into about 512 items of at least 8, but for 128 or more
+    of even length (a dense or random mask) up to 32 -- 192 and 16 below head_dim 64 --
+    where more workgroups per CU do not pay for the partials. Never less than the
     library's own chunk for very long walks (about 8192 items in all).
 
     Measured (backward us, 32-iteration items -> these): B1 H16 N8192 D128 W2048 511 ->
@@ -371,7 +373,11 @@ def balanced_chunk(col_ptr_host: torch.Tensor, group: int, bh_kv: int, head_dim:
     154 / 146, H32/4 N8192 285 / 279 / 309, B2 H64/8 N2048 235 / 238 / 249; D32 H16/4
     N8192 110 / 114 / 118. B4 H16 N8192 D64 W1024 (walks of 17, a sink column of 128) is
     best at 32 (48: 590, 80: 605 against 584); a 32-block global column over 1024
-    short ones (D32) 42 -> 23."""
+    short ones (D32) 42 -> 23. Dense masks at 8 / whole: B2 H8 N1000 (256 columns of 16)
+    D32 33.4 / 30.7, D64 46.0 / 40.0, D128 61.7 / 51.9; B1 H8 N1000 (128) 27.7 / 29.7, 36.9 /
+    38.0, 51.9 / 49.5; N2048 causal (256 of up to 32) D16 34.2 / 39.6, D32 39.0 / 42.6, D64
+    55.0 / 56.4, D128 82.2 / 77.2; B1 H4 N700 (44 of 11) 20.9 / 22.2, 27.3 / 29.6, 36.5 /
+    38.1. Sinks over short walks at 8 / 16 / 32: B1 H4 N4096 W256 D64 29.0 / 37.1 / 53.7."""
     lens = (col_ptr_host[1:] - col_ptr_host[:-1]).to(torch.int64) * group
     total = int(lens.sum()) * bh_kv
     if total == 0:
@@ -380,6 +386,10 @@ def balanced_chunk(col_ptr_host: torch.Tensor, group: int, bh_kv: int, head_dim:
     spread = max(8, -(-total // 512))
     if columns >= 512:
         spread = max(spread, typical)              # no typical walk in two for a little
+    elif int(lens.max()) <= 2 * typical:           # nothing long to balance
+        few, short = (128, 32) if head_dim >= 64 else (192, 16)
+        if columns >= few and typical <= short:
+            spread = max(spread, 16, typical)
     whole, piece = (48, 32) if head_dim < 128 and 512 <= columns < 1024 else (80, 80)
     chunk = min(max(32, typical) if typical <= whole else piece, spread)
     return max(chunk, -(-total // 8192))

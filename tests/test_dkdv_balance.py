@@ -59,10 +59,21 @@ def test_fp32_long_walks(lens, group, want):
     ([128] + [18] * 127, 8, 4, 32), ([128] + [18] * 127, 8, 8, 80),
     ([64] + [33] * 63, 1, 8, 33),             # walks of up to 48: whole
     ([64] + [18] * 63, 4, 4, 38),             # fewer columns: total / 512
+    ([16] * 16, 1, 16, 16), ([9, 7, 12] * 7, 1, 24, 16),   # even walks: whole
+    ([16] * 16, 1, 7, 8),                     # too few of them
+    ([32] + [9] * 31, 1, 8, 8),               # a long one among them
 ])
 def test_chunk_where_more_workgroups_fit(lens, group, bh, want):
     for head_dim in (16, 32, 64):
         assert balanced_chunk(_ptr(lens), group, bh, head_dim) == want
+
+
+@pytest.mark.parametrize("lens,bh,wide,narrow", [
+    ([24] * 24, 8, 24, 9), ([16] * 16, 8, 16, 8), ([16] * 16, 12, 16, 16), ([17] * 17, 12, 17, 8),
+])
+def test_even_walks_by_head_dim(lens, bh, wide, narrow):
+    for head_dim, want in ((16, narrow), (32, narrow), (64, wide), (128, wide)):
+        assert balanced_chunk(_ptr(lens), 1, bh, head_dim) == want
 
 
 @pytest.mark.parametrize("chunk", [1, 5, 32, 80, 1 << 20])
