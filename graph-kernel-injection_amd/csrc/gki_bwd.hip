@@ -5,11 +5,12 @@
 //   * `_bwd_preprocess_kernel` (sparse_triton_kernel.py:354-392),
 //       Delta[q] = sum_d fp32(O) * fp32(dO) over the stored O, inside the dQ
 //       kernel, which runs first and stores it (negated for 16-bit inputs) for
-//       dK/dV. For 16-bit inputs the dQ kernel also turns the stored natural LSE into base 2
-//       once per row (second half of the row-term workspace), so the 16-bit
-//       kernels form P = exp(S scale - LSE) as one exp2 of an fma; the fp32
-//       kernels form it as exp2(fma(S, scale, -LSE) log2 e) from the stored
-//       LSE, as the fp32 forward computed its exponents.
+//       dK/dV. For 16-bit inputs it also stores, once per row, the LSE as the
+//       16-bit kernels take it (second half of the row-term workspace): in base 2
+//       at head_dim 64, P = exp2 of one fma of the score; elsewhere -LSE / scale,
+//       from which the score accumulates, P = exp2 of one product. The fp32
+//       kernels form P as exp2(fma(S, scale, -LSE) log2 e) from the stored LSE, as
+//       the fp32 forward computed its exponents.
 //   * dkdv_kernel   <- `_bwd_dkdv_kernel` (sparse_triton_kernel.py:394-509):
 //       one workgroup per 64-row KV tile, loop over the kept q tiles of its
 //       column (CSC list), P = exp(S - LSE), dV += P^T dO,
@@ -385,7 +386,7 @@ __global__ __launch_bounds__(256, D <= 32 ? 4 : FORM != kBwdPlain ? 2 : 1) void 
 // halves' fp32 dK / dV sums meet once, through LDS, at the end of the item
 // (the qh = 0 wave adds the qh = 1 wave's, a fixed order). Waves leave out the
 // 32 x 32 blocks they cannot see: B4 H16 N8192 W1024 fp16 backward 0.586 ->
-// 0.577 ms, B1 H16 N131072 W4096 7.02 -> 7.00.
+// 0.577 ms (level on walks of 65, B1 H16 N131072 W4096).
 // ---------------------------------------------------------------------------
 template <typename T, bool PRE>
 __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
@@ -470,78 +471,78 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
     const int qw0 = q0 + 32 * qh;              // the wave's first q row
     // left out where none of the wave's rows sees one of its keys
     if (!tile_unseen(g, qw0, qw0 + 31, k_w, 32)) {
-    const bool need_mask = partial || (qw0 + 32 > g.n_q) || (k_w + 31 >= g.n_kv) ||
-                           !tile_all_visible(g, qw0, min(qw0 + 31, g.n_q - 1), k_w, kv_hi_wave);
-    floatx4 p[2][2], ds[2][2];                 // [subtile 2 qh + u][kv block]
+      const bool need_mask = partial || (qw0 + 32 > g.n_q) || (k_w + 31 >= g.n_kv) ||
+                             !tile_all_visible(g, qw0, min(qw0 + 31, g.n_q - 1), k_w, kv_hi_wave);
+      floatx4 p[2][2], ds[2][2];                 // [subtile 2 qh + u][kv block]
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int t = 2 * qh + u;
-      const int qr0 = rho(t, 4 * grp);
-      const float4 lse4 = *(const float4*)(&slse[buf][qr0]);
-      const float4 ndl4 = *(const float4*)(&sdlt[buf][qr0]);
-      floatx4 sc[2], dp[2];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        sc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
-        dp[b] = floatx4{ndl4.x, ndl4.y, ndl4.z, ndl4.w};
-      }
-      const int r = rho(t, col);
-      mfma_priority_hi<true>();
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int d0 = 32 * ks + 8 * grp;
-        const uint4 aq = lds_row8<D>(cq, r, d0);
-        const uint4 ad = lds_row8<D>(cdo, r, d0);
+      for (int u = 0; u < 2; ++u) {
+        const int t = 2 * qh + u;
+        const int qr0 = rho(t, 4 * grp);
+        const float4 lse4 = *(const float4*)(&slse[buf][qr0]);
+        const float4 ndl4 = *(const float4*)(&sdlt[buf][qr0]);
+        floatx4 sc[2], dp[2];
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-          sc[b] = T::mfma(aq, kf[b][ks], sc[b]);
-          dp[b] = T::mfma(ad, vf[b][ks], dp[b]);
+          sc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+          dp[b] = floatx4{ndl4.x, ndl4.y, ndl4.z, ndl4.w};
+        }
+        const int r = rho(t, col);
+        mfma_priority_hi<true>();
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const int d0 = 32 * ks + 8 * grp;
+          const uint4 aq = lds_row8<D>(cq, r, d0);
+          const uint4 ad = lds_row8<D>(cdo, r, d0);
+#pragma unroll
+          for (int b = 0; b < 2; ++b) {
+            sc[b] = T::mfma(aq, kf[b][ks], sc[b]);
+            dp[b] = T::mfma(ad, vf[b][ks], dp[b]);
+          }
+        }
+        mfma_priority_lo<true>();
+        const float lv[4] = {lse4.x, lse4.y, lse4.z, lse4.w};
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[b][i], g.scale_log2, -lv[i]));
+            p[u][b][i] = pv;
+            ds[u][b][i] = PRE ? pv * dp[b][i] : pv * (dp[b][i] * g.scale);
+          }
+      }
+      if (need_mask) {     // masked elements: P = dS = 0 (bit select)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const LaneBits vis(col_valid_bits(g, k_w + 16 * b + col, q0, partial), grp);
+          const uint32_t wq = qh ? vis.w[1] : vis.w[0];   // uniform select, not an index
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int m = __builtin_amdgcn_sbfe((int)wq, 4 * u + i, 1);   // 0 or -1
+              p[u][b][i] = __int_as_float(__float_as_int(p[u][b][i]) & m);
+              ds[u][b][i] = __int_as_float(__float_as_int(ds[u][b][i]) & m);
+            }
+        }
+      }
+      uint4 ap[2], as[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        ap[b] = pack8<T>(p[0][b], p[1][b]);
+        as[b] = pack8<T>(ds[0][b], ds[1][b]);
+      }
+      mfma_priority_hi<true>();
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const uint4 bo = lds_tr8<D>(cdo, 32 * qh, 16 * dt, lane);
+        const uint4 bq = lds_tr8<D>(cq, 32 * qh, 16 * dt, lane);
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          dv[b][dt] = T::mfma(ap[b], bo, dv[b][dt]);
+          dk[b][dt] = T::mfma(as[b], bq, dk[b][dt]);
         }
       }
       mfma_priority_lo<true>();
-      const float lv[4] = {lse4.x, lse4.y, lse4.z, lse4.w};
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[b][i], g.scale_log2, -lv[i]));
-          p[u][b][i] = pv;
-          ds[u][b][i] = PRE ? pv * dp[b][i] : pv * (dp[b][i] * g.scale);
-        }
-    }
-    if (need_mask) {     // masked elements: P = dS = 0 (bit select)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const LaneBits vis(col_valid_bits(g, k_w + 16 * b + col, q0, partial), grp);
-        const uint32_t wq = qh ? vis.w[1] : vis.w[0];   // uniform select, not an index
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int m = __builtin_amdgcn_sbfe((int)wq, 4 * u + i, 1);   // 0 or -1
-            p[u][b][i] = __int_as_float(__float_as_int(p[u][b][i]) & m);
-            ds[u][b][i] = __int_as_float(__float_as_int(ds[u][b][i]) & m);
-          }
-      }
-    }
-    uint4 ap[2], as[2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      ap[b] = pack8<T>(p[0][b], p[1][b]);
-      as[b] = pack8<T>(ds[0][b], ds[1][b]);
-    }
-    mfma_priority_hi<true>();
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      const uint4 bo = lds_tr8<D>(cdo, 32 * qh, 16 * dt, lane);
-      const uint4 bq = lds_tr8<D>(cq, 32 * qh, 16 * dt, lane);
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        dv[b][dt] = T::mfma(ap[b], bo, dv[b][dt]);
-        dk[b][dt] = T::mfma(as[b], bq, dk[b][dt]);
-      }
-    }
-    mfma_priority_lo<true>();
     }
     dma_wait();        // the next tile's LDS-DMA has landed before the barrier
     __syncthreads();
@@ -604,11 +605,10 @@ __global__ __launch_bounds__(256, 3) void dkdv_kernel_q64(
 // dK / dV, fp32
 // ---------------------------------------------------------------------------
 // Bound by the fp32 matrix cores and, beside them, the VALU (exponents, the
-// compensated folds): B1 H16 N8192 D64 W1024 1281 -> 763 us (dQ 671 -> 557, the
-// forward 432 -> 335; 459, 344 and 229 us at the nominal MFMA rate) against
-// 4-byte LDS reads, tiles staged through registers behind two barriers, folds
-// per 16 rows and a separate Delta launch; D128 N4096 backward 2.08 -> 1.41 ms.
-// Three waves per SIMD ran 12% slower than two (head_dim 64).
+// compensated folds): B1 H16 N8192 D64 W1024 backward 1.97 -> 1.30 ms (dK/dV and dQ
+// 803 us at the nominal MFMA rate), D128 N4096 2.08 -> 1.41, against 4-byte LDS
+// reads, tiles staged through registers behind two barriers and a separate Delta
+// launch. Three waves per SIMD ran 12% slower than two (head_dim 64).
 // As the forward, a workgroup's four waves are KB blocks of 16 kv rows x 4 / KB
 // shares of the q rows of each staged step (16 rows each; two subtiles when
 // KB = 4), and an item of the work list is 4 / KB workgroups. The shares' sums
@@ -751,9 +751,9 @@ __global__ __launch_bounds__(256, D >= 128 || (D == 64 && KB == 1) ? 1 : 2) void
     // shares 1 .. QS - 1 hand their sums over through LDS (free: every wave
     // passed the last barrier); share 0 folds them in, in order
     constexpr int SZ = 2 * 2 * 16 * D;                   // dk, ck, dv, cv of a wave
-    static_assert((QS - 1) * KB * SZ <= 2 * 2 * TR * D, "the sums fit the staging buffers");
-    float* red = sq[0];                                  // sq and sdo are contiguous (one array each, in order)
-    float* red2 = sdo[0];
+    static_assert((QS - 1) * KB * SZ / 2 <= 2 * TR * D, "half of the sums fits each staging array");
+    float* red = &sq[0][0];
+    float* red2 = &sdo[0][0];
     const int blk = wave % KB;
     // dk / ck through sq, dv / cv through sdo
     const size_t at = ((size_t)(share - 1) * KB + blk) * (SZ / 2) + lane;
@@ -877,7 +877,7 @@ __global__ __launch_bounds__(256, D > 64 ? 2 : 4) void dq_kernel_16(
       // Delta = rowsum(O * dO) in fp32 over the stored O (the preprocessing pass,
       // sparse_triton_kernel.py:354-392, fused here): the lane already holds its
       // half of the row's dO, the two halves are summed across. Every q row has
-      // exactly one dQ workgroup, which writes it (and the base-2 LSE) for the
+      // exactly one dQ workgroup, which writes it (and the LSE's form) for the
       // dK/dV kernel that runs next.
       if (ok) {
         const uint4 o4 = *(const uint4*)(O + o);
@@ -1091,66 +1091,66 @@ __global__ __launch_bounds__(256, 4) void dq_kernel_q64(
     const int kw0 = k0 + 32 * kh;              // the wave's first kv row
     // left out where none of the wave's rows sees one of its keys
     if (!tile_unseen(g, q0w, q0w + 31, kw0, 32)) {
-    const bool need_mask = partial || (q0w + 31 >= g.n_q) || (kw0 + 32 > g.n_kv) ||
-                           !tile_all_visible(g, q0w, q_hi_wave, kw0, kw0 + 31);
-    floatx4 ds[2][2];                          // [subtile 2 kh + u][q block]
+      const bool need_mask = partial || (q0w + 31 >= g.n_q) || (kw0 + 32 > g.n_kv) ||
+                             !tile_all_visible(g, q0w, q_hi_wave, kw0, kw0 + 31);
+      floatx4 ds[2][2];                          // [subtile 2 kh + u][q block]
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int r = rho(2 * kh + u, col);
-      floatx4 sc[2], dp[2];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        sc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
-        dp[b] = floatx4{ndlt[b], ndlt[b], ndlt[b], ndlt[b]};
-      }
-      mfma_priority_hi<true>();
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int d0 = 32 * ks + 8 * grp;
-        const uint4 ak = lds_row8<D>(ck, r, d0);
-        const uint4 av = lds_row8<D>(cv, r, d0);
+      for (int u = 0; u < 2; ++u) {
+        const int r = rho(2 * kh + u, col);
+        floatx4 sc[2], dp[2];
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-          sc[b] = T::mfma(ak, qf[b][ks], sc[b]);
-          dp[b] = T::mfma(av, df[b][ks], dp[b]);
+          sc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+          dp[b] = floatx4{ndlt[b], ndlt[b], ndlt[b], ndlt[b]};
         }
-      }
-      mfma_priority_lo<true>();
+        mfma_priority_hi<true>();
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+        for (int ks = 0; ks < KS; ++ks) {
+          const int d0 = 32 * ks + 8 * grp;
+          const uint4 ak = lds_row8<D>(ck, r, d0);
+          const uint4 av = lds_row8<D>(cv, r, d0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[b][i], g.scale_log2, -lse2[b]));
-          ds[u][b][i] = PRE ? pv * dp[b][i] : pv * (dp[b][i] * g.scale);
+          for (int b = 0; b < 2; ++b) {
+            sc[b] = T::mfma(ak, qf[b][ks], sc[b]);
+            dp[b] = T::mfma(av, df[b][ks], dp[b]);
+          }
         }
-    }
-    if (need_mask) {     // masked elements: dS = 0 (bit select)
+        mfma_priority_lo<true>();
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const LaneBits vis(row_valid_bits(g, q0w + 16 * b + col, k0, partial), grp);
-        // the word of subtiles 2 kh, 2 kh + 1, chosen by a uniform select (an
-        // index by kh would put the pair in scratch)
-        const uint32_t wk = kh ? vis.w[1] : vis.w[0];
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int b = 0; b < 2; ++b)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int m = __builtin_amdgcn_sbfe((int)wk, 4 * u + i, 1);   // 0 or -1
-            ds[u][b][i] = __int_as_float(__float_as_int(ds[u][b][i]) & m);
+            const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[b][i], g.scale_log2, -lse2[b]));
+            ds[u][b][i] = PRE ? pv * dp[b][i] : pv * (dp[b][i] * g.scale);
           }
       }
-    }
-    uint4 pb[2];
+      if (need_mask) {     // masked elements: dS = 0 (bit select)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) pb[b] = pack8<T>(ds[0][b], ds[1][b]);
-    mfma_priority_hi<true>();
+        for (int b = 0; b < 2; ++b) {
+          const LaneBits vis(row_valid_bits(g, q0w + 16 * b + col, k0, partial), grp);
+          // the word of subtiles 2 kh, 2 kh + 1, chosen by a uniform select (an
+          // index by kh would put the pair in scratch)
+          const uint32_t wk = kh ? vis.w[1] : vis.w[0];
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      const uint4 a = lds_tr8<D>(ck, 32 * kh, 16 * dt, lane);
+          for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) dq[b][dt] = T::mfma(a, pb[b], dq[b][dt]);
-    }
-    mfma_priority_lo<true>();
+            for (int i = 0; i < 4; ++i) {
+              const int m = __builtin_amdgcn_sbfe((int)wk, 4 * u + i, 1);   // 0 or -1
+              ds[u][b][i] = __int_as_float(__float_as_int(ds[u][b][i]) & m);
+            }
+        }
+      }
+      uint4 pb[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) pb[b] = pack8<T>(ds[0][b], ds[1][b]);
+      mfma_priority_hi<true>();
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const uint4 a = lds_tr8<D>(ck, 32 * kh, 16 * dt, lane);
+#pragma unroll
+        for (int b = 0; b < 2; ++b) dq[b][dt] = T::mfma(a, pb[b], dq[b][dt]);
+      }
+      mfma_priority_lo<true>();
     }
     dma_wait();        // the next tile's LDS-DMA has landed before the barrier
     __syncthreads();
@@ -1309,7 +1309,7 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : 2) void dq_
   if constexpr (KB > 1) {              // the shares' sums, through LDS, in order
     constexpr int SZ = 2 * 16 * D;                       // dq, cq of a wave
     static_assert((KB - 1) * QB * SZ <= 2 * TR * D, "the sums fit one staging array");
-    float* red = sk[0];
+    float* red = &sk[0][0];
     const int blk = wave % QB;
     if (share > 0) {
       float* dst = red + ((size_t)(share - 1) * QB + blk) * SZ + lane;
@@ -1362,7 +1362,7 @@ __global__ __launch_bounds__(256, D * (QB == 1 ? 4 : 2) >= 512 ? 1 : 2) void dq_
   }
 }
 
-// dQ first: it also produces -Delta and the base-2 LSE rows, which dK/dV reads
+// dQ first: it also produces the -Delta and LSE rows, which dK/dV reads
 // from the two halves of the row-term workspace
 template <typename T, int D, int FORM>
 void launch_bwd16_as(const Geom& g, const void* q, const void* k, const void* v, const void* o,

@@ -448,10 +448,11 @@ struct DmaTileF32 {
 };
 
 // ---------------------------------------------------------------------------
-// Kernel tiling. The forward uses 128x64 (q x kv) tiles, four waves per
-// workgroup, each wave owning 32 query rows; the backward kernels use 64x64
-// tiles, each wave owning 16 rows of the tile's outer axis. The decode kernel
-// (n_q <= kDecodeMaxQ) uses a single 16-row q tile.
+// Kernel tiling. The 16-bit forward uses 128x64 (q x kv) tiles, four waves of 32
+// query rows each (on short grids two workgroups of eight waves, fwd_split_16);
+// the backward kernels use 64x64 tiles, a 32x32 quadrant per wave; the fp32
+// kernels 64x64 tiles in blocks of 16 rows. The decode kernel (n_q <=
+// kDecodeMaxQ) uses a single 16-row q tile.
 // ---------------------------------------------------------------------------
 constexpr int kTileM = 64;       // q rows of the dQ / dK-dV tiles
 constexpr int kTileN = 64;       // kv rows of every tile

@@ -273,7 +273,7 @@ class _BlockSparseFlashAttention(torch.autograd.Function):
         dq = torch.empty_like(q)
         dk = torch.empty_like(k)
         dv = torch.empty_like(v)
-        # row terms: Delta, then the base-2 LSE rows (internal to the backward)
+        # row terms: Delta, then a form of the LSE rows (internal to the backward)
         delta = torch.empty((2, B, H, N_Q), dtype=torch.float32, device=q.device)
         with _on_device(q.device):
             stream = _current_stream(q.device)

@@ -153,8 +153,9 @@ int gki_bsa_fwd(const void* q, const void* k, const void* v, void* o, float* lse
  * [B * H_kv][n_pslots][2][64][head_dim], needed when n_split > 0) and dQ over
  * the CSR list, both over bwd_tile_m x tile_n tiles. `lse` is the forward's
  * (natural) LSE. `delta` is a caller-owned fp32 [2, B, H, N_Q] workspace for
- * the row terms (its contents on return are internal: Delta -- negated and
- * scaled for fp16 / bf16 -- then each row's LSE in base 2). dq, dk, dv are
+ * the row terms (its contents on return are internal: Delta -- negated, for some
+ * scales scaled, for fp16 / bf16 -- then, for these, a form of each row's LSE that
+ * the kernels of its head_dim and scale start from). dq, dk, dv are
  * fully written (no zero-fill needed). dq_order: NULL (index order) or a
  * device copy of gki_fwd_order's table for the backward CSR and B * H (the
  * dQ grid runs each XCD's q tiles longest list first). */
