@@ -341,18 +341,21 @@ def _typical_walk(lens: torch.Tensor) -> int:
     return int(lens.sort().values[(9 * (lens.numel() - 1)) // 10])
 
 
-def long_walk_chunk(col_ptr_host: torch.Tensor, group: int) -> int:
+def long_walk_chunk(col_ptr_host: torch.Tensor, group: int, bh_kv: int) -> int:
     """Iterations per fp32 dK/dV work item of a grid that fills the card: columns
     stay whole but for those longer than a typical walk and a quarter (and 5
     iterations). A sink column of 32 iterations among walks of 5 is a chain that
-    outlasts the grid.
+    outlasts the grid. Never less than the library's own chunk for very long walks
+    (about 8192 items in all: each is 128 rows of fp32 partials, 36 GB where 200
+    global columns of 2048 iterations over 16 heads were cut at 6).
 
     Measured (fp32 backward us, columns whole up to 32 -> cut so): B1 N2048 W256 H64
     (walks of 5 and 32) D16 400 -> 140, D32 461 -> 247, D64 725 -> 465, D128 1444 ->
     1044 (cut at 8: 145, 253, 466, 1014); B1 H64 N512 W64 (2 and 8) D64 118 -> 87 (at 8
     128); B1 H16 N8192 W1024 (17 and 128) D64 1306 -> 1303 (at 25 1312)."""
-    typical = _typical_walk((col_ptr_host[1:] - col_ptr_host[:-1]).to(torch.int64) * group)
-    return max(5, typical + typical // 4)
+    lens = (col_ptr_host[1:] - col_ptr_host[:-1]).to(torch.int64) * group
+    typical = _typical_walk(lens)
+    return max(5, typical + typical // 4, -(-int(lens.sum()) * bh_kv // 8192))
 
 
 def balanced_chunk(col_ptr_host: torch.Tensor, group: int, bh_kv: int, head_dim: int = 128) -> int:
@@ -417,7 +420,7 @@ def bwd_schedule(mask: torch.Tensor, n_q: int, n_kv: int, block_m: int, block_n:
         else:
             chunk = max_chunk or spread_chunk(col_ptr, group, bh_kv, spread_to)
             if spread_to and not chunk:
-                chunk = long_walk_chunk(col_ptr, group)
+                chunk = long_walk_chunk(col_ptr, group, bh_kv)
             cut = dkdv_items(col_ptr, group, bh_kv, chunk)
         items, split, n_items, n_split, n_pslots = cut
         dev = mask.device

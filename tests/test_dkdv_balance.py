@@ -50,7 +50,20 @@ def test_chunk_and_list(lens, group, bh, want):
     ([5, 3, 3, 2, 1], 1, 5), ([0, 0, 0], 1, 5), ([1], 1, 5),
 ])
 def test_fp32_long_walks(lens, group, want):
-    assert long_walk_chunk(_ptr(lens), group) == want
+    assert long_walk_chunk(_ptr(lens), group, 16) == want
+
+
+@pytest.mark.parametrize("lens,group,bh", [
+    ([512] * 50 + [5] * 462, 1, 16),          # a tenth of the columns over every row
+    ([2048] * 200 + [5] * 1848, 1, 16), ([2048] + [65] * 2047, 1, 16), ([300] * 9 + [2] * 91, 8, 8),
+])
+def test_fp32_long_walks_bounded_partials(lens, group, bh):
+    """Many long columns over short typical ones: still about 8192 items in all, each
+    of which is 128 rows of fp32 partials."""
+    ptr = _ptr(lens)
+    chunk = long_walk_chunk(ptr, group, bh)
+    n_pslots = dkdv_items(ptr, group, bh, chunk)[4]
+    assert n_pslots * bh <= 8192 + len(lens) * bh
 
 
 @pytest.mark.parametrize("lens,group,bh,want", [
